@@ -1,6 +1,6 @@
 """The reverse index's radix sort (bf_radix_sort_keys) against numpy's stable argsort of the same bit
-field, for every digit plan it picks: 9-bit digits with 2048-, 4096- and 6144-key tiles, 8-bit digits, one
-partial tile, a single-bit field, all 64 bits (sign bit included) and an empty bit range. Keys mix
+field, for every digit plan it picks: 6- to 10-bit digits with each of their tile sizes, at the first key past
+each size's range, one partial tile, a single-bit field, all 64 bits (sign bit included) and an empty bit range. Keys mix
 uniform 64-bit patterns with fields drawn from a steep power law (long runs of one digit, many equal
 fields), so stability is checked on ties. Integer work: bit-exact."""
 import numpy as np
@@ -37,10 +37,20 @@ def _expected(keys, b0, b1):
 
 @pytest.mark.parametrize("n,b0,b1", [
     (1, 0, 5),
+    (1023, 2, 14),             # 12 bits: two 6-bit passes, one partial 1024-key tile
+    (65_536, 0, 14),           # 14 bits: two 7-bit passes, the last size of the 1024-key tiles
+    (65_537, 9, 25),           # 16 bits: two 8-bit passes, one key past them (2048-key tiles)
+    (60_001, 30, 50),          # 20 bits: two 10-bit passes at the smallest sizes (2048-key tiles)
+    (2_097_153, 11, 31),       # 10-bit digits, one key past the 2048-key tiles (4096)
+    (4_194_305, 3, 22),        # 19 bits: 10-bit digits, one key past the 4096-key tiles (8192)
+    (7_000_003, 0, 21),        # 21 bits: three 7-bit passes, 4096-key tiles of eight waves
+    (16_777_217, 20, 42),      # 22 bits: 8-bit digits, one key past them (4096-key tiles of four waves)
+    (67_108_865, 31, 49),      # 9-bit digits, one key past the 4096-key tiles (8192)
+    (1_170_000, 0, 36),        # 36 bits: four 9-bit passes, the keys of an edge list
     (1000, 3, 21),             # 18 bits: two 9-bit passes, one partial tile
-    (823_801, 22, 40),         # the c2 reverse-index shape
-    (5_000_000, 10, 28),       # 18 bits past 4M keys: 4096-key tiles
-    (34_000_000, 5, 23),       # 18 bits past 32M keys: 6144-key tiles
+    (823_801, 22, 40),         # a small reverse index's shape: 9-bit digits, 2048-key tiles
+    (5_000_000, 10, 28),       # 18 bits past 2M keys: 4096-key tiles of eight waves
+    (34_000_000, 5, 23),       # 18 bits past 16M keys: 4096-key tiles of four waves
     (3_000_000, 20, 42),       # 22 bits: three 8-bit passes
     (2_000_000, 0, 27),        # 27 bits: three 9-bit passes
     (300_000, 0, 64),          # every bit, the top one included: eight 8-bit passes
