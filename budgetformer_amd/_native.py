@@ -20,6 +20,10 @@ ABI_VERSION = 303                   # the header's BF_ABI_VERSION this binding i
 BF_MAX_ITEMS_PER_ROW = 160          # items a split row is cut into at most (the header's #define) ...
 BF_LONG_ROW_FACTOR = 64             # ... unless it is longer than 160 * 64 items' worth (the header's #define)
 
+# what a COO list holds (the header's BF_COO_* bits) and bf_coo_order's workspace in bytes
+COO_IDS, COO_TYPES, COO_ROW_MAJOR, COO_COL_MAJOR, COO_STRICT, COO_BY_COL, COO_BY_ROW = 1, 2, 4, 8, 16, 32, 64
+COO_ORDER_WORKSPACE = 4096
+
 i32, i64, u64, sz, f32 = C.c_int32, C.c_int64, C.c_uint64, C.c_size_t, C.c_float
 vp = C.c_void_p
 P_i32 = vp  # device pointers are passed as plain addresses
@@ -71,6 +75,7 @@ _SIGS = {
                               vp]),
     "bf_coalesce_workspace_size": (C.c_int, [i64, C.POINTER(sz)]),
     "bf_coalesce": (C.c_int, [P_i64, P_i64, i64, i64, P_i64, P_i64, C.POINTER(i64), vp, sz, vp]),
+    "bf_coalesce_bidirected": (C.c_int, [P_i64, P_i64, i64, i64, P_i64, P_i64, C.POINTER(i64), vp, sz, vp]),
     "bf_walk_records": (C.c_int, [P_i64, P_i32, i64, i64, vp, vp]),
     "bf_rw_select": (C.c_int, [P_i64, P_i32, vp, i64, i64, i64, i32, i32, i32, i64, P_f32, u64, u64, P_i32, P_i32,
                                vp]),
@@ -91,6 +96,12 @@ _SIGS = {
     "bf_scan_workspace_size": (C.c_int, [i64, C.POINTER(sz)]),
     "bf_coo_to_csr_workspace_size": (C.c_int, [i64, i64, C.POINTER(sz)]),
     "bf_coo_to_csr": (C.c_int, [P_i64, P_i64, i64, i64, i64, P_i64, P_i32, vp, sz, vp]),
+    "bf_coo_order": (C.c_int, [P_i64, P_i64, P_i64, i64, i64, i64, C.POINTER(i32), vp, sz, vp]),
+    "bf_coo_to_csr_ordered_workspace_size": (C.c_int, [i64, i64, i64, i32, i32, C.POINTER(sz)]),
+    "bf_coo_to_csr_ordered": (C.c_int, [P_i64, P_i64, P_i64, i64, i64, i64, i32, P_i64, P_i32, vp, vp, sz, vp]),
+    "bf_coo_reverse_workspace_size": (C.c_int, [i64, i64, i64, i32, i32, C.POINTER(sz)]),
+    "bf_coo_reverse": (C.c_int, [vp, i64, i64, i64, i32, i32, P_i64, P_i32, vp, sz, vp]),
+    "bf_coo_reverse_slots": (C.c_int, [P_i64, P_i32, P_i64, P_i32, i64, i64, P_i32, vp]),
     "bf_reverse_index_workspace_size": (C.c_int, [i64, i64, C.POINTER(sz)]),
     "bf_reverse_index": (C.c_int, [P_i64, P_i32, i64, i64, i64, P_i64, P_i32, P_i32, vp, sz, vp]),
     "bf_reverse_index_packed_workspace_size": (C.c_int, [i64, C.POINTER(sz)]),

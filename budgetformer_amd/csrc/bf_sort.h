@@ -193,7 +193,7 @@ __global__ __launch_bounds__(THREADS) void radix_count_kernel(Load in, int64_t c
   }
 }
 
-__global__ __launch_bounds__(kThreads) void radix_scan_kernel(uint32_t* __restrict__ counts, int64_t tiles,
+static __global__ __launch_bounds__(kThreads) void radix_scan_kernel(uint32_t* __restrict__ counts, int64_t tiles,
                                                               uint32_t* __restrict__ totals) {
   __shared__ uint32_t tmp[kThreads / 64];
   uint32_t* row = counts + int64_t(blockIdx.x) * tiles;

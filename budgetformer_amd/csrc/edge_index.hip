@@ -273,20 +273,6 @@ __global__ void boundaries_kernel(const K* __restrict__ keys, int64_t n, uint64_
   fill_gap(r_prev, r_here, i, [&](int64_t r, int64_t v) { ptr[r] = v; });
 }
 
-__global__ void coo_keys_kernel(const int64_t* __restrict__ src, const int64_t* __restrict__ dst, int64_t nnz,
-                                uint64_t n_kv, uint64_t* __restrict__ keys) {
-  const int64_t i = int64_t(blockIdx.x) * kThreads + threadIdx.x;
-  if (i >= nnz) return;
-  keys[i] = uint64_t(dst[i]) * n_kv + uint64_t(src[i]);
-}
-
-__global__ void coo_kv_kernel(const uint64_t* __restrict__ keys, int64_t nnz, uint64_t n_kv,
-                              int32_t* __restrict__ kv) {
-  const int64_t i = int64_t(blockIdx.x) * kThreads + threadIdx.x;
-  if (i >= nnz) return;
-  kv[i] = int32_t(keys[i] % n_kv);
-}
-
 // ---------------------------------------------------------------- reverse index
 // rows[i] = r with ptr[r] <= i < ptr[r+1] (binary search; balanced for any row length).
 template <typename R>
@@ -775,47 +761,6 @@ extern "C" int bf_table_to_csr(const int32_t* table, const int32_t* row_len, int
   return BF_OK;
 }
 
-extern "C" int bf_coo_to_csr_workspace_size(int64_t nnz, int64_t n_q, size_t* bytes) {
-  BF_CHECK_ARG(bytes && nnz >= 0 && n_q >= 0, "coo_to_csr_workspace_size: bad arguments");
-  size_t sort_bytes = 0;
-  (void)prim::sort_keys(nullptr, sort_bytes, static_cast<const uint64_t*>(nullptr), static_cast<uint64_t*>(nullptr),
-                        nnz > 0 ? nnz : 1, 0, 64, hipStream_t(nullptr));
-  *bytes = 2 * align_up(size_t(nnz > 0 ? nnz : 1) * sizeof(uint64_t)) + align_up(sort_bytes) + 256;
-  (void)n_q;
-  return BF_OK;
-}
-
-extern "C" int bf_coo_to_csr(const int64_t* src, const int64_t* dst, int64_t nnz, int64_t n_q, int64_t n_kv,
-                             int64_t* qptr, int32_t* kv, void* workspace, size_t workspace_bytes, void* stream) {
-  BF_CHECK_ARG(nnz >= 0 && n_q >= 0 && n_kv > 0 && qptr, "coo_to_csr: bad arguments");
-  BF_CHECK_ARG(n_kv < (int64_t(1) << 31) && nnz < (int64_t(1) << 31), "coo_to_csr: sizes must fit int32");
-  size_t need = 0;
-  bf_coo_to_csr_workspace_size(nnz, n_q, &need);
-  BF_CHECK_ARG(workspace && workspace_bytes >= need, "coo_to_csr: workspace %zu < %zu bytes", workspace_bytes, need);
-  hipStream_t st = as_stream(stream);
-  if (nnz == 0) {
-    BF_CHECK_HIP(hipMemsetAsync(qptr, 0, size_t(n_q + 1) * sizeof(int64_t), st));
-    return BF_OK;
-  }
-  auto* keys_in = static_cast<uint64_t*>(workspace);
-  auto* keys_out = reinterpret_cast<uint64_t*>(static_cast<char*>(workspace) + align_up(size_t(nnz) * 8));
-  void* temp = static_cast<char*>(workspace) + 2 * align_up(size_t(nnz) * 8);
-  size_t temp_bytes = 0;
-  (void)prim::sort_keys(nullptr, temp_bytes, static_cast<const uint64_t*>(keys_in), keys_out, nnz, 0, 64, st);
-  BF_LAUNCH("coo_keys_kernel", coo_keys_kernel, dim3(blocks_for(nnz)), dim3(kThreads), 0, st, src, dst, nnz,
-                     uint64_t(n_kv), keys_in);
-  BF_CHECK_LAUNCH();
-  const int end_bit = bits_for(uint64_t(n_q) * uint64_t(n_kv));
-  BF_CHECK_HIP(prim::sort_keys(temp, temp_bytes, static_cast<const uint64_t*>(keys_in), keys_out, nnz, 0, end_bit, st));
-  BF_LAUNCH("coo_kv_kernel", coo_kv_kernel, dim3(blocks_for(nnz)), dim3(kThreads), 0, st, keys_out, nnz,
-                     uint64_t(n_kv), kv);
-  BF_CHECK_LAUNCH();
-  BF_LAUNCH("boundaries_kernel", boundaries_kernel<uint64_t>, dim3(blocks_for(nnz + 1)), dim3(kThreads), 0, st, keys_out,
-                     nnz, uint64_t(n_kv), n_q, qptr);
-  BF_CHECK_LAUNCH();
-  return BF_OK;
-}
-
 extern "C" int bf_reverse_index_workspace_size(int64_t nnz, int64_t n_kv, size_t* bytes) {
   BF_CHECK_ARG(bytes && nnz >= 0 && n_kv >= 0, "reverse_index_workspace_size: bad arguments");
   size_t sort_bytes = 0;
@@ -1042,7 +987,7 @@ extern "C" int bf_split_plan_first_row(int64_t n_rows, int32_t n_items, int32_t*
   return BF_OK;
 }
 
-// ---------------------------------------------------------------- hop pool and coalesce
+// ---------------------------------------------------------------- hop pool
 namespace bf {
 namespace {
 
@@ -1076,28 +1021,6 @@ __global__ void hop_fill_kernel(const int64_t* __restrict__ walks, int64_t n_wal
 __global__ void i32_to_i64_kernel(const int32_t* __restrict__ a, int64_t n, int64_t* __restrict__ b) {
   const int64_t i = int64_t(blockIdx.x) * kThreads + threadIdx.x;
   if (i < n) b[i] = a[i];
-}
-
-__global__ void coalesce_keys_kernel(const int64_t* __restrict__ src, const int64_t* __restrict__ dst, int64_t nnz,
-                                     uint64_t n, uint64_t* __restrict__ keys) {
-  const int64_t i = int64_t(blockIdx.x) * kThreads + threadIdx.x;
-  if (i < nnz) keys[i] = uint64_t(src[i]) * n + uint64_t(dst[i]);
-}
-
-__global__ void unique_flags_kernel(const uint64_t* __restrict__ keys, int64_t nnz, int64_t* __restrict__ flags) {
-  const int64_t i = int64_t(blockIdx.x) * kThreads + threadIdx.x;
-  if (i < nnz) flags[i] = (i == 0 || keys[i] != keys[i - 1]) ? 1 : 0;
-}
-
-__global__ void unique_fill_kernel(const uint64_t* __restrict__ keys, const int64_t* __restrict__ incl, int64_t nnz,
-                                   uint64_t n, int64_t* __restrict__ out_src, int64_t* __restrict__ out_dst) {
-  const int64_t i = int64_t(blockIdx.x) * kThreads + threadIdx.x;
-  if (i >= nnz) return;
-  if (i == 0 || keys[i] != keys[i - 1]) {
-    const int64_t p = incl[i] - 1;
-    out_src[p] = int64_t(keys[i] / n);
-    out_dst[p] = int64_t(keys[i] % n);
-  }
 }
 
 }  // namespace
@@ -1150,54 +1073,6 @@ extern "C" int bf_hop_pool(const int64_t* walks, int64_t n_walks, int32_t walk_l
   return BF_OK;
 }
 
-extern "C" int bf_coalesce_workspace_size(int64_t nnz, size_t* bytes) {
-  BF_CHECK_ARG(bytes && nnz >= 0, "coalesce_workspace_size: bad arguments");
-  const int64_t n = nnz > 0 ? nnz : 1;
-  size_t sort_bytes = 0, scan_bytes = 0;
-  (void)prim::sort_keys(nullptr, sort_bytes, static_cast<const uint64_t*>(nullptr), static_cast<uint64_t*>(nullptr),
-                        n, 0, 64, hipStream_t(nullptr));
-  (void)prim::inclusive_sum(nullptr, scan_bytes, static_cast<const int64_t*>(nullptr), static_cast<int64_t*>(nullptr),
-                            n, hipStream_t(nullptr));
-  *bytes = 4 * align_up(size_t(n) * 8) + align_up(sort_bytes > scan_bytes ? sort_bytes : scan_bytes) + 256;
-  return BF_OK;
-}
-
-extern "C" int bf_coalesce(const int64_t* src, const int64_t* dst, int64_t nnz, int64_t num_nodes, int64_t* out_src,
-                           int64_t* out_dst, int64_t* count_host, void* workspace, size_t workspace_bytes,
-                           void* stream) {
-  BF_CHECK_ARG(count_host && nnz >= 0 && num_nodes > 0, "coalesce: bad arguments");
-  BF_CHECK_ARG(nnz < (int64_t(1) << 31) && num_nodes < (int64_t(1) << 32), "coalesce: sizes out of range");
-  *count_host = 0;
-  if (nnz == 0) return BF_OK;
-  BF_CHECK_ARG(src && dst && out_src && out_dst, "coalesce: null tensor");
-  size_t need = 0;
-  bf_coalesce_workspace_size(nnz, &need);
-  BF_CHECK_ARG(workspace && workspace_bytes >= need, "coalesce: workspace %zu < %zu bytes", workspace_bytes, need);
-  hipStream_t st = as_stream(stream);
-  const size_t slab = align_up(size_t(nnz) * 8);
-  auto* keys_in = static_cast<uint64_t*>(workspace);
-  auto* keys = reinterpret_cast<uint64_t*>(static_cast<char*>(workspace) + slab);
-  auto* flags = reinterpret_cast<int64_t*>(static_cast<char*>(workspace) + 2 * slab);
-  auto* incl = reinterpret_cast<int64_t*>(static_cast<char*>(workspace) + 3 * slab);
-  void* temp = static_cast<char*>(workspace) + 4 * slab;
-  size_t sort_bytes = 0, scan_bytes = 0;
-  (void)prim::sort_keys(nullptr, sort_bytes, static_cast<const uint64_t*>(keys_in), keys, nnz, 0, 64, st);
-  (void)prim::inclusive_sum(nullptr, scan_bytes, static_cast<const int64_t*>(flags), incl, nnz, st);
-  BF_LAUNCH("coalesce_keys_kernel", coalesce_keys_kernel, dim3(blocks_for(nnz)), dim3(kThreads), 0, st, src, dst, nnz,
-            uint64_t(num_nodes), keys_in);
-  BF_CHECK_LAUNCH();
-  const int end_bit = bits_for(uint64_t(num_nodes) * uint64_t(num_nodes));
-  BF_CHECK_HIP(prim::sort_keys(temp, sort_bytes, static_cast<const uint64_t*>(keys_in), keys, nnz, 0, end_bit, st));
-  BF_LAUNCH("unique_flags_kernel", unique_flags_kernel, dim3(blocks_for(nnz)), dim3(kThreads), 0, st, keys, nnz, flags);
-  BF_CHECK_LAUNCH();
-  BF_CHECK_HIP(prim::inclusive_sum(temp, scan_bytes, static_cast<const int64_t*>(flags), incl, nnz, st));
-  BF_LAUNCH("unique_fill_kernel", unique_fill_kernel, dim3(blocks_for(nnz)), dim3(kThreads), 0, st, keys, incl, nnz,
-            uint64_t(num_nodes), out_src, out_dst);
-  BF_CHECK_LAUNCH();
-  BF_CHECK_HIP(hipMemcpyAsync(count_host, incl + nnz - 1, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  BF_CHECK_HIP(hipStreamSynchronize(st));
-  return BF_OK;
-}
 
 namespace {
 // The order kernels' per-block bucket counts and bucket totals, then (plans

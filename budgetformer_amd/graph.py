@@ -91,10 +91,11 @@ class CSRGraph:
         pass a coalesced edge list as the reference does.
         """
         ei = edge_index.to(device)
-        rowptr, col = hip_ops.coo_to_csr(torch.stack([ei[1], ei[0]]), num_nodes, num_nodes)
+        src, dst = hip_ops._pair_lists(ei)
+        rowptr, col = hip_ops.coo_rows_to_csr(src, dst, num_nodes, num_nodes)
         if symmetric:
             return cls(rowptr, col, rowptr, col, int(num_nodes))
-        in_ptr, in_src = hip_ops.coo_to_csr(ei, num_nodes, num_nodes)
+        in_ptr, in_src = hip_ops.coo_rows_to_csr(dst, src, num_nodes, num_nodes)
         return cls(rowptr, col, in_ptr, in_src, int(num_nodes))
 
 
@@ -150,6 +151,8 @@ def coalesce_edges(edge_index: torch.Tensor, num_nodes: int, max_chunk: int = _S
 
 def to_bidirected(edge_index: torch.Tensor, num_nodes: int, max_chunk: int = _SORT_LIMIT) -> torch.Tensor:
     """``_to_bidirected_edge_index`` (utils/fullgraph_sp_support.py:570-572): coalesce(E ∪ flip(E))."""
+    if edge_index.dim() == 2 and edge_index.size(0) == 2 and 2 * int(edge_index.size(1)) <= max_chunk:
+        return hip_ops.coalesce_bidirected(edge_index, int(num_nodes))
     return coalesce_edges(torch.cat([edge_index, edge_index.flip(0)], dim=1), num_nodes, max_chunk)
 
 

@@ -346,8 +346,8 @@ def _get_random_walk_graph(edge_index: torch.Tensor, num_nodes: int, device):
     # the entry pins its source tensor, so a hit is the same tensor (same version), not a reused address
     if hit is not None and hit[0] is edge_index and hit[1] == edge_index._version:
         return hit[2]
-    ei = hip_ops.coalesce(edge_index.to(dev), num_nodes)
-    rowptr, col = hip_ops.coo_to_csr(torch.stack([ei[1], ei[0]]), num_nodes, num_nodes)
+    src, dst = hip_ops._pair_lists(hip_ops.coalesced(edge_index.to(dev), num_nodes))
+    rowptr, col = hip_ops.coo_rows_to_csr(src, dst, num_nodes, num_nodes)
     placeholder = torch.empty((2, 0), dtype=edge_index.dtype, device=dev)
     _RANDOM_WALK_GRAPH_CACHE.clear()
     _RANDOM_WALK_GRAPH_CACHE[key] = (edge_index, edge_index._version, (placeholder, rowptr, col))
@@ -418,8 +418,8 @@ def compute_khop_pool_dgl_neighbor(edge_index: torch.Tensor, num_nodes: int, fan
         return torch.zeros((2, 0), dtype=torch.long, device=out_dev)
     dev = out_dev if out_dev.type == "cuda" else torch.device("cuda", torch.cuda.current_device())
     n = max(int(num_nodes), int(edge_index.max().item()) + 1)
-    ei = edge_index.to(dev)
-    rowptr, col = hip_ops.coo_to_csr(torch.stack([ei[1], ei[0]]), n, n)     # out-neighbour CSR
+    src, dst = hip_ops._pair_lists(edge_index.to(dev))
+    rowptr, col = hip_ops.coo_rows_to_csr(src, dst, n, n)     # out-neighbour CSR
     seed = _draw_walk_seed() if seed is None else int(seed)
     return hip_ops.khop_fanout_pool(rowptr, col, [int(f) for f in fanout], seed=seed,
                                     min_hop=int(min_hop)).to(out_dev)

@@ -179,18 +179,61 @@ def khop_fanout_pool(rowptr: torch.Tensor, col: torch.Tensor, fanout, seed: int 
     return torch.cat(parts, dim=1)
 
 
-def coalesce(edge_index: torch.Tensor, num_nodes: int) -> torch.Tensor:
-    """Sort by (src, dst) and drop duplicates (torch_geometric.utils.coalesce), on the device."""
+def _pair_lists(edge_index: torch.Tensor):
+    """Rows 0 and 1 of an edge list as contiguous int64 tensors (views where they are that already)."""
+    return edge_index[0].to(torch.int64).contiguous(), edge_index[1].to(torch.int64).contiguous()
+
+
+def _coo_holds(row: torch.Tensor, col: torch.Tensor, n_row: int, n_col: int,
+               types: Optional[torch.Tensor] = None) -> int:
+    """The N.COO_* bits an edge list keeps to (bf_coo_order): one pass over it and one host read."""
+    dev = row.device
+    stream = _stream(dev)
+    ws = _workspace(N.COO_ORDER_WORKSPACE, dev)
+    holds = C.c_int32(0)
+    N.call("bf_coo_order", _p(row), _p(col), _p(types), row.numel(), n_row, n_col, C.byref(holds), _p(ws), ws.numel(),
+           stream)
+    return holds.value
+
+
+def _coalesced(fn: str, edge_index: torch.Tensor, num_nodes: int, capacity: int) -> torch.Tensor:
     dev = edge_index.device
-    src = edge_index[0].to(torch.int64).contiguous()
-    dst = edge_index[1].to(torch.int64).contiguous()
-    nnz = src.numel()
-    out = torch.empty(2, max(nnz, 1), dtype=torch.int64, device=dev)
-    ws = _workspace(_size_query("bf_coalesce_workspace_size", nnz), dev)
+    src, dst = _pair_lists(edge_index)
+    stream = _stream(dev)
+    out = torch.empty(2, max(capacity, 1), dtype=torch.int64, device=dev)
+    ws = _workspace(_size_query("bf_coalesce_workspace_size", capacity), dev)
     cnt = C.c_int64(0)
-    N.call("bf_coalesce", _p(src), _p(dst), nnz, num_nodes, C.c_void_p(out[0].data_ptr()),
-           C.c_void_p(out[1].data_ptr()), C.byref(cnt), _p(ws), ws.numel(), _stream(dev))
+    N.call(fn, _p(src), _p(dst), src.numel(), num_nodes, C.c_void_p(out[0].data_ptr()),
+           C.c_void_p(out[1].data_ptr()), C.byref(cnt), _p(ws), ws.numel(), stream)
     return out[:, : cnt.value]
+
+
+def _is_coalesced(edge_index: torch.Tensor, num_nodes: int) -> bool:
+    src, dst = _pair_lists(edge_index)
+    if not 0 < src.numel() < 2 ** 31:
+        return False
+    holds = _coo_holds(src, dst, num_nodes, num_nodes)
+    return bool(holds & N.COO_STRICT and holds & N.COO_IDS)
+
+
+def coalesce(edge_index: torch.Tensor, num_nodes: int) -> torch.Tensor:
+    """Sort by (src, dst) and drop duplicates (torch_geometric.utils.coalesce), on the device. A list that is
+    coalesced already is copied, not sorted again."""
+    if _is_coalesced(edge_index, num_nodes):
+        return torch.stack(_pair_lists(edge_index))
+    return _coalesced("bf_coalesce", edge_index, num_nodes, edge_index[0].numel())
+
+
+def coalesced(edge_index: torch.Tensor, num_nodes: int) -> torch.Tensor:
+    """``coalesce`` for a caller that only reads the result: a coalesced list itself, else its coalesced copy."""
+    if _is_coalesced(edge_index, num_nodes):
+        return edge_index
+    return _coalesced("bf_coalesce", edge_index, num_nodes, edge_index[0].numel())
+
+
+def coalesce_bidirected(edge_index: torch.Tensor, num_nodes: int) -> torch.Tensor:
+    """``coalesce`` of a list and its mirror image (dst, src), without writing the doubled list."""
+    return _coalesced("bf_coalesce_bidirected", edge_index, num_nodes, 2 * edge_index[0].numel())
 
 
 def walk_uniforms(q_lo: int, n_q: int, walks_per_node: int, walk_length: int, philox_seed: int,
@@ -511,23 +554,60 @@ def split_row_items(length: int, item_size: int = DEFAULT_ITEM) -> int:
     return int(N.load().bf_split_row_items(int(length), int(item_size)))
 
 
+def coo_rows_to_csr(rows: torch.Tensor, cols: torch.Tensor, n_rows: int, n_cols: int,
+                    types: Optional[torch.Tensor] = None, with_keys: bool = False):
+    """CSR of the entries (rows[i], cols[i]) (int64, any order): (ptr int64 [n_rows+1], ids int32 [nnz] ascending
+    within a row). ``types`` (int64, 0 or 1): rows ordered by (type, id), the type in bit 31 of each id. With
+    ``with_keys`` also (keys, in_order): the entries' sort keys for ``coo_reverse``. Ids are checked on the device
+    (ValueError), and a list that is in row or column order already is sorted by the missing bits only."""
+    dev = rows.device
+    stream = _stream(dev)
+    nnz = rows.numel()
+    holds = _coo_holds(rows, cols, n_rows, n_cols, types)
+    if types is not None and not holds & N.COO_TYPES:
+        raise ValueError("edge types must be 0 or 1")
+    if not holds & N.COO_IDS:
+        raise ValueError(f"edge_index ids outside [0,{n_cols}) x [0,{n_rows})")
+    typed = int(types is not None)
+    ws = _workspace(_size_query("bf_coo_to_csr_ordered_workspace_size", nnz, n_rows, n_cols, typed, holds), dev)
+    ptr = torch.empty(n_rows + 1, dtype=torch.int64, device=dev)
+    ids = torch.empty(max(nnz, 1), dtype=torch.int32, device=dev)[:nnz]
+    keys = torch.empty(max(nnz, 1), dtype=torch.int64, device=dev)[:nnz] if with_keys else None
+    N.call("bf_coo_to_csr_ordered", _p(rows), _p(cols), _p(types), nnz, n_rows, n_cols, holds, _p(ptr), _p(ids),
+           _p(keys), _p(ws), ws.numel(), stream)
+    if not with_keys:
+        return ptr, ids
+    return ptr, ids, (keys, bool(holds & N.COO_COL_MAJOR) and not typed)
+
+
 def coo_to_csr(edge_index: torch.Tensor, n_q: int, n_kv: int):
     """Reference COO [2, nnz] (row 0 = kv, row 1 = query) -> (qptr, kv), rows ascending in kv."""
-    dev = edge_index.device
     if edge_index.dim() != 2 or edge_index.size(0) < 2:
         raise ValueError(f"edge_index must be [2, E] (got {tuple(edge_index.shape)})")
-    src = edge_index[0].to(torch.int64).contiguous()
-    dst = edge_index[1].to(torch.int64).contiguous()
-    nnz = src.numel()
-    if nnz:
-        lo = torch.stack([src.min(), dst.min()]).min().item()
-        if lo < 0 or src.max().item() >= n_kv or dst.max().item() >= n_q:
-            raise ValueError(f"edge_index ids outside [0,{n_kv}) x [0,{n_q})")
-    ws = _workspace(_size_query("bf_coo_to_csr_workspace_size", nnz, n_q), dev)
-    qptr = torch.empty(n_q + 1, dtype=torch.int64, device=dev)
-    kv = torch.empty(max(nnz, 1), dtype=torch.int32, device=dev)[:nnz]
-    N.call("bf_coo_to_csr", _p(src), _p(dst), nnz, n_q, n_kv, _p(qptr), _p(kv), _p(ws), ws.numel(), _stream(dev))
-    return qptr, kv
+    src, dst = _pair_lists(edge_index)
+    return coo_rows_to_csr(dst, src, n_q, n_kv)
+
+
+def coo_reverse(keys, n_q: int, n_kv: int, typed: bool = False):
+    """(kptr int64 [n_kv+1], kq int32 [nnz]) of a list's reverse index from ``coo_rows_to_csr``'s (keys, in_order):
+    sorted by (kv, CSR position), as ``reverse_index`` gives them (a typed entry's type in bit 31 of kq)."""
+    keys, in_order = keys
+    dev = keys.device
+    nnz = keys.numel()
+    ws = _workspace(_size_query("bf_coo_reverse_workspace_size", nnz, n_q, n_kv, int(typed), int(in_order)), dev)
+    kptr = torch.empty(n_kv + 1, dtype=torch.int64, device=dev)
+    kq = torch.empty(max(nnz, 1), dtype=torch.int32, device=dev)[:nnz]
+    N.call("bf_coo_reverse", _p(keys), nnz, n_q, n_kv, int(typed), int(in_order), _p(kptr), _p(kq), _p(ws),
+           ws.numel(), _stream(dev))
+    return kptr, kq
+
+
+def coo_reverse_slots(qptr: torch.Tensor, kv: torch.Tensor, kptr: torch.Tensor, kq: torch.Tensor) -> torch.Tensor:
+    """ks (each reverse entry's slot in its query's row, int32) of an index whose rows ascend (bf_coo_reverse_slots)."""
+    ks = torch.empty(max(kq.numel(), 1), dtype=torch.int32, device=kq.device)[:kq.numel()]
+    N.call("bf_coo_reverse_slots", _p(qptr), _p(kv), _p(kptr), _p(kq), kq.numel(), kptr.numel() - 1, _p(ks),
+           _stream(kq.device))
+    return ks
 
 
 def reverse_index(qptr: torch.Tensor, kv: torch.Tensor, n_kv: int):
@@ -843,6 +923,7 @@ class AttentionIndex:
     _rows: Optional[torch.Tensor] = field(default=None, repr=False)
     _rkeys: Optional[ReverseKeys] = field(default=None, repr=False)   # from_table: sort keys, until used
     _sorted: Optional[ReverseKeys] = field(default=None, repr=False)  # sorted keys, until ks is needed
+    _coo_keys: Optional[tuple] = field(default=None, repr=False)      # from a COO list: coo_reverse's keys, until used
     _counts: Optional[torch.Tensor] = field(default=None, repr=False)  # both plans' device counts
     # True: the plans leave their counts on the device and the attention calls size their grids for the
     # capacities (no host read at all between building the index and using it, e.g. for a caller that
@@ -882,6 +963,8 @@ class AttentionIndex:
 
     @property
     def ks(self) -> Optional[torch.Tensor]:
+        if self.ks_all is None and self.kptr is not None and self._sorted is None and self.cap:
+            self.ensure_entries()           # a COO list's slots are searched on first use
         return None if self.ks_all is None else self.ks_all[:self.nnz]
 
     @property
@@ -927,6 +1010,11 @@ class AttentionIndex:
                 else:
                     self._sorted = srt
                 self._rkeys = None
+            elif self._coo_keys is not None:
+                self.kptr, self.kq_all = coo_reverse(self._coo_keys, self.n_q, self.n_kv, self.typed)
+                self._coo_keys = None
+                if entries:
+                    self.ks_all = coo_reverse_slots(self.qptr, self.kv_all, self.kptr, self.kq_all)
             else:
                 self.kptr, kq, ks = reverse_index(self.qptr, self.kv, self.n_kv)
                 self.kq_all, self.ks_all = _to_cap(kq, self.cap), _to_cap(ks, self.cap)
@@ -948,8 +1036,11 @@ class AttentionIndex:
         factor is indexed by."""
         self.ensure_backward()
         if self.ks_all is None and self.cap:
-            self.ks_all = reverse_slots(self._sorted, self.qptr)
-            self._sorted = None
+            if self._sorted is None:
+                self.ks_all = coo_reverse_slots(self.qptr, self.kv_all, self.kptr, self.kq_all)
+            else:
+                self.ks_all = reverse_slots(self._sorted, self.qptr)
+                self._sorted = None
         return self
 
     def entry_rows(self) -> torch.Tensor:
@@ -1095,24 +1186,22 @@ class AttentionIndex:
             raise ValueError(f"a typed edge set is [3, E] (got {tuple(edge_index.shape)})")
         if 2 * n_kv >= 2 ** 31 or n_q >= 2 ** 31:
             raise ValueError("typed indexes need n_q and 2 * n_kv below 2^31")
-        types = edge_index[2].to(torch.int64)
-        if types.numel() and (types.min().item() < 0 or types.max().item() > 1):
-            raise ValueError("edge types must be 0 or 1")
-        src = edge_index[0].to(torch.int64)
-        # rows ordered by (type, kv): the CSR of the type-shifted ids, then the type moved to bit 31
-        qptr, kvp = coo_to_csr(torch.stack([src + types * n_kv, edge_index[1].to(torch.int64)]), n_q, 2 * n_kv)
-        nnz = kvp.numel()
-        kvp = kvp.to(torch.int64)
-        one = kvp >= n_kv
-        kv_enc = torch.where(one, kvp - n_kv - 2 ** 31, kvp).to(torch.int32)
-        kptr, kq, ks = reverse_index(qptr, torch.where(one, kvp - n_kv, kvp).to(torch.int32), n_kv)
-        pos = qptr[kq.to(torch.int64)] + ks.to(torch.int64)
-        kq_enc = torch.where(kv_enc[pos] < 0, kq.to(torch.int64) - 2 ** 31, kq.to(torch.int64)).to(torch.int32)
-        idx = cls(n_q=n_q, n_kv=n_kv, qptr=qptr, kv_all=kv_enc, chunk=chunk, item=item, _nnz=nnz, typed=True)
-        # no split query rows: the query plan's threshold is above every row's length
-        idx.qplan = split_plan(qptr, nnz, min(nnz + 1, 2 ** 31 - 1), item, resolve=False,
-                               counts=idx._plan_counts(0), known=(0, 0), host_copy=False)
-        idx.kptr, idx.kq_all, idx.ks_all = kptr, kq_enc, ks
+        src, dst = _pair_lists(edge_index)
+        types = edge_index[2].to(torch.int64).contiguous()
+        try:
+            qptr, kv, keys = coo_rows_to_csr(dst, src, n_q, n_kv, types, with_keys=True)
+        except ValueError:
+            # an id is taken with its type as one number, id + type * n_kv below 2 * n_kv
+            both = src + types * n_kv
+            if types.min().item() < 0 or types.max().item() > 1 or both.min().item() < 0 or \
+                    both.max().item() >= 2 * n_kv:
+                raise
+            types = (both >= n_kv).to(torch.int64)
+            qptr, kv, keys = coo_rows_to_csr(dst, both - types * n_kv, n_q, n_kv, types, with_keys=True)
+        idx = cls(n_q=n_q, n_kv=n_kv, qptr=qptr, kv_all=kv, chunk=chunk, item=item, _nnz=kv.numel(), typed=True,
+                  _coo_keys=keys)
+        # no split query rows: a plan of none
+        idx.qplan = split_plan_first_row(n_q, 0, kv.numel(), kv.numel() + 1, item, idx._plan_counts(0))
         idx.ensure_backward()
         return idx
 
@@ -1120,8 +1209,11 @@ class AttentionIndex:
     def from_coo(cls, edge_index, n_q: int, n_kv: Optional[int] = None, chunk: int = DEFAULT_CHUNK,
                  item: int = DEFAULT_ITEM):
         n_kv = n_q if n_kv is None else n_kv
-        qptr, kv = coo_to_csr(edge_index, n_q, n_kv)
-        return cls(n_q=n_q, n_kv=n_kv, qptr=qptr, kv_all=kv, chunk=chunk, item=item, _nnz=kv.numel())
+        if edge_index.dim() != 2 or edge_index.size(0) < 2:
+            raise ValueError(f"edge_index must be [2, E] (got {tuple(edge_index.shape)})")
+        src, dst = _pair_lists(edge_index)
+        qptr, kv, keys = coo_rows_to_csr(dst, src, n_q, n_kv, with_keys=True)
+        return cls(n_q=n_q, n_kv=n_kv, qptr=qptr, kv_all=kv, chunk=chunk, item=item, _nnz=kv.numel(), _coo_keys=keys)
 
 
 # ------------------------------------------------------------------ attention

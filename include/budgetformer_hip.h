@@ -356,6 +356,49 @@ int bf_coo_to_csr_workspace_size(int64_t nnz, int64_t n_q, size_t* bytes);
 int bf_coo_to_csr(const int64_t* src, const int64_t* dst, int64_t nnz, int64_t n_q, int64_t n_kv,
                   int64_t* qptr, int32_t* kv, void* workspace, size_t workspace_bytes, void* stream);
 
+/* What order a COO list holds already: bits of *holds_host (BF_COO_*), each set
+ * when every entry (pair of neighbouring entries) keeps to it. row / col int64
+ * [nnz]; type (may be NULL) int64 [nnz] of 0 or 1, a column then being (type,
+ * col). The reference's lists come out of coalesce (gt_sp/utils.py:877-887),
+ * in (src, dst) order. One pass and one read back: synchronises the stream.
+ * Workspace: BF_COO_ORDER_WORKSPACE bytes.                                  */
+#define BF_COO_IDS 1         /* rows in [0, n_row), columns in [0, n_col)     */
+#define BF_COO_TYPES 2       /* types 0 or 1                                  */
+#define BF_COO_ROW_MAJOR 4   /* ascending by (row, column)                    */
+#define BF_COO_COL_MAJOR 8   /* ascending by (column, row)                    */
+#define BF_COO_STRICT 16     /* strictly ascending by (row, column)           */
+#define BF_COO_BY_COL 32     /* columns never descend                         */
+#define BF_COO_BY_ROW 64     /* rows never descend                            */
+#define BF_COO_ORDER_WORKSPACE 4096
+int bf_coo_order(const int64_t* row, const int64_t* col, const int64_t* type, int64_t nnz, int64_t n_row,
+                 int64_t n_col, int32_t* holds_host, void* workspace, size_t workspace_bytes, void* stream);
+
+/* bf_coo_to_csr for a list of known order: ptr int64 [n_row + 1], ids int32
+ * [nnz] ascending within a row (with type: by (type, id), the type in bit 31).
+ * holds: bf_coo_order's bits for the same list with BF_COO_IDS set, or 0 when
+ * nothing is known but that the ids are in range; the sort takes only the bits
+ * the list is not ordered by. rkeys (may be NULL) uint64 [nnz]: the entries'
+ * sort keys for bf_coo_reverse, whose `sorted` is 1 when holds has
+ * BF_COO_COL_MAJOR and type is NULL (they are then in reverse order already).
+ * (models/graphormer_dist_node_level.py:231-232,
+ * models/exphormer_dist_node_level.py:77-121.)                              */
+int bf_coo_to_csr_ordered_workspace_size(int64_t nnz, int64_t n_row, int64_t n_col, int32_t typed, int32_t holds,
+                                         size_t* bytes);
+int bf_coo_to_csr_ordered(const int64_t* row, const int64_t* col, const int64_t* type, int64_t nnz, int64_t n_row,
+                          int64_t n_col, int32_t holds, int64_t* ptr, int32_t* ids, uint64_t* rkeys,
+                          void* workspace, size_t workspace_bytes, void* stream);
+/* The reverse index of such a list from its rkeys: kptr int64 [n_col + 1] and
+ * kq int32 [nnz] in (column, CSR position) order, as bf_reverse_index gives
+ * them (a typed entry's type in bit 31 of kq). The entries' slots, which only
+ * a bias, factor or dropout needs, come from bf_coo_reverse_slots: a search of
+ * each entry's place in its query's ascending row.                          */
+int bf_coo_reverse_workspace_size(int64_t nnz, int64_t n_row, int64_t n_col, int32_t typed, int32_t sorted,
+                                  size_t* bytes);
+int bf_coo_reverse(const uint64_t* rkeys, int64_t nnz, int64_t n_row, int64_t n_col, int32_t typed, int32_t sorted,
+                   int64_t* kptr, int32_t* kq, void* workspace, size_t workspace_bytes, void* stream);
+int bf_coo_reverse_slots(const int64_t* qptr, const int32_t* kv, const int64_t* kptr, const int32_t* kq, int64_t nnz,
+                         int64_t n_kv, int32_t* ks, void* stream);
+
 /* Coalesce of a COO edge list: torch_geometric.utils.coalesce as used by
  * _merge_edge_index_list (gt_sp/utils.py:877-887): sorted by (src, dst) with
  * duplicates removed. out_src / out_dst int64 need capacity nnz; the number of
@@ -365,6 +408,13 @@ int bf_coalesce_workspace_size(int64_t nnz, size_t* bytes);
 int bf_coalesce(const int64_t* src, const int64_t* dst, int64_t nnz, int64_t num_nodes,
                 int64_t* out_src, int64_t* out_dst, int64_t* count_host,
                 void* workspace, size_t workspace_bytes, void* stream);
+/* The same of the list and its mirror image (_to_bidirected_edge_index,
+ * utils/fullgraph_sp_support.py:570-572), neither of them written out first:
+ * out_src / out_dst need capacity 2 * nnz. Workspace:
+ * bf_coalesce_workspace_size(2 * nnz).                                      */
+int bf_coalesce_bidirected(const int64_t* src, const int64_t* dst, int64_t nnz, int64_t num_nodes,
+                           int64_t* out_src, int64_t* out_dst, int64_t* count_host,
+                           void* workspace, size_t workspace_bytes, void* stream);
 
 /* Reverse (key-major) index of an attention CSR: kptr int64 [n_kv+1], and for
  * each reverse entry its query kq int32 [nnz] and its slot ks int32 [nnz] (its

@@ -1,0 +1,97 @@
+"""An edge list's index (coo_rows_to_csr, coo_reverse, coo_reverse_slots) and its coalesced form against numpy, for
+every order a list can come in: none, column order, coalesced (column-major), row-major, with repeated entries,
+typed or not, and the two lists the sorts never see (empty, one entry). Integer work: bit-exact."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+N_Q, N_KV = 70, 4000
+
+
+def _list(order, nnz, typed, seed):
+    rng = np.random.default_rng(seed)
+    kv = np.minimum((N_KV * rng.random(nnz) ** 3).astype(np.int64), N_KV - 3)     # skewed, the last ids unused
+    q = rng.integers(0, N_Q - 2, nnz)
+    t = rng.integers(0, 2, nnz) if typed else np.zeros(nnz, dtype=np.int64)
+    if nnz > 20:
+        kv[10:14], q[10:14], t[10:14] = kv[10], q[10], t[10]                       # a pair four times over
+    keys = {"none": None, "by_col": (kv, t), "col_major": (q, kv, t), "row_major": (kv, t, q)}[order]
+    if keys is not None:
+        o = np.lexsort(keys)
+        kv, q, t = kv[o], q[o], t[o]
+    return kv, q, t
+
+
+@pytest.mark.parametrize("typed", [False, True])
+@pytest.mark.parametrize("order", ["none", "by_col", "col_major", "row_major"])
+@pytest.mark.parametrize("nnz", [1, 1023, 1024, 70_001])
+def test_list_index_in_every_order(hip_device, order, nnz, typed):
+    from budgetformer_amd import hip_ops
+    kv, q, t = _list(order, nnz, typed, nnz)
+    dev = [torch.from_numpy(x).to(hip_device) for x in (q, kv, t)]
+    qptr, ids, keys = hip_ops.coo_rows_to_csr(dev[0], dev[1], N_Q, N_KV, dev[2] if typed else None, with_keys=True)
+    kptr, kq = hip_ops.coo_reverse(keys, N_Q, N_KV, typed)
+    ks = hip_ops.coo_reverse_slots(qptr, ids, kptr, kq)
+    o = np.lexsort((kv, t, q))                       # rows ascend by (type, kv)
+    kv, q, t = kv[o], q[o], t[o]
+    slot = np.arange(nnz) - np.searchsorted(q, q)
+    assert np.array_equal(qptr.cpu().numpy(), np.searchsorted(q, np.arange(N_Q + 1)))
+    assert np.array_equal(ids.cpu().numpy().view(np.uint32), (kv | (t << 31)).astype(np.uint32))
+    r = np.argsort(kv, kind="stable")
+    assert np.array_equal(kptr.cpu().numpy(), np.searchsorted(kv[r], np.arange(N_KV + 1)))
+    assert np.array_equal(kq.cpu().numpy().view(np.uint32), (q[r] | (t[r] << 31)).astype(np.uint32))
+    assert np.array_equal(ks.cpu().numpy(), slot[r])
+    if not typed:
+        ref = hip_ops.reverse_index(qptr, ids, N_KV)
+        assert all(torch.equal(a, b) for a, b in zip((kptr, kq, ks), ref))
+
+
+def test_typed_index_takes_an_id_and_its_type_as_one_number(hip_device):
+    """(n_kv + i, type 0) is (i, type 1); what no pair gives is refused."""
+    from budgetformer_amd.hip_ops import AttentionIndex
+    ei = torch.tensor([[3, 5, 1], [0, 1, 1], [0, 1, 0]], device=hip_device)
+    same = torch.tensor([[3, 15, 1], [0, 1, 1], [0, 0, 0]], device=hip_device)
+    a, b = AttentionIndex.from_typed_coo(ei, 2, 10), AttentionIndex.from_typed_coo(same, 2, 10)
+    assert torch.equal(a.kv, b.kv) and torch.equal(a.kq, b.kq) and torch.equal(a.ks, b.ks)
+    for bad, what in (([[20], [0], [0]], "ids outside"), ([[3], [2], [0]], "ids outside"), ([[3], [0], [2]], "types")):
+        with pytest.raises(ValueError, match=what):
+            AttentionIndex.from_typed_coo(torch.tensor(bad, device=hip_device), 2, 10)
+    for bad in ([[10], [0]], [[-1], [0]], [[0], [2]], [[0], [-1]]):
+        with pytest.raises(ValueError, match="ids outside"):
+            AttentionIndex.from_coo(torch.tensor(bad, device=hip_device), 2, 10)
+
+
+def test_slots_of_a_list_index_come_on_first_use(hip_device):
+    from budgetformer_amd.hip_ops import AttentionIndex
+    kv, q, _ = _list("none", 3000, False, 5)
+    ei = torch.from_numpy(np.stack([kv, q])).to(hip_device)
+    a = AttentionIndex.from_coo(ei, N_Q, N_KV).ensure_backward()
+    assert a.ks_all is None
+    b = AttentionIndex.from_coo(ei, N_Q, N_KV).ensure_backward(entries=True)
+    assert b.ks_all is not None and torch.equal(a.ks, b.ks) and torch.equal(a.to_coo(), b.to_coo())
+    empty = AttentionIndex.from_coo(ei[:, :0], N_Q, N_KV).ensure_backward()
+    assert empty.nnz == 0 and int(empty.qptr[-1]) == 0 and int(empty.kptr[-1]) == 0
+
+
+@pytest.mark.parametrize("nnz", [0, 1, 4096, 4097, 100_003])
+@pytest.mark.parametrize("n", [50, 3001])
+def test_coalesce_and_bidirected(hip_device, nnz, n):
+    """Many duplicates (50 nodes) and few; a coalesced list comes back equal, in memory of its own."""
+    from budgetformer_amd import hip_ops
+    from budgetformer_amd.graph import to_bidirected
+    rng = np.random.default_rng(nnz + n)
+    ei = rng.integers(0, n, (2, nnz))
+
+    def ref(x):
+        return np.stack(np.divmod(np.unique(x[0] * n + x[1]), n)) if x.size else x
+
+    dev = torch.from_numpy(ei).to(hip_device)
+    got = hip_ops.coalesce(dev, n)
+    assert np.array_equal(got.cpu().numpy(), ref(ei))
+    assert np.array_equal(to_bidirected(dev, n).cpu().numpy(), ref(np.concatenate([ei, ei[::-1]], axis=1)))
+    again = hip_ops.coalesce(got, n)
+    assert torch.equal(again, got) and (nnz == 0 or again.data_ptr() != got.data_ptr())
+    assert hip_ops.coalesced(again, n) is again or nnz == 0
+    assert np.array_equal(hip_ops.coalesced(dev, n).cpu().numpy(), ref(ei))
