@@ -1726,14 +1726,23 @@ __global__ __launch_bounds__(kBlock) void attn_bwd_q_typed_kernel(
 }
 
 // out[b][c] = sum of rec[r][c] over records r in [b * per_block, (b + 1) * per_block), in record order
-// (cols floats per record): one pass of the fixed-order reduction of the dE records.
+// (cols floats per record): one pass of the fixed-order reduction of the dE records. The sum is one chain of
+// dependent adds per column, so its loads are issued kModUnroll at a time ahead of them.
+constexpr int kModUnroll = 16;
+
 __global__ __launch_bounds__(kBlock) void mod_rec_reduce_kernel(const float* __restrict__ rec, int64_t n_rec, int cols,
                                                                 int64_t per_block, float* __restrict__ out) {
   const int64_t r0 = int64_t(blockIdx.x) * per_block;
   const int64_t r1 = r0 + per_block < n_rec ? r0 + per_block : n_rec;
   for (int c = threadIdx.x; c < cols; c += kBlock) {
     float s = 0.f;
-    for (int64_t r = r0; r < r1; ++r) s += rec[r * cols + c];
+    for (int64_t r = r0; r < r1; r += kModUnroll) {
+      float x[kModUnroll];
+#pragma unroll
+      for (int u = 0; u < kModUnroll; ++u) x[u] = r + u < r1 ? rec[(r + u) * cols + c] : 0.f;
+#pragma unroll
+      for (int u = 0; u < kModUnroll; ++u) s += x[u];
+    }
     out[int64_t(blockIdx.x) * cols + c] = s;
   }
 }
@@ -2035,7 +2044,10 @@ inline int64_t typed_q_blocks(int64_t n_q, const Shape& sh) {
   return int64_t(grid_for(ceil_div(n_q, typed_rows_per_group(n_q, sh)), sh));
 }
 
-constexpr int64_t kModRecPerBlock = 256;   // dE records summed per workgroup in the first reduce pass
+// dE records summed per workgroup in the first reduce pass. About the square root of the records of a large
+// query set (2344 at 600K queries), so that neither pass is a long chain on a few workgroups: 256 records on 10
+// workgroups, then 10, took 104 us (now 10).
+constexpr int64_t kModRecPerBlock = 48;
 
 int check_typed(const bf_attn_index* idx, const float* mod) {
   BF_CHECK_ARG(mod != nullptr, "attn typed: type_mod is NULL");
