@@ -102,6 +102,11 @@ _SIGS = {
     "bf_coo_reverse_workspace_size": (C.c_int, [i64, i64, i64, i32, i32, C.POINTER(sz)]),
     "bf_coo_reverse": (C.c_int, [vp, i64, i64, i64, i32, i32, P_i64, P_i32, vp, sz, vp]),
     "bf_coo_reverse_slots": (C.c_int, [P_i64, P_i32, P_i64, P_i32, i64, i64, P_i32, vp]),
+    "bf_table_list_check_workspace_size": (C.c_int, [i64, C.POINTER(sz)]),
+    "bf_table_list_check": (C.c_int, [P_i32, P_i32, i64, i32, i64, C.POINTER(i64), vp, sz, vp]),
+    "bf_table_to_list_workspace_size": (C.c_int, [i64, i64, C.POINTER(sz)]),
+    "bf_table_to_list": (C.c_int, [P_i32, P_i32, i64, i32, i64, i64, P_i32, i64, i32, i64, i64, i64, vp, P_i64, vp, sz,
+                                   vp]),
     "bf_reverse_index_workspace_size": (C.c_int, [i64, i64, C.POINTER(sz)]),
     "bf_reverse_index": (C.c_int, [P_i64, P_i32, i64, i64, i64, P_i64, P_i32, P_i32, vp, sz, vp]),
     "bf_reverse_index_packed_workspace_size": (C.c_int, [i64, C.POINTER(sz)]),

@@ -11,6 +11,8 @@
 // Against the former route (four torch reductions with three host reads, a
 // 64-bit onesweep sort over all bits, separate passes for the ids and the row
 // pointers) a 1.17M-entry list's CSR went from 430 to 190 us, host reads included.
+#include <vector>
+
 #include "bf_common.h"
 #include "bf_sort.h"
 
@@ -288,6 +290,150 @@ __global__ __launch_bounds__(kThreads) void unique_write_kernel(const uint64_t* 
   }
 }
 
+// ---------------------------------------------------------------- table -> list
+// A table's edge list in coalesce order without its CSR: a block of kListRows table rows checks its lengths and
+// ids and adds up its lengths (bf_table_list_check), writes its entries' keys id << qb | row at the places that
+// follow from the blocks before it, and the keys sorted by id are the list. The virtual node's entries have
+// fixed places behind them and are written with the list.
+constexpr int kListRows = 512;
+constexpr int kListWidth32 = 1 << 22;    // kListRows rows of at most this many slots are numbered in 32 bits
+
+// Row lengths of block b's rows into LDS, those outside [0, width] as 0 (and counted).
+__device__ __forceinline__ uint32_t list_lengths(const int32_t* __restrict__ row_len, int64_t n_rows, int width,
+                                                 int32_t (&len)[kListRows]) {
+  uint32_t bad = 0;
+#pragma unroll
+  for (int u = 0; u < kListRows / kThreads; ++u) {
+    const int j = u * kThreads + threadIdx.x;
+    const int64_t r = int64_t(blockIdx.x) * kListRows + j;
+    int32_t l = r < n_rows ? row_len[r] : 0;
+    if (l < 0 || l > width) {
+      ++bad;
+      l = 0;
+    }
+    len[j] = l;
+  }
+  return bad;
+}
+
+__device__ __forceinline__ uint32_t block_sum(uint32_t v, uint32_t* wave /*[kThreads / 64]*/) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  __syncthreads();                       // an earlier sum's words are read
+  if ((threadIdx.x & 63) == 0) wave[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return wave[0] + wave[1] + wave[2] + wave[3];
+}
+
+template <typename I>   // of a slot within the block: 32 bits unless the rows are very wide
+__global__ __launch_bounds__(kThreads) void table_list_check_kernel(const int32_t* __restrict__ table,
+                                                                    const int32_t* __restrict__ row_len,
+                                                                    int64_t n_rows, int width, int64_t id_limit,
+                                                                    uint32_t* __restrict__ sums,
+                                                                    uint32_t* __restrict__ bad) {
+  __shared__ int32_t len[kListRows];
+  __shared__ uint32_t wave[kThreads / 64];
+  const uint32_t bad_len = list_lengths(row_len, n_rows, width, len);
+  __syncthreads();
+  uint32_t total = 0, bad_id = 0;
+#pragma unroll
+  for (int u = 0; u < kListRows / kThreads; ++u) total += uint32_t(len[u * kThreads + threadIdx.x]);
+  const int64_t r0 = int64_t(blockIdx.x) * kListRows;
+  const int rows = int(n_rows - r0 < kListRows ? n_rows - r0 : kListRows);
+  const I slots = I(rows) * I(width);
+  const int32_t* t = table + r0 * width;
+  for (I i0 = threadIdx.x; i0 < slots; i0 += kThreads * kPerThread) {
+    int32_t id[kPerThread];
+#pragma unroll
+    for (int u = 0; u < kPerThread; ++u) id[u] = i0 + u * kThreads < slots ? t[i0 + u * kThreads] : 0;
+#pragma unroll
+    for (int u = 0; u < kPerThread; ++u) {
+      const I i = i0 + u * kThreads;
+      if (i >= slots) break;
+      const uint32_t r = uint32_t(i / I(width)), c = uint32_t(i - I(r) * I(width));
+      bad_id += (int32_t(c) < len[r] && (id[u] < 0 || int64_t(id[u]) >= id_limit)) ? 1u : 0u;
+    }
+  }
+  const uint32_t s = block_sum(total, wave), bl = block_sum(bad_len, wave), bi = block_sum(bad_id, wave);
+  if (threadIdx.x == 0) {
+    sums[blockIdx.x] = s;                  // a list of 2^31 entries or more is refused on the host
+    bad[2 * int64_t(blockIdx.x)] = bl;
+    bad[2 * int64_t(blockIdx.x) + 1] = bi;
+  }
+}
+
+template <typename I>   // of a slot within the block: 32 bits unless the rows are very wide
+__global__ __launch_bounds__(kThreads) void table_list_keys_kernel(const int32_t* __restrict__ table,
+                                                                   const int32_t* __restrict__ row_len,
+                                                                   int64_t n_rows, int width,
+                                                                   const uint32_t* __restrict__ prefix, int qb,
+                                                                   uint64_t* __restrict__ keys) {
+  __shared__ int32_t len[kListRows];
+  __shared__ uint32_t off[kListRows];
+  __shared__ uint32_t tmp[kThreads / 64];
+  list_lengths(row_len, n_rows, width, len);
+  __syncthreads();
+  constexpr int kRows = kListRows / kThreads;      // consecutive rows per thread
+  uint32_t mine = 0, total;
+#pragma unroll
+  for (int u = 0; u < kRows; ++u) mine += uint32_t(len[threadIdx.x * kRows + u]);
+  uint32_t at = sort::block_excl_scan<kThreads>(mine, tmp, &total) + prefix[blockIdx.x];
+#pragma unroll
+  for (int u = 0; u < kRows; ++u) {
+    off[threadIdx.x * kRows + u] = at;
+    at += uint32_t(len[threadIdx.x * kRows + u]);
+  }
+  __syncthreads();
+  const int64_t r0 = int64_t(blockIdx.x) * kListRows;
+  const int rows = int(n_rows - r0 < kListRows ? n_rows - r0 : kListRows);
+  const I slots = I(rows) * I(width);
+  const int32_t* t = table + r0 * width;
+  for (I i0 = threadIdx.x; i0 < slots; i0 += kThreads * kPerThread) {
+    int32_t id[kPerThread];
+#pragma unroll
+    for (int u = 0; u < kPerThread; ++u) id[u] = i0 + u * kThreads < slots ? t[i0 + u * kThreads] : 0;
+#pragma unroll
+    for (int u = 0; u < kPerThread; ++u) {
+      const I i = i0 + u * kThreads;
+      if (i >= slots) break;
+      const uint32_t r = uint32_t(i / I(width)), c = uint32_t(i - I(r) * I(width));
+      if (int32_t(c) < len[r]) keys[off[r] + c] = (uint64_t(uint32_t(id[u])) << qb) | uint64_t(r0 + r);
+    }
+  }
+}
+
+// The list: out[0..total) the sources, out[total..2 total) the queries. Entry i < nnz is key i; then token_row
+// entries (v + 1 -> 0), then token_col entries (0 -> token_q0 + j).
+__global__ __launch_bounds__(kThreads) void list_write_kernel(const uint64_t* __restrict__ keys, int64_t nnz, int qb,
+                                                              const int32_t* __restrict__ query_ids, int64_t q_lo,
+                                                              int shift, int64_t token_row, int64_t token_q0,
+                                                              int64_t total, int64_t* __restrict__ out) {
+  const int64_t base = int64_t(blockIdx.x) * (kThreads * kPerThread) + threadIdx.x;
+  uint64_t k[kPerThread];
+#pragma unroll
+  for (int u = 0; u < kPerThread; ++u) {
+    const int64_t i = base + int64_t(u) * kThreads;
+    k[u] = i < nnz ? keys[i] : 0;
+  }
+#pragma unroll
+  for (int u = 0; u < kPerThread; ++u) {
+    const int64_t i = base + int64_t(u) * kThreads;
+    if (i >= total) break;
+    int64_t src, dst;
+    if (i < nnz) {
+      const int64_t row = int64_t(k[u] & ((uint64_t(1) << qb) - 1));
+      src = int64_t(k[u] >> qb) + shift;
+      dst = (query_ids ? int64_t(query_ids[row]) : q_lo + row) + shift;
+    } else {
+      const int64_t j = i - nnz;
+      src = j < token_row ? j + 1 : 0;
+      dst = j < token_row ? 0 : token_q0 + (j - token_row);
+    }
+    out[i] = src;
+    out[total + i] = dst;
+  }
+}
+
 struct Carve {            // consecutive 256-byte aligned pieces of a workspace
   char* p;
   template <typename T>
@@ -514,4 +660,108 @@ extern "C" int bf_coalesce_bidirected(const int64_t* src, const int64_t* dst, in
   BF_CHECK_ARG(src && dst && out_src && out_dst, "coalesce_bidirected: null tensor");
   return coalesce_list(PairKeys{src, dst, nnz, uint64_t(num_nodes)}, 2 * nnz, num_nodes, out_src, out_dst, count_host,
                        workspace, workspace_bytes, as_stream(stream));
+}
+
+namespace {
+int64_t list_blocks(int64_t n_rows) { return ceil_div(n_rows, int64_t(kListRows)); }
+size_t list_sums_bytes(int64_t n_rows) { return align_up(size_t(list_blocks(n_rows)) * 4 + 4); }
+}  // namespace
+
+extern "C" int bf_table_list_check_workspace_size(int64_t n_rows, size_t* bytes) {
+  BF_CHECK_ARG(bytes && n_rows >= 0, "table_list_check_workspace_size: bad arguments");
+  *bytes = list_sums_bytes(n_rows) + align_up(size_t(list_blocks(n_rows)) * 8) + 256;
+  return BF_OK;
+}
+
+extern "C" int bf_table_list_check(const int32_t* table, const int32_t* row_len, int64_t n_rows, int32_t width,
+                                   int64_t id_limit, int64_t* nnz_host, void* workspace, size_t workspace_bytes,
+                                   void* stream) {
+  BF_CHECK_ARG(n_rows >= 0 && width >= 0 && id_limit >= 0 && nnz_host,
+               "table_list_check: bad arguments");
+  *nnz_host = 0;
+  if (n_rows == 0) return BF_OK;
+  BF_CHECK_ARG((table || width == 0) && row_len, "table_list_check: null tensor");
+  size_t need = 0;
+  BF_CHECK_OK(bf_table_list_check_workspace_size(n_rows, &need));
+  BF_CHECK_ARG(workspace && workspace_bytes >= need, "table_list_check: workspace %zu < %zu bytes", workspace_bytes,
+               need);
+  hipStream_t st = as_stream(stream);
+  const int64_t blocks = list_blocks(n_rows);
+  auto* sums = static_cast<uint32_t*>(workspace);
+  auto* bad = reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) + list_sums_bytes(n_rows));
+  if (width <= kListWidth32)
+    BF_LAUNCH("table_list_check_kernel", table_list_check_kernel<uint32_t>, dim3(unsigned(blocks)), dim3(kThreads), 0,
+              st, table, row_len, n_rows, width, id_limit, sums, bad);
+  else
+    BF_LAUNCH("table_list_check_kernel", table_list_check_kernel<uint64_t>, dim3(unsigned(blocks)), dim3(kThreads), 0,
+              st, table, row_len, n_rows, width, id_limit, sums, bad);
+  BF_CHECK_LAUNCH();
+  std::vector<uint32_t> h(size_t(blocks) * 3);
+  BF_CHECK_HIP(hipMemcpyAsync(h.data(), sums, size_t(blocks) * 4, hipMemcpyDeviceToHost, st));
+  BF_CHECK_HIP(hipMemcpyAsync(h.data() + blocks, bad, size_t(blocks) * 8, hipMemcpyDeviceToHost, st));
+  BF_CHECK_HIP(hipStreamSynchronize(st));
+  int64_t nnz = 0, bad_len = 0, bad_id = 0;
+  for (int64_t b = 0; b < blocks; ++b) {
+    nnz += h[size_t(b)];
+    bad_len += h[size_t(blocks + 2 * b)];
+    bad_id += h[size_t(blocks + 2 * b + 1)];
+  }
+  BF_CHECK_ARG(bad_len == 0, "check_table: %lld row lengths outside [0, %d]", (long long)bad_len, width);
+  BF_CHECK_ARG(bad_id == 0, "check_table: %lld table ids outside [0, %lld)", (long long)bad_id, (long long)id_limit);
+  BF_CHECK_ARG(nnz < (int64_t(1) << 31), "table_list_check: %lld entries (at most 2^31 - 1)", (long long)nnz);
+  *nnz_host = nnz;
+  return BF_OK;
+}
+
+extern "C" int bf_table_to_list_workspace_size(int64_t nnz, int64_t id_limit, size_t* bytes) {
+  BF_CHECK_ARG(bytes && nnz >= 0 && id_limit >= 0, "table_to_list_workspace_size: bad arguments");
+  *bytes = 256;
+  if (nnz == 0) return BF_OK;
+  *bytes += 2 * align_up(size_t(nnz) * 8) +
+            sort::workspace_bytes(nnz, bits_for(uint64_t(id_limit > 0 ? id_limit - 1 : 0)));
+  return BF_OK;
+}
+
+extern "C" int bf_table_to_list(const int32_t* table, const int32_t* row_len, int64_t n_rows, int32_t width,
+                                int64_t nnz, int64_t id_limit, const int32_t* query_ids, int64_t q_lo, int32_t shift,
+                                int64_t token_row, int64_t token_q0, int64_t token_col, void* checked,
+                                int64_t* out, void* workspace, size_t workspace_bytes, void* stream) {
+  BF_CHECK_ARG(n_rows >= 0 && n_rows < (int64_t(1) << 31) && width >= 0 && nnz >= 0 &&
+                   id_limit >= 0 && id_limit < (int64_t(1) << 31) && token_row >= 0 && token_col >= 0,
+               "table_to_list: bad arguments");
+  const int64_t total = nnz + token_row + token_col;
+  if (total == 0) return BF_OK;
+  size_t need = 0;
+  BF_CHECK_OK(bf_table_to_list_workspace_size(nnz, id_limit, &need));
+  BF_CHECK_ARG(out && workspace && workspace_bytes >= need, "table_to_list: workspace %zu < %zu bytes",
+               workspace_bytes, need);
+  hipStream_t st = as_stream(stream);
+  const int qb = bits_for(uint64_t(n_rows > 0 ? n_rows - 1 : 0));
+  const int ib = bits_for(uint64_t(id_limit > 0 ? id_limit - 1 : 0));
+  uint64_t* sorted = nullptr;
+  if (nnz > 0) {
+    BF_CHECK_ARG(table && row_len && checked, "table_to_list: null tensor");
+    Carve ws{static_cast<char*>(workspace)};
+    auto* keys = ws.take<uint64_t>(size_t(nnz) * 8);
+    sorted = ws.take<uint64_t>(size_t(nnz) * 8);
+    const int64_t blocks = list_blocks(n_rows);
+    auto* sums = static_cast<uint32_t*>(checked);    // become the blocks' first places
+    BF_LAUNCH("radix_scan_kernel", sort::radix_scan_kernel, dim3(1), dim3(sort::kThreads), 0, st, sums, blocks,
+              sums + blocks);
+    BF_CHECK_LAUNCH();
+    if (width <= kListWidth32)
+      BF_LAUNCH("table_list_keys_kernel", table_list_keys_kernel<uint32_t>, dim3(unsigned(blocks)), dim3(kThreads), 0,
+                st, table, row_len, n_rows, width, sums, qb, keys);
+    else
+      BF_LAUNCH("table_list_keys_kernel", table_list_keys_kernel<uint64_t>, dim3(unsigned(blocks)), dim3(kThreads), 0,
+                st, table, row_len, n_rows, width, sums, qb, keys);
+    BF_CHECK_LAUNCH();
+    // stable over the id bits: each id's entries stay in row order
+    BF_CHECK_OK(sort::radix_sort(sort::StoredKeys{keys}, sorted, nnz, qb, qb + ib, ws.p,
+                                 workspace_bytes - size_t(ws.p - static_cast<char*>(workspace)), st));
+  }
+  BF_LAUNCH("list_write_kernel", list_write_kernel, dim3(unsigned(ceil_div(total, int64_t(kThreads) * kPerThread))),
+            dim3(kThreads), 0, st, sorted, nnz, qb, query_ids, q_lo, shift, token_row, token_q0, total, out);
+  BF_CHECK_LAUNCH();
+  return BF_OK;
 }

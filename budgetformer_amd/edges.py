@@ -83,27 +83,17 @@ class EdgeTable:
         v] when this table holds the token row, then [0 -> (q+1)] for each of
         its queries q (all N for a full build).
         """
-        base = AttentionIndex.from_table(self.table, self.row_len, False, n_kv=self.num_nodes)
-        coo = base.to_coo()
-        if self.query_ids is not None:
-            coo = torch.stack([coo[0], self.query_ids.to(torch.int64)[coo[1]]])
-        elif self.q_lo:
-            coo = torch.stack([coo[0], coo[1] + self.q_lo])
-        if not self.global_token:
-            return coo
-        n = self.num_nodes
-        ar = torch.arange(1, n + 1, dtype=torch.int64, device=coo.device)
-        if self.query_ids is not None:
+        n, q_lo = self.num_nodes, 0 if self.query_ids is not None else self.q_lo
+        token = {}
+        if self.global_token and self.query_ids is not None:
             # a filtered (probe) build keeps every virtual edge, as the reference applies fix_edge_index
             # to the whole probe edge set
-            return torch.cat([coo + 1, torch.stack([ar, torch.zeros_like(ar)]),
-                              torch.stack([torch.zeros_like(ar), ar])], dim=1)
-        qs = torch.arange(self.q_lo + 1, self.q_lo + self.n_rows + 1, dtype=torch.int64, device=coo.device)
-        parts = [coo + 1]
-        if self.holds_token_row:
-            parts.append(torch.stack([ar, torch.zeros_like(ar)]))
-        parts.append(torch.stack([torch.zeros_like(qs), qs]))
-        return torch.cat(parts, dim=1)
+            token = {"shift": 1, "token_row": n, "token_col": n}
+        elif self.global_token:
+            token = {"shift": 1, "token_row": n if self.holds_token_row else 0, "token_q0": q_lo + 1,
+                     "token_col": self.n_rows}
+        ids = None if self.query_ids is None else self.query_ids.to(torch.int32).contiguous()
+        return hip_ops.table_to_list(self.table, self.row_len, n, q_lo, ids, **token)
 
 
 def build_attention_edges(graph: CSRGraph, *, real_edges_per_query: int, rw_edges_per_query: int,

@@ -549,6 +549,35 @@ def table_to_csr(table: torch.Tensor, row_len: torch.Tensor, global_token: bool 
     return (qptr, kv, rk) if with_keys else (qptr, kv)
 
 
+def table_to_list(table: torch.Tensor, row_len: torch.Tensor, num_nodes: int, q_lo: int = 0,
+                  query_ids: Optional[torch.Tensor] = None, shift: int = 0, token_row: int = 0, token_q0: int = 1,
+                  token_col: int = 0) -> torch.Tensor:
+    """The table's edge list [2, E] int64 in (src, dst) order with ids raised by ``shift``, then ``token_row`` edges
+    (v+1 -> 0) and ``token_col`` edges (0 -> token_q0 + j) (bf_table_to_list). The table is checked on the device
+    (ValueError, as ``check_table``) in the pass that counts its entries: one host read."""
+    dev = table.device
+    _require(table, "table", torch.int32)
+    _require(row_len, "row_len", torch.int32, dev)
+    if table.dim() != 2 or row_len.shape != (table.shape[0],):
+        raise ValueError("table must be [n, width] and row_len [n]")
+    n_rows, width = table.shape
+    if query_ids is not None:
+        _require(query_ids, "query_ids", torch.int32, dev)
+        if query_ids.numel() != n_rows:
+            raise ValueError(f"query_ids must hold one id per table row ({n_rows})")
+    stream = _stream(dev)
+    checked = _workspace(_size_query("bf_table_list_check_workspace_size", n_rows), dev)
+    cnt = C.c_int64(0)
+    N.call("bf_table_list_check", _p(table), _p(row_len), n_rows, width, int(num_nodes), C.byref(cnt), _p(checked),
+           checked.numel(), stream)
+    nnz = cnt.value
+    out = torch.empty(2, nnz + token_row + token_col, dtype=torch.int64, device=dev)
+    ws = _workspace(_size_query("bf_table_to_list_workspace_size", nnz, int(num_nodes)), dev)
+    N.call("bf_table_to_list", _p(table), _p(row_len), n_rows, width, nnz, int(num_nodes), _p(query_ids), int(q_lo),
+           int(shift), int(token_row), int(token_q0), int(token_col), _p(checked), _p(out), _p(ws), ws.numel(), stream)
+    return out
+
+
 def split_row_items(length: int, item_size: int = DEFAULT_ITEM) -> int:
     """Items a split row of ``length`` entries is cut into (bf_split_row_items)."""
     return int(N.load().bf_split_row_items(int(length), int(item_size)))

@@ -416,6 +416,27 @@ int bf_coalesce_bidirected(const int64_t* src, const int64_t* dst, int64_t nnz, 
                            int64_t* out_src, int64_t* out_dst, int64_t* count_host,
                            void* workspace, size_t workspace_bytes, void* stream);
 
+/* A query-major table's edge list in the reference's form: int64 out[2][total]
+ * (row 0 key/value node, row 1 query), the table's entries in (src, dst) order
+ * as coalesce leaves them (gt_sp/utils.py:877-887), ids raised by `shift`, then
+ * the Graphormer virtual edges fix_edge_index appends (gt_sp/utils.py:113-130):
+ * token_row entries (v+1 -> 0) and token_col entries (0 -> token_q0 + j). Row r
+ * is query query_ids[r], or q_lo + r without query_ids.
+ * bf_table_list_check validates the table as bf_check_table does (lengths in
+ * [0, width], ids in [0, id_limit): else BF_ERR_INVALID) and returns its entry
+ * count; it synchronises the stream. Its workspace
+ * (bf_table_list_check_workspace_size) goes to bf_table_to_list as `checked`,
+ * which consumes it; out holds total = nnz + token_row + token_col per row.
+ * Workspace: bf_table_to_list_workspace_size.                               */
+int bf_table_list_check_workspace_size(int64_t n_rows, size_t* bytes);
+int bf_table_list_check(const int32_t* table, const int32_t* row_len, int64_t n_rows, int32_t width,
+                        int64_t id_limit, int64_t* nnz_host, void* workspace, size_t workspace_bytes, void* stream);
+int bf_table_to_list_workspace_size(int64_t nnz, int64_t id_limit, size_t* bytes);
+int bf_table_to_list(const int32_t* table, const int32_t* row_len, int64_t n_rows, int32_t width, int64_t nnz,
+                     int64_t id_limit, const int32_t* query_ids, int64_t q_lo, int32_t shift, int64_t token_row,
+                     int64_t token_q0, int64_t token_col, void* checked, int64_t* out, void* workspace,
+                     size_t workspace_bytes, void* stream);
+
 /* Reverse (key-major) index of an attention CSR: kptr int64 [n_kv+1], and for
  * each reverse entry its query kq int32 [nnz] and its slot ks int32 [nnz] (its
  * position in the query's row: CSR position = qptr[kq] + ks), sorted by (kv,

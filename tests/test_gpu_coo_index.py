@@ -95,3 +95,41 @@ def test_coalesce_and_bidirected(hip_device, nnz, n):
     assert torch.equal(again, got) and (nnz == 0 or again.data_ptr() != got.data_ptr())
     assert hip_ops.coalesced(again, n) is again or nnz == 0
     assert np.array_equal(hip_ops.coalesced(dev, n).cpu().numpy(), ref(ei))
+
+
+@pytest.mark.parametrize("token", [False, True])
+@pytest.mark.parametrize("how", ["full", "shard", "ids"])
+@pytest.mark.parametrize("n_rows,width", [(1, 1), (511, 3), (513, 8), (5000, 33)])
+def test_table_to_list_equals_the_index_route(hip_device, n_rows, width, how, token):
+    """A table's list against its CSR's reverse index (the route it replaces) and fix_edge_index's order; rows empty,
+    full and past a block of rows, one row with the multiset's repeated id; bad tables refused."""
+    from budgetformer_amd.edges import EdgeTable
+    from budgetformer_amd.hip_ops import AttentionIndex
+    rng = np.random.default_rng(n_rows + width)
+    n = 6000
+    ids = np.sort(np.minimum((n * rng.random((n_rows, width)) ** 3).astype(np.int32), n - 1), axis=1)
+    ids[0, -1] = n - 1
+    if width > 2:
+        ids[0, 1] = ids[0, 0]
+    row_len = rng.integers(0, width + 1, n_rows).astype(np.int32)
+    row_len[0] = width
+    ids[np.arange(width)[None, :] >= row_len[:, None]] = -1
+    table, lens = torch.from_numpy(ids).to(hip_device), torch.from_numpy(row_len).to(hip_device)
+    q_lo = 700 if how == "shard" else 0
+    qids = torch.arange(3, 3 + n_rows, dtype=torch.int32, device=hip_device) if how == "ids" else None
+    tab = EdgeTable(table, lens, n, q_lo=q_lo, global_token=token, query_ids=qids)
+    got = tab.to_edge_index()
+    coo = AttentionIndex.from_table(table, lens, False, n_kv=n).to_coo()
+    ref = torch.stack([coo[0], coo[1] + (3 if how == "ids" else q_lo)])
+    if token:
+        ar = torch.arange(1, n + 1, device=hip_device)
+        rows = ar if how == "ids" else torch.arange(q_lo + 1, q_lo + n_rows + 1, device=hip_device)
+        parts = [ref + 1] + ([torch.stack([ar, torch.zeros_like(ar)])] if how != "shard" else [])
+        ref = torch.cat(parts + [torch.stack([torch.zeros_like(rows), rows])], dim=1)
+    assert torch.equal(got, ref)
+    table[-1, 0], lens[-1] = n, 1
+    with pytest.raises(ValueError, match="table ids outside"):
+        EdgeTable(table, lens, n).to_edge_index()
+    lens[-1] = width + 1
+    with pytest.raises(ValueError, match="row lengths outside"):
+        EdgeTable(table, lens, n).to_edge_index()
