@@ -86,6 +86,10 @@ _SIGS = {
     "bf_real_select_rows": (C.c_int, [P_i64, P_i32, i64, P_i32, i64, i32, i64, P_i32, i64, i64, P_i32, P_i32, P_i32,
                                       P_i32, vp]),
     "bf_assemble_rows": (C.c_int, [P_i32, P_i32, i32, i32, P_i32, P_i32, i32, i32, i32, i64, P_i32, i32, P_i32, vp]),
+    "bf_node_set_workspace_size": (C.c_int, [i64, C.POINTER(sz)]),
+    "bf_reception_cone": (C.c_int, [P_i64, P_i32, P_i64, P_i32, i64, i64, P_i64, i64, i32, P_i64, C.POINTER(i64), vp, sz,
+                                    vp]),
+    "bf_probe_queries": (C.c_int, [P_i64, i64, i64, P_i64, P_i32, i64, P_i32, P_i32, C.POINTER(i64), vp, sz, vp]),
     "bf_mark_in_neighbors": (C.c_int, [P_i64, P_i32, i64, vp, vp, vp]),
     "bf_build_edge_table_workspace_size": (C.c_int, [i64, i32, i64, i32, C.POINTER(sz)]),
     "bf_build_edge_table": (C.c_int, [P_i64, P_i32, vp, P_i64, P_i32, i64, i64, i64, i64, i32, i32, i32, i32, i64,

@@ -324,14 +324,17 @@ def _check_qids(qids: torch.Tensor, num_nodes: int, dev) -> None:
 
 def rw_select_rows(rowptr, col, qids: torch.Tensor, walks_per_node: int, walk_length: int, k_rw: int,
                    key_seed: int, u=None, philox_seed: int = 0, philox_offset: int = 0, subtract=None,
-                   walk_rec=None):
+                   walk_rec=None, ids_checked: bool = False):
     """bf_rw_select for an explicit query list; ``subtract=(in_ptr, in_src)`` drops candidates that are
-    already graph edges into the query. Returns (sel_kv [n,k_rw] key order, sel_cnt [n])."""
+    already graph edges into the query. ``ids_checked``: the ids are known to lie in the graph. Returns (sel_kv [n,k_rw] key order, sel_cnt [n])."""
     dev = rowptr.device
     _require(rowptr, "rowptr", torch.int64)
     _require(col, "col", torch.int32, dev)
     n_nodes = rowptr.numel() - 1
-    _check_qids(qids, n_nodes, dev)
+    if ids_checked:
+        _require(qids, "query_ids", torch.int32, dev)
+    else:
+        _check_qids(qids, n_nodes, dev)
     n = qids.numel()
     if u is not None:
         _require(u, "u", torch.float32, dev)
@@ -353,12 +356,16 @@ def rw_select_rows(rowptr, col, qids: torch.Tensor, walks_per_node: int, walk_le
 
 
 def real_select_rows(in_ptr, in_src, qids: torch.Tensor, k_real: int, key_seed: int,
-                     hubs: Optional[torch.Tensor] = None, hub_threshold: int = HUB_THRESHOLD):
-    """Real-edge top-k_real in key order for an explicit query list: (sel_kv [n,k_real], sel_cnt [n])."""
+                     hubs: Optional[torch.Tensor] = None, hub_threshold: int = HUB_THRESHOLD,
+                     ids_checked: bool = False):
+    """Real-edge top-k_real in key order for an explicit query list (``ids_checked`` as in rw_select_rows): (sel_kv [n,k_real], sel_cnt [n])."""
     dev = in_ptr.device
     _require(in_ptr, "in_ptr", torch.int64)
     _require(in_src, "in_src", torch.int32, dev)
-    _check_qids(qids, in_ptr.numel() - 1, dev)
+    if ids_checked:
+        _require(qids, "query_ids", torch.int32, dev)
+    else:
+        _check_qids(qids, in_ptr.numel() - 1, dev)
     n = qids.numel()
     sel = torch.empty(n, k_real, dtype=torch.int32, device=dev)
     cnt = torch.empty(n, dtype=torch.int32, device=dev)
@@ -396,6 +403,46 @@ def assemble_rows(real=None, rw=None, b_real: int = 0, b_rw: int = 0, dedup: boo
            _p(rw[1]) if rw is not None else None, rw[0].shape[1] if rw is not None else 0, b_rw, int(bool(dedup)), n,
            _p(table), width, _p(row_len), _stream(dev))
     return table, row_len
+
+
+def reception_cone(rowptr, col, in_ptr, in_src, probe_ids: torch.Tensor, hops: int) -> torch.Tensor:
+    """Ascending int64 ids of ``probe_ids`` (int64; those below the edges' id bound) and every node reaching one of
+    them over at most ``hops`` edges (bf_reception_cone); one host read."""
+    dev = in_ptr.device
+    _require(in_ptr, "in_ptr", torch.int64)
+    _require(rowptr, "rowptr", torch.int64, dev)
+    _require(in_src, "in_src", torch.int32, dev)
+    _require(col, "col", torch.int32, dev)
+    _require(probe_ids, "probe_ids", torch.int64, dev)
+    n = in_ptr.numel() - 1
+    ids = torch.empty(n, dtype=torch.int64, device=dev)
+    ws = _workspace(_size_query("bf_node_set_workspace_size", n), dev)
+    cnt = C.c_int64(0)
+    N.call("bf_reception_cone", _p(rowptr), _p(col), _p(in_ptr), _p(in_src), n, col.numel(), _p(probe_ids),
+           probe_ids.numel(), int(hops), _p(ids), C.byref(cnt), _p(ws), ws.numel(), _stream(dev))
+    return ids[: cnt.value].clone() if 4 * cnt.value < n else ids[: cnt.value]
+
+
+def probe_queries(dst_filter: torch.Tensor, in_ptr: torch.Tensor, hubs: Optional[torch.Tensor] = None):
+    """A probe's destination filter (int64 [m]) as its query list (bf_probe_queries, one host read): (query_ids int32
+    ascending and distinct, the entries of ``hubs`` among them, whether some query has an in-edge), or None when an
+    id lies outside the graph."""
+    dev = in_ptr.device
+    _require(in_ptr, "in_ptr", torch.int64)
+    _require(dst_filter, "dst_filter", torch.int64, dev)
+    n, m = in_ptr.numel() - 1, dst_filter.numel()
+    n_hubs = 0 if hubs is None else hubs.numel()
+    if n_hubs:
+        _require(hubs, "hubs", torch.int32, dev)
+    ids = torch.empty(max(min(m, n), 1), dtype=torch.int32, device=dev)
+    kept = torch.empty(max(n_hubs, 1), dtype=torch.int32, device=dev)
+    ws = _workspace(_size_query("bf_node_set_workspace_size", n), dev)
+    info = (C.c_int64 * 4)()
+    N.call("bf_probe_queries", _p(dst_filter), m, n, _p(in_ptr), _p(hubs) if n_hubs else None, n_hubs, _p(ids),
+           _p(kept) if n_hubs else None, info, _p(ws), ws.numel(), _stream(dev))
+    if info[3]:
+        return None
+    return ids[: info[0]], kept[: info[2]], bool(info[1])
 
 
 def mark_in_neighbors(in_ptr, in_src, frontier: torch.Tensor, reached: torch.Tensor) -> None:

@@ -32,17 +32,6 @@ from .edges import REAL_SEED_OFFSET, RW_SEED_OFFSET, EdgeTable
 from .graph import CSRGraph
 
 
-def _edge_id_bound(graph: CSRGraph) -> int:
-    """max node id appearing in an edge + 1 (0 without edges): the reference
-    sizes its reception mask by ``edge_index.max() + 1`` (:2284-2286)."""
-    if graph.num_edges == 0:
-        return 0
-    deg = graph.rowptr[1:] - graph.rowptr[:-1]
-    has_out = torch.nonzero(deg > 0).view(-1)
-    top_src = int(has_out[-1]) if has_out.numel() else -1
-    return max(int(graph.col.max()), top_src) + 1
-
-
 def reception_cone(graph: CSRGraph, probe_ids: torch.Tensor, n_layers: int) -> torch.Tensor:
     """``_expand_probe_idx_for_reception`` (:2261-2309) as a device BFS over the in-neighbour CSR.
 
@@ -53,22 +42,8 @@ def reception_cone(graph: CSRGraph, probe_ids: torch.Tensor, n_layers: int) -> t
     """
     if n_layers <= 1 or probe_ids is None or probe_ids.numel() == 0 or graph.num_edges == 0:
         return probe_ids
-    n = graph.num_nodes
-    bound = _edge_id_bound(graph)
-    ids = probe_ids.to(graph.device, torch.int64).view(-1)
-    ids = ids[(ids >= 0) & (ids < bound)]
-    mask = torch.zeros(n, dtype=torch.uint8, device=graph.device)
-    mask[ids] = 1
-    frontier = mask.clone()
-    for _ in range(n_layers - 1):
-        reached = torch.zeros_like(mask)
-        hip_ops.mark_in_neighbors(graph.in_ptr, graph.in_src, frontier, reached)
-        new = reached & (1 - mask)
-        if not bool(new.any()):
-            break
-        mask |= new
-        frontier = new
-    return torch.nonzero(mask).view(-1)
+    ids = probe_ids.to(graph.device, torch.int64).view(-1).contiguous()
+    return hip_ops.reception_cone(graph.rowptr, graph.col, graph.in_ptr, graph.in_src, ids, n_layers - 1)
 
 
 @dataclass
@@ -138,30 +113,33 @@ def build_probe(graph: CSRGraph, dst_filter: torch.Tensor, *, max_real: int, max
     [n*P, L], rows in ascending filter order) injects the walk uniforms.
     """
     dev = graph.device
-    qids = torch.unique(dst_filter.to(dev).view(-1)).to(torch.int32)
+    ids = dst_filter.to(dev).view(-1).to(torch.int64).contiguous()
+    all_hubs = graph.hubs(hub_threshold) if use_real and max_real > 0 else None
+    found = hip_ops.probe_queries(ids, graph.in_ptr, all_hubs)
+    checked = found is not None
+    if checked:
+        qids, hubs, has_edges = found
+    else:                       # an id outside the graph: the ranking calls refuse it
+        qids, hubs, has_edges = torch.unique(ids).to(torch.int32), None, False
     n = qids.numel()
     P = max(int(walks_per_node), 1)
     L = max(int(walk_length), 1)
     seed = int(edge_seed if philox_seed is None else philox_seed)
-    real_nonempty = False
+    real_nonempty = bool(use_real and n and has_edges)
     real = rw = None
-    if use_real and n:
-        deg = graph.in_ptr[qids.long() + 1] - graph.in_ptr[qids.long()]
-        real_nonempty = bool((deg > 0).any())
-        if max_real > 0:
-            hubs = graph.hubs(hub_threshold)
-            hubs = hubs[torch.isin(hubs, qids)] if hubs.numel() else hubs
-            real = hip_ops.real_select_rows(graph.in_ptr, graph.in_src, qids, int(max_real),
-                                            int(edge_seed) + REAL_SEED_OFFSET, hubs=hubs if hubs.numel() else None,
-                                            hub_threshold=hub_threshold)
+    if use_real and n and max_real > 0:
+        real = hip_ops.real_select_rows(graph.in_ptr, graph.in_src, qids, int(max_real),
+                                        int(edge_seed) + REAL_SEED_OFFSET,
+                                        hubs=hubs if hubs is not None and hubs.numel() else None,
+                                        hub_threshold=hub_threshold, ids_checked=checked)
     rw_nonempty = False
     if use_rw and walks_per_node > 0 and n:
         subtract = (graph.in_ptr, graph.in_src) if real_nonempty else None
         k = max(int(max_rw), 1)
         sel, cnt = hip_ops.rw_select_rows(graph.rowptr, graph.col, qids, P, L, k, int(edge_seed) + RW_SEED_OFFSET,
                                           u=u, philox_seed=seed, philox_offset=philox_offset, subtract=subtract,
-                                          walk_rec=graph.walk_records())
-        rw_nonempty = bool((cnt > 0).any())
+                                          walk_rec=graph.walk_records(), ids_checked=checked)
+        rw_nonempty = bool(cnt.any())
         if max_rw > 0:
             rw = (sel, cnt)
     return ProbeBuild(graph, qids, real, rw, real_nonempty, rw_nonempty, global_token=global_token)

@@ -260,6 +260,27 @@ int bf_assemble_rows(const int32_t* real_kv, const int32_t* real_cnt, int32_t re
                      int32_t rw_stride, int32_t b_rw, int32_t dedup, int64_t n_rows,
                      int32_t* table, int32_t width, int32_t* row_len, void* stream);
 
+/* A probe's reception cone (_expand_probe_idx_for_reception,
+ * utils/fullgraph_sp_support.py:2261-2309): the probe ids below the edges'
+ * largest id + 1 and every node that reaches one of them over at most `hops`
+ * edges, ascending in ids int64 (capacity num_nodes), their number in
+ * *count_host (synchronises the stream). rowptr / col: the out-neighbour CSR,
+ * in_ptr / in_src: the in-neighbour CSR.
+ * bf_probe_queries: a destination filter (int64, any order, repeats allowed) as
+ * the probe build takes it: query_ids int32 (capacity min(n_filter, num_nodes))
+ * ascending and distinct, hubs_out the entries of hubs (ascending) among them,
+ * and info_host[4] = {queries, 1 if one has an in-edge, hubs_out's length, 1 if
+ * an id lies outside [0, num_nodes)} (_build_probe_edge_pools, :1743-1821).
+ * Synchronises the stream. Workspace of both: bf_node_set_workspace_size,
+ * 16-byte aligned.                                                          */
+int bf_node_set_workspace_size(int64_t num_nodes, size_t* bytes);
+int bf_reception_cone(const int64_t* rowptr, const int32_t* col, const int64_t* in_ptr, const int32_t* in_src,
+                      int64_t num_nodes, int64_t num_edges, const int64_t* probe_ids, int64_t n_probe, int32_t hops,
+                      int64_t* ids, int64_t* count_host, void* workspace, size_t workspace_bytes, void* stream);
+int bf_probe_queries(const int64_t* filter, int64_t n_filter, int64_t num_nodes, const int64_t* in_ptr,
+                     const int32_t* hubs, int64_t n_hubs, int32_t* query_ids, int32_t* hubs_out, int64_t* info_host,
+                     void* workspace, size_t workspace_bytes, void* stream);
+
 /* One layer of the probe's reception-cone expansion
  * (_expand_probe_idx_for_reception, utils/fullgraph_sp_support.py:2261-2309):
  * reached[s] = 1 for every edge s -> v of the in-neighbour CSR with

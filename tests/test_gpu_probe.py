@@ -118,3 +118,42 @@ def test_probe_wide_budgets_and_long_walks(hip_device):
             assert np.array_equal(got, ref)
         else:
             assert _pairs(got) == _pairs(ref)
+
+
+@pytest.mark.parametrize("n", [15, 4096, 4097, 9001])
+@pytest.mark.parametrize("layers", [2, 4])
+def test_cone_and_query_list_at_the_edges_of_their_tiles(hip_device, n, layers):
+    """Directed edges (nodes past the last edge id dropped, a hub row longer than a workgroup's share), probe ids out
+    of range, repeated and in any order; the query list, its hubs and its flags against numpy."""
+    from budgetformer_amd import hip_ops
+    from budgetformer_amd.graph import CSRGraph
+    from budgetformer_amd.probe import reception_cone
+    rng = np.random.default_rng(n + layers)
+    top = n - 3                                             # no edge at the last nodes
+    ei = np.stack([rng.integers(0, top, 2 * n), rng.integers(0, top, 2 * n)])
+    ei = np.concatenate([ei, np.stack([np.arange(top), np.full(top, top // 2)])], axis=1)    # a hub
+    ei = et.coalesce(ei, n)
+    g = CSRGraph.from_edge_index(torch.from_numpy(ei).to(hip_device), n)
+    probe = torch.tensor([3, n - 1, top // 2, 3, -1, n + 5, n - 4], dtype=torch.int64)
+    got = reception_cone(g, probe.to(hip_device), layers)
+    assert np.array_equal(got.cpu().numpy(), np.asarray(et.reception_cone(ei, probe.numpy(), layers)))
+    ids = torch.from_numpy(rng.integers(0, n, n // 2 + 1))
+    deg = np.bincount(ei[1], minlength=n)
+    hubs = np.flatnonzero(deg > 2).astype(np.int32)
+    q, h, has = hip_ops.probe_queries(ids.to(hip_device), g.in_ptr, torch.from_numpy(hubs).to(hip_device))
+    uniq = np.unique(ids.numpy())
+    assert np.array_equal(q.cpu().numpy(), uniq) and np.array_equal(h.cpu().numpy(), np.intersect1d(hubs, uniq))
+    assert has == bool((deg[uniq] > 0).any())
+    assert hip_ops.probe_queries(torch.tensor([n - 1], device=hip_device), g.in_ptr)[2] is False
+    assert hip_ops.probe_queries(torch.tensor([0, n], device=hip_device), g.in_ptr) is None
+
+
+def test_probe_refuses_ids_outside_the_graph_and_takes_an_empty_filter(hip_device):
+    from budgetformer_amd.probe import build_probe
+    g, _ = _setup(500, 3000, 2, hip_device)
+    for bad in ([0, 500], [-1, 4]):
+        with pytest.raises(ValueError, match="query_ids"):
+            build_probe(g, torch.tensor(bad, device=hip_device), max_real=4, max_rw=4)
+    pb = build_probe(g, torch.zeros(0, dtype=torch.int64, device=hip_device), max_real=4, max_rw=4)
+    assert pb.query_ids.numel() == 0 and not pb.real_nonempty and not pb.rw_nonempty
+    assert pb.table(4, 4).to_edge_index().shape == (2, 0)
