@@ -575,6 +575,92 @@ __global__ void split_count_kernel(const int64_t* __restrict__ ptr, int64_t n_ro
   if (r < n_rows) packed[r] = split_count(ptr[r + 1] - ptr[r], threshold, item_size);
 }
 
+// The plan of up to kPtrInBlockMax blocks of kPtrRows rows in two launches, as
+// the table's row pointers: each block's sum of its rows' packed counts, then
+// each block adds up the sums before it, scans its own rows and writes. A scan
+// over every row's count (a packed array written, scanned and read back) took
+// 58 us at 2.9M rows, this 31. Rows to split are few: a wave scans only a
+// round of 64 rows that holds one, and writes a split row's items together.
+__device__ __forceinline__ uint64_t block_sum_u64(uint64_t v, uint64_t* tmp /*[kThreads / 64]*/) {
+  return uint64_t(block_sum_i64(int64_t(v), reinterpret_cast<int64_t*>(tmp)));
+}
+
+__global__ __launch_bounds__(kThreads) void plan_sums_kernel(const int64_t* __restrict__ ptr, int64_t n_rows,
+                                                             int threshold, int item_size,
+                                                             uint64_t* __restrict__ bsum) {
+  __shared__ uint64_t tmp[kThreads / 64];
+  const int64_t t0 = int64_t(blockIdx.x) * kPtrRows + threadIdx.x;
+  uint64_t s = 0;
+#pragma unroll
+  for (int u = 0; u < kPtrRowsPerThread; ++u) {
+    const int64_t r = t0 + u * kThreads;
+    if (r < n_rows) s += split_count(ptr[r + 1] - ptr[r], threshold, item_size);
+  }
+  s = block_sum_u64(s, tmp);
+  if (threadIdx.x == 0) bsum[blockIdx.x] = s;
+}
+
+__global__ __launch_bounds__(kThreads) void plan_write_kernel(
+    const int64_t* __restrict__ ptr, int64_t n_rows, int threshold, int item_size, const uint64_t* __restrict__ bsum,
+    int64_t item_cap, int32_t* __restrict__ nitems, int32_t* __restrict__ item_off, int32_t* __restrict__ item_row,
+    int32_t* __restrict__ heavy_rows, int64_t heavy_cap, int32_t* __restrict__ counts) {
+  __shared__ uint64_t tmp[kThreads / 64], wtot[kThreads / 64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  uint64_t before = 0;
+  for (int64_t k = threadIdx.x; k < int64_t(blockIdx.x); k += kThreads) before += bsum[k];
+  before = block_sum_u64(before, tmp);
+  const int64_t t0 = int64_t(blockIdx.x) * kPtrRows + int64_t(w) * (64 * kPtrRowsPerThread) + lane;
+  uint64_t v[kPtrRowsPerThread], mine = 0;
+#pragma unroll
+  for (int u = 0; u < kPtrRowsPerThread; ++u) {
+    const int64_t r = t0 + u * 64;
+    v[u] = r < n_rows ? split_count(ptr[r + 1] - ptr[r], threshold, item_size) : 0;
+    mine += v[u];
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) mine += __shfl_xor(mine, o, 64);
+  if (lane == 0) wtot[w] = mine;
+  __syncthreads();
+  uint64_t base = before;
+#pragma unroll
+  for (int i = 0; i < kThreads / 64; ++i)
+    if (i < w) base += wtot[i];
+#pragma unroll
+  for (int u = 0; u < kPtrRowsPerThread; ++u) {
+    const int64_t r = t0 + u * 64;
+    uint64_t x = v[u];
+    uint64_t split = __ballot(x != 0);
+    if (split) {                                     // uniform over the wave
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint64_t y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
+      }
+    }
+    const uint64_t off = base + x - v[u];            // items and split rows before row r
+    if (split) base += __shfl(x, 63, 64);
+    const int32_t n = int32_t(v[u] >> 32);
+    const int64_t slot = int64_t(uint32_t(off));
+    if (r < n_rows) {
+      nitems[r] = n;
+      item_off[r] = int32_t(off >> 32);
+      if (n > 0 && slot < heavy_cap) heavy_rows[slot] = int32_t(r);
+      if (r == n_rows - 1) {
+        const int64_t items = int64_t(off >> 32) + n, heavy = slot + (n > 0 ? 1 : 0);
+        counts[0] = int32_t(items < item_cap ? items : item_cap);
+        counts[1] = int32_t(heavy < heavy_cap ? heavy : heavy_cap);
+      }
+    }
+    while (split) {                                  // each split row's items by the whole wave
+      const int src = __ffsll((unsigned long long)split) - 1;
+      split &= split - 1;
+      const int32_t row = int32_t(t0 - lane) + u * 64 + src, cnt = __shfl(n, src, 64);
+      const int64_t first = int64_t(__shfl(off, src, 64) >> 32);
+      for (int64_t j = lane; j < cnt && first + j < item_cap; j += 64) item_row[first + j] = row;
+    }
+  }
+}
+
 // nitems, item_off, the heavy-row list (compacted by the scanned flags),
 // item_row of each item and the two plan counts, one thread per slot: slot j
 // is row j, or with an order row order[j], and then only the split rows'
@@ -958,16 +1044,23 @@ extern "C" int bf_split_plan(const int64_t* ptr, int64_t n_rows, int32_t thresho
   void* temp = static_cast<char*>(workspace) + 2 * slab;
   size_t temp_bytes = 0;
   (void)prim::exclusive_sum(nullptr, temp_bytes, static_cast<const uint64_t*>(packed), packed_off, n_rows, st);
+  const int64_t ptr_blocks = ceil_div(n_rows, kPtrRows);
+  if (ptr_blocks <= kPtrInBlockMax) {               // packed: one sum per block
+    BF_LAUNCH("plan_sums_kernel", plan_sums_kernel, dim3(unsigned(ptr_blocks)), dim3(kThreads), 0, st, ptr, n_rows,
+              threshold, item_size, packed);
+    BF_CHECK_LAUNCH();
+    BF_LAUNCH("plan_write_kernel", plan_write_kernel, dim3(unsigned(ptr_blocks)), dim3(kThreads), 0, st, ptr, n_rows,
+              threshold, item_size, packed, item_cap, nitems, item_off, item_row, heavy_rows, heavy_cap, counts);
+    BF_CHECK_LAUNCH();
+    return BF_OK;
+  }
   BF_LAUNCH("split_count_kernel", split_count_kernel, dim3(blocks_for(n_rows)), dim3(kThreads), 0, st, ptr, n_rows,
             threshold, item_size, packed);
   BF_CHECK_LAUNCH();
-  const bool in_block = n_rows <= kPlanInBlockSlots;
-  if (!in_block)
-    BF_CHECK_HIP(prim::exclusive_sum(temp, temp_bytes, static_cast<const uint64_t*>(packed), packed_off, n_rows,
-                                     st));
+  BF_CHECK_HIP(prim::exclusive_sum(temp, temp_bytes, static_cast<const uint64_t*>(packed), packed_off, n_rows, st));
   BF_LAUNCH("split_rows_kernel", split_rows_kernel, dim3(blocks_for(n_rows)), dim3(kThreads), 0, st, packed,
-            in_block ? nullptr : packed_off, static_cast<const int32_t*>(nullptr), n_rows, item_cap, nitems,
-            item_off, item_row, heavy_rows, heavy_cap, counts);
+            packed_off, static_cast<const int32_t*>(nullptr), n_rows, item_cap, nitems, item_off, item_row, heavy_rows,
+            heavy_cap, counts);
   BF_CHECK_LAUNCH();
   return BF_OK;
 }

@@ -133,3 +133,23 @@ def test_table_to_list_equals_the_index_route(hip_device, n_rows, width, how, to
     lens[-1] = width + 1
     with pytest.raises(ValueError, match="row lengths outside"):
         EdgeTable(table, lens, n).to_edge_index()
+
+
+@pytest.mark.parametrize("n_rows", [1, 63, 4095, 4096, 4097, 70_000])
+@pytest.mark.parametrize("threshold,item,share", [(8, 3, 0.01), (1, 1, 1.0), (1000, 768, 0.0)])
+def test_split_plan_at_block_edges(hip_device, n_rows, threshold, item, share):
+    """Few rows to split, every row, none; one row of more items than a wave has lanes, at the end of a block."""
+    from budgetformer_amd import hip_ops
+    rng = np.random.default_rng(n_rows + threshold)
+    lens = rng.integers(0, threshold + 1, n_rows)
+    lens[rng.random(n_rows) < share] += threshold + 5
+    lens[min(n_rows - 1, 4095)] += 150 * item if share else 0
+    ptr = np.concatenate([[0], np.cumsum(lens)])
+    plan = hip_ops.split_plan(torch.from_numpy(ptr).to(hip_device), int(ptr[-1]), threshold, item)
+    n = np.array([hip_ops.split_row_items(int(x), item) if x > threshold else 0 for x in lens])
+    off = np.concatenate([[0], np.cumsum(n)])[:-1]
+    assert (plan.items, plan.heavy) == (n.sum(), (n > 0).sum())
+    assert np.array_equal(plan.nitems.cpu().numpy()[:n_rows], n)
+    assert np.array_equal(plan.item_off.cpu().numpy()[:n_rows], off)
+    assert np.array_equal(plan.item_row.cpu().numpy()[:plan.items], np.repeat(np.arange(n_rows), n))
+    assert np.array_equal(plan.heavy_rows.cpu().numpy()[:plan.heavy], np.flatnonzero(n))
