@@ -533,6 +533,43 @@ __device__ __forceinline__ int64_t row_slot(const Shape& sh, unsigned first_bloc
   return int64_t(blockIdx.x - first_block) * (kBlock >> sh.lpr_log2) + (threadIdx.x >> sh.lpr_log2);
 }
 
+// A short query row and its entries, as its lane group takes them.
+struct RowPick {
+  int64_t row, beg, end;   // row >= n_q: none
+};
+
+// The query row of this lane's group. deal (deal_rows): the workgroup's rows (kBlock / lanes per row consecutive
+// ones) go to its groups longest first, so that the groups of a wave walk rows of about one length. A wave runs
+// until its longest row ends; with rows in id order the lanes of the shorter ones idled (2.9M rows of 128 bf16 with
+// dropout, 0 to 32 entries, 11 on average, four rows to a wave: forward 2.72 -> 2.29 ms, dq pass 2.40 -> 2.13).
+// Each wave ranks the rows by itself, from one load of their row pointers. Split rows (longer than `chunk`) rank
+// last: their groups leave at once.
+__device__ __forceinline__ RowPick pick_row(const Shape& sh, unsigned first_block, const int64_t* __restrict__ qptr,
+                                            int64_t n_q, int chunk, int deal) {
+  const int gpb = kBlock >> sh.lpr_log2;
+  const int64_t r0 = int64_t(blockIdx.x - first_block) * gpb;
+  const int grp = threadIdx.x >> sh.lpr_log2;
+  if (!deal) {
+    const int64_t row = r0 + grp;
+    return row < n_q ? RowPick{row, qptr[row], qptr[row + 1]} : RowPick{row, 0, 0};
+  }
+  const int lane = threadIdx.x & 63;
+  const bool mine = lane < gpb && r0 + lane < n_q;
+  const int64_t b = mine ? qptr[r0 + lane] : 0;
+  const int len = mine ? int(qptr[r0 + lane + 1] - b) : 0;
+  const int key = len > chunk ? 0 : len;
+  int rank = 0;
+  for (int i = 0; i < gpb; ++i) {
+    const int k = __builtin_amdgcn_readlane(key, i);
+    rank += (k > key || (k == key && i < lane)) ? 1 : 0;
+  }
+  // rank -> row of the workgroup: lane `rank` receives `lane` (lanes past the rows keep to themselves)
+  const int perm = __builtin_amdgcn_ds_permute((lane < gpb ? rank : lane) << 2, lane);
+  const int src = __shfl(perm, grp, 64);
+  const int64_t beg = __shfl(b, src, 64);
+  return RowPick{r0 + src, beg, beg + __shfl(len, src, 64)};
+}
+
 // Sums `nv` lane vectors of V floats (and, if with_z, one float per head) over
 // the groups of the workgroup, in group order. Every thread must call it; the
 // result is valid in group 0.
@@ -672,7 +709,7 @@ template <typename T, int EX>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(FwdWaves<T, EX>::kMin))) void attn_fwd_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
     const int64_t* __restrict__ qptr, const int32_t* __restrict__ kv, EdgeIn ex,
-    T* __restrict__ out, float* __restrict__ Z, Items it, int n_items_arg, int64_t n_q, Shape sh, int chunk,
+    T* __restrict__ out, float* __restrict__ Z, Items it, int n_items_arg, int64_t n_q, Shape sh, int chunk, int deal,
     const int32_t* __restrict__ plan_counts) {
   constexpr int V = Elem<T>::kPerVec;
   const GroupPos g = group_pos<T>(sh);
@@ -699,9 +736,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(FwdWaves
     }
     return;
   }
-  const int64_t row = row_slot(sh, unsigned(n_items_arg));
+  const RowPick pick = pick_row(sh, unsigned(n_items_arg), qptr, n_q, chunk, deal);
+  const int64_t row = pick.row, beg = pick.beg, end = pick.end;
   if (row >= n_q) return;
-  const int64_t beg = qptr[row], end = qptr[row + 1];
   if (end - beg > chunk) return;  // split row: its items and the reduce write it
   const typename Elem<T>::Raw qr = load_row_raw_nt(q, row, sh.D, g);
   fwd_segment<T, EX>(k, v, kv, ex, beg, end, int32_t(row), beg, sh, g, qr, acc, z);
@@ -966,7 +1003,7 @@ __global__ __launch_bounds__(kBlock) void attn_bwd_q_kernel(
     const int64_t* __restrict__ qptr, const int32_t* __restrict__ kv, EdgeIn ex,
     const float* __restrict__ Z, const T* __restrict__ dout,
     T* __restrict__ dq, float* __restrict__ dbias, float2* __restrict__ rstat, Items it, int n_items_arg,
-    int64_t n_q, Shape sh, int chunk, float* __restrict__ token_rec, int tok_first,
+    int64_t n_q, Shape sh, int chunk, int deal, float* __restrict__ token_rec, int tok_first,
     const int32_t* __restrict__ plan_counts) {
   constexpr int V = Elem<T>::kPerVec;
   extern __shared__ float lds[];
@@ -1006,14 +1043,10 @@ __global__ __launch_bounds__(kBlock) void attn_bwd_q_kernel(
     if (token_rec && grp == 0) store_token_record<V>(token_rec + int64_t(blockIdx.x) * (2 * sh.D), sh, g, fk, fv);
     return;
   }
-  const int64_t row = row_slot(sh, unsigned(n_items_arg));
-  int64_t beg = 0, end = 0;
-  bool live = row < n_q;
-  if (live) {
-    beg = qptr[row];
-    end = qptr[row + 1];
-    live = end - beg <= chunk;    // a split row: its items and the reduce write it
-  }
+  const RowPick pick = pick_row(sh, unsigned(n_items_arg), qptr, n_q, chunk, deal);
+  const int64_t row = pick.row, end = pick.end;
+  int64_t beg = pick.beg;
+  const bool live = row < n_q && end - beg <= chunk;    // a split row: its items and the reduce write it
   if (!token_rec && !live) return;
   typename Elem<T>::Raw qr = Elem<T>::zero_raw(), gr = Elem<T>::zero_raw();
   float inv_dprime = 1.f;
@@ -1827,6 +1860,15 @@ inline unsigned grid_for(int64_t rows, const Shape& sh) {
   return unsigned(ceil_div(rows, per_block));
 }
 
+// Whether the query passes deal a workgroup's rows out by length (pick_row): where a wave holds four rows or more
+// (with two the ranking costs what it spares: 169K nodes, float32 rows of 128, step 659 -> 663 us), ranks them all
+// (at most 64 to a workgroup) and they are long enough to differ by iterations: more than 10 entries a row by the
+// index's entry count, which is its capacity for a small table (rows of a budget of 8 and the token's entries end
+// within three iterations: 411K rows of 64 fp16, forward 97.5 -> 98.0 us with the ranking).
+inline int deal_rows(const bf_attn_index* idx, const Shape& sh) {
+  return sh.lpr_log2 <= 4 && (kBlock >> sh.lpr_log2) <= 64 && idx->nnz > 10 * idx->n_q ? 1 : 0;
+}
+
 inline size_t combine_lds_bytes(const Shape& sh) {
   return size_t(kBlock >> sh.lpr_log2) * size_t(2 * sh.D + sh.H) * sizeof(float);
 }
@@ -1888,7 +1930,8 @@ int fwd_impl(const bf_attn_index* idx, const Shape& sh, const void* q, const voi
     const size_t lds = n_items > 0 ? combine_lds_bytes(sh) : 0;
 #define BF_LAUNCH_FWD(EX)                                                                                        \
   BF_LAUNCH("attn_fwd_kernel", (attn_fwd_kernel<T, EX>), dim3(unsigned(blocks)), dim3(kBlock), lds, st, Q, K, Vv,  \
-            idx->qptr, idx->kv, ex, O, Z, it, n_items, idx->n_q, sh, idx->chunk, idx->plan_counts)
+            idx->qptr, idx->kv, ex, O, Z, it, n_items, idx->n_q, sh, idx->chunk, deal_rows(idx, sh),                           \
+            idx->plan_counts)
     // the dropout-only instance stores the keep mask a window at a time, for one byte per entry (H <= 8)
     // and groups wide enough to share an iteration's draws; other shapes (more heads; H <= 3 with one lane
     // per head) take the general instance, which stores it too
@@ -2001,7 +2044,7 @@ int bwd_impl(const bf_attn_index* idx, const Shape& sh, const void* q, const voi
 #define BF_LAUNCH_Q(EX)                                                                                          \
   BF_LAUNCH("attn_bwd_q_kernel", (attn_bwd_q_kernel<T, EX>), dim3(unsigned(q_blocks)), dim3(kBlock), lds, st, Q, K, \
             Vv, idx->qptr, idx->kv, ex, Z, dO, static_cast<T*>(dq), dbias, rstat, qit, idx->q_items,                \
-            idx->n_q, sh, idx->chunk, token_rec, tok_first, idx->plan_counts)
+            idx->n_q, sh, idx->chunk, deal_rows(idx, sh), token_rec, tok_first, idx->plan_counts)
     // the mask is read back where an entry's bits fill one byte (H <= 8); wider rows of heads draw
     switch (edge_mode(ex, dbias != nullptr)) {
       case 4:

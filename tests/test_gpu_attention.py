@@ -508,3 +508,35 @@ def test_query_passes_past_16m_rows_equal_the_compact_problem(hip_device):
     for t in (out_b, z_b, dq_b):
         t[touched] = 0
         assert not t.any()
+
+
+@pytest.mark.parametrize("dtype,H,hn", [(torch.bfloat16, 8, 16), (torch.float16, 8, 8), (torch.bfloat16, 8, 32),
+                                        (torch.float32, 4, 8), (torch.float32, 8, 16)])
+@pytest.mark.parametrize("n", [1, 33, 1000])
+def test_rows_dealt_by_length(hip_device, dtype, H, hn, n):
+    """Rows of 0 to 40 entries, more than 10 on average, so that a workgroup's rows go to its groups by length (all
+    shapes but float32 rows of 128, which keep id order): a partial last workgroup, empty rows, split rows among the
+    short ones (chunk 36), against the float64 oracle."""
+    g = torch.Generator().manual_seed(n + H * hn)
+    lens = torch.randint(0, 41, (n,), generator=g)
+    lens[n // 2] = 40
+    rows = torch.repeat_interleave(torch.arange(n), lens)
+    kv = torch.randint(0, 500, (rows.numel(),), generator=g)
+    q, dout = (torch.randn(n, H, hn, generator=g).to(dtype) for _ in range(2))
+    k, v = (torch.randn(500, H, hn, generator=g).to(dtype) for _ in range(2))
+    ei = torch.stack([kv, rows])
+    from budgetformer_amd.attention import sparse_edge_attention
+    from budgetformer_amd.hip_ops import AttentionIndex
+    from parity_helpers import assert_close
+    idx = AttentionIndex.from_coo(ei.to(hip_device), n, 500, chunk=36)
+    qd, kd, vd = (t.to(hip_device).requires_grad_(True) for t in (q, k, v))
+    out = sparse_edge_attention(qd, kd, vd, idx)
+    out.backward(dout.to(hip_device))
+    M = max(n, 500)
+    pad = [torch.cat([t.double(), torch.zeros(M - t.size(0), H, hn, dtype=torch.float64)]) for t in (k, q, v, dout)]
+    ro, rZ = sa.attention_forward_stats(pad[0], pad[1], pad[2], ei)
+    rdq, rdk, rdv, _ = sa.attention_backward_closed_form(pad[0], pad[1], pad[2], ei, ro, rZ, pad[3])
+    tol = {torch.float32: 1e-5, torch.bfloat16: 2e-2, torch.float16: 5e-3}[dtype]
+    for name, got, ref in (("out", out, ro[:n]), ("dq", qd.grad, rdq[:n]), ("dk", kd.grad, rdk[:500]),
+                           ("dv", vd.grad, rdv[:500])):
+        assert_close(name, got.detach(), ref, tol)
