@@ -53,10 +53,13 @@ class _SparseEdgeAttention(torch.autograd.Function):
         ctx.score_clamp = score_clamp
         ctx.need_dbias = bias_e is not None and ctx.needs_input_grad[3]
         ctx.mark_non_differentiable(Z)
+        ctx.set_materialize_grads(False)     # no zero gradient is filled for Z
         return out, Z
 
     @staticmethod
     def backward(ctx, dout, _dZ):
+        if dout is None:
+            return (None,) * 8
         q, k, v, Z, bias_e, factor_e = ctx.saved_tensors
         dq, dk, dv, dbias = hip_ops.attn_backward(ctx.index, q, k, v, None, Z, dout.contiguous(), bias_e, factor_e,
                                                   need_dbias=ctx.need_dbias, dropout=ctx.dropout,

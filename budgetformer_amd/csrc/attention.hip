@@ -750,13 +750,15 @@ __global__ __launch_bounds__(kBlock) void attn_fwd_reduce_kernel(T* __restrict__
                                                                  Items it, Shape sh,
                                                                  const int32_t* __restrict__ plan_counts) {
   constexpr int V = Elem<T>::kPerVec;
-  if (plan_counts && int(blockIdx.x) >= plan_counts[1]) return;
   extern __shared__ float lds[];
   const GroupPos g = group_pos<T>(sh);
-  float acc[V], unused[V], z;
-  const int row = reduce_row_records<V, 80 / V>(it, blockIdx.x, lds, sh, g, acc, unused, false, z, true);
-  if (row < 0 || (threadIdx.x >> sh.lpr_log2) != 0) return;
-  store_out(out, Z, row, sh, g, acc, z);
+  const int n_heavy = plan_counts ? plan_counts[1] : int(gridDim.x);
+  for (int h = blockIdx.x; h < n_heavy; h += gridDim.x) {
+    if (h != int(blockIdx.x)) __syncthreads();
+    float acc[V], unused[V], z;
+    const int row = reduce_row_records<V, 80 / V>(it, h, lds, sh, g, acc, unused, false, z, true);
+    if (row >= 0 && (threadIdx.x >> sh.lpr_log2) == 0) store_out(out, Z, row, sh, g, acc, z);
+  }
 }
 
 // ------------------------------------------------------------------ backward, query-major (dq)
@@ -1111,26 +1113,29 @@ __global__ __launch_bounds__(kBlock) void attn_bwd_q_reduce_kernel(
     float* __restrict__ dbias, float2* __restrict__ rstat, Items it, Shape sh, float* __restrict__ token_rec,
     int tok_first, const int32_t* __restrict__ plan_counts) {
   constexpr int V = Elem<T>::kPerVec;
-  if (plan_counts && int(blockIdx.x) >= plan_counts[1]) return;
   extern __shared__ float lds[];
   const GroupPos g = group_pos<T>(sh);
-  float A[V], B[V], c;
-  const int row = reduce_row_records<V, 40 / V>(it, blockIdx.x, lds, sh, g, A, B, true, c, true);
-  if (row < 0 || (threadIdx.x >> sh.lpr_log2) != 0) return;
-  const float inv_dprime = row_inv_dprime<T>(Z, row, sh, g);
-  const int64_t e_tok = it.ptr[row];
-  const bool tok = token_rec != nullptr && row >= tok_first && e_tok < it.ptr[row + 1];
-  float fk[V], fv[V];
+  const int n_heavy = plan_counts ? plan_counts[1] : int(gridDim.x);
+  for (int h = blockIdx.x; h < n_heavy; h += gridDim.x) {
+    if (h != int(blockIdx.x)) __syncthreads();
+    float A[V], B[V], c;
+    const int row = reduce_row_records<V, 40 / V>(it, h, lds, sh, g, A, B, true, c, true);
+    if (row < 0 || (threadIdx.x >> sh.lpr_log2) != 0) continue;
+    const float inv_dprime = row_inv_dprime<T>(Z, row, sh, g);
+    const int64_t e_tok = it.ptr[row];
+    const bool tok = token_rec != nullptr && row >= tok_first && e_tok < it.ptr[row + 1];
+    float fk[V], fv[V];
 #pragma unroll
-  for (int i = 0; i < V; ++i) fk[i] = fv[i] = 0.f;
-  const float dd = c * inv_dprime;
-  store_dq<T, V>(dq, rstat, row, sh, g, A, B, inv_dprime, dd, false);
-  if (tok) {   // key 0 was summed by item 0; its scalars are recomputed here to finish its terms
-    const typename Elem<T>::Raw qr = load_row_raw(q, row, sh.D, g);
-    const typename Elem<T>::Raw gr = load_row_raw(dout, row, sh.D, g);
-    const TokenEntry te = token_entry<T, 2, false>(k, v, ex, e_tok, row, sh, g, inv_dprime, qr, gr, A, B, c);
-    finish_token<T, 2>(te, inv_dprime, dd, qr, gr, dbias, e_tok, sh, g, fk, fv);
-    store_token_record<V>(token_rec + int64_t(it.item_off[row]) * (2 * sh.D), sh, g, fk, fv);
+    for (int i = 0; i < V; ++i) fk[i] = fv[i] = 0.f;
+    const float dd = c * inv_dprime;
+    store_dq<T, V>(dq, rstat, row, sh, g, A, B, inv_dprime, dd, false);
+    if (tok) {   // key 0 was summed by item 0; its scalars are recomputed here to finish its terms
+      const typename Elem<T>::Raw qr = load_row_raw(q, row, sh.D, g);
+      const typename Elem<T>::Raw gr = load_row_raw(dout, row, sh.D, g);
+      const TokenEntry te = token_entry<T, 2, false>(k, v, ex, e_tok, row, sh, g, inv_dprime, qr, gr, A, B, c);
+      finish_token<T, 2>(te, inv_dprime, dd, qr, gr, dbias, e_tok, sh, g, fk, fv);
+      store_token_record<V>(token_rec + int64_t(it.item_off[row]) * (2 * sh.D), sh, g, fk, fv);
+    }
   }
 }
 
@@ -1549,14 +1554,17 @@ __global__ __launch_bounds__(kBlock) void attn_bwd_kv_reduce_kernel(T* __restric
                                                                     Items it, Shape sh,
                                                                     const int32_t* __restrict__ plan_counts) {
   constexpr int V = Elem<T>::kPerVec;
-  if (plan_counts && int(blockIdx.x) >= plan_counts[3]) return;
   extern __shared__ float lds[];
   const GroupPos g = group_pos<T>(sh);
-  float ak[V], av[V], z;
-  const int row = reduce_row_records<V, 40 / V>(it, blockIdx.x, lds, sh, g, ak, av, true, z, false);
-  if (row < 0 || (threadIdx.x >> sh.lpr_log2) != 0 || !g.act) return;
-  Elem<T>::store(dk + int64_t(row) * sh.D + g.col0, ak);
-  Elem<T>::store(dv + int64_t(row) * sh.D + g.col0, av);
+  const int n_heavy = plan_counts ? plan_counts[3] : int(gridDim.x);
+  for (int h = blockIdx.x; h < n_heavy; h += gridDim.x) {
+    if (h != int(blockIdx.x)) __syncthreads();
+    float ak[V], av[V], z;
+    const int row = reduce_row_records<V, 40 / V>(it, h, lds, sh, g, ak, av, true, z, false);
+    if (row < 0 || (threadIdx.x >> sh.lpr_log2) != 0 || !g.act) continue;
+    Elem<T>::store(dk + int64_t(row) * sh.D + g.col0, ak);
+    Elem<T>::store(dv + int64_t(row) * sh.D + g.col0, av);
+  }
 }
 
 // ------------------------------------------------------------------ typed-edge query passes
@@ -1878,6 +1886,15 @@ inline Items query_items(const bf_attn_index* idx, const Shape& sh, float* parti
                idx->item, 2 * sh.D + sh.H};
 }
 
+// Workgroups of a reduce launch: the split rows where the host has their count, else (the counts on the device) the
+// capacity, at most kMaxReduceBlocks: a workgroup then takes every kMaxReduceBlocks-th row until the count ends. The
+// pass kernels' items stay one per workgroup, up to the capacity (a slot past the count exits at once): a loop over
+// items took their instances 10 to 30 registers, a wave or two per SIMD.
+constexpr int kMaxReduceBlocks = 1024;
+inline unsigned reduce_blocks(const bf_attn_index* idx, int n_heavy) {
+  return unsigned(idx->plan_counts && n_heavy > kMaxReduceBlocks ? kMaxReduceBlocks : n_heavy);
+}
+
 // Key-side records follow the query-side ones, so the dk/dv launch can reduce
 // the dq split rows while its items write their own records.
 inline Items key_items(const bf_attn_index* idx, const Shape& sh, float* partials) {
@@ -1952,7 +1969,7 @@ int fwd_impl(const bf_attn_index* idx, const Shape& sh, const void* q, const voi
     BF_CHECK_LAUNCH();
   }
   if (idx->q_heavy > 0) {
-    BF_LAUNCH("attn_fwd_reduce_kernel", attn_fwd_reduce_kernel<T>, dim3(unsigned(idx->q_heavy)), dim3(kBlock),
+    BF_LAUNCH("attn_fwd_reduce_kernel", attn_fwd_reduce_kernel<T>, dim3(reduce_blocks(idx, idx->q_heavy)), dim3(kBlock),
               combine_lds_bytes(sh), st, O, Z, it, sh, idx->plan_counts);
     BF_CHECK_LAUNCH();
   }
@@ -2015,7 +2032,7 @@ int kv_pass_impl(const bf_attn_index* idx, const Shape& sh, const T* Q, const T*
     BF_CHECK_LAUNCH();
   }
   if (idx->k_heavy > 0) {
-    BF_LAUNCH("attn_bwd_kv_reduce_kernel", attn_bwd_kv_reduce_kernel<T>, dim3(unsigned(idx->k_heavy)), dim3(kBlock),
+    BF_LAUNCH("attn_bwd_kv_reduce_kernel", attn_bwd_kv_reduce_kernel<T>, dim3(reduce_blocks(idx, idx->k_heavy)), dim3(kBlock),
               combine_lds_bytes(sh), st, static_cast<T*>(dk), static_cast<T*>(dv), kit, sh, idx->plan_counts);
     BF_CHECK_LAUNCH();
   }
@@ -2063,7 +2080,7 @@ int bwd_impl(const bf_attn_index* idx, const Shape& sh, const void* q, const voi
   }
   // the query-side split rows finish (dq, row stats) before the key-major pass gathers their stats
   if (idx->q_heavy > 0) {
-    BF_LAUNCH("attn_bwd_q_reduce_kernel", attn_bwd_q_reduce_kernel<T>, dim3(unsigned(idx->q_heavy)), dim3(kBlock),
+    BF_LAUNCH("attn_bwd_q_reduce_kernel", attn_bwd_q_reduce_kernel<T>, dim3(reduce_blocks(idx, idx->q_heavy)), dim3(kBlock),
               combine_lds_bytes(sh), st, Q, K, Vv, ex, Z, dO, static_cast<T*>(dq), dbias, rstat, qit, sh,
               token_rec, tok_first, idx->plan_counts);
     BF_CHECK_LAUNCH();

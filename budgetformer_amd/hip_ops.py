@@ -804,10 +804,11 @@ def row_order_and_plan(ptr: torch.Tensor, nnz: int, threshold: int, item_size: i
 class SplitPlan:
     """Rows longer than `threshold` cut into `item_size`-entry items.
 
-    ``items`` / ``heavy`` are host ints once resolved (-1 while ``counts``, the
-    device copy, is still pending: several plans resolve with one read)."""
-    items: int
-    heavy: int
+    ``items`` / ``heavy`` are host ints: known from the start, or read from the
+    pinned copy of ``counts`` (waiting for it), or -1 while the counts are only
+    on the device (several such plans resolve with one read)."""
+    _items: int
+    _heavy: int
     nitems: torch.Tensor
     item_off: torch.Tensor
     item_row: torch.Tensor
@@ -819,9 +820,30 @@ class SplitPlan:
     ready: Optional[object] = None               # (a torch.cuda.Event recorded after the copy)
     _slot: Optional[object] = field(default=None, repr=False)   # returns the pinned slot to its pool
 
+    def _read(self) -> None:
+        self.ready.synchronize()
+        self._items, self._heavy = (int(x) for x in self.host_counts.tolist())
+        self.counts = self.host_counts = self.ready = None
+        self._slot()               # the slot goes back to the pool (the finalizer runs once)
+
+    @property
+    def items(self) -> int:
+        if self._items < 0 and self.ready is not None:
+            self._read()
+        return self._items
+
+    @property
+    def heavy(self) -> int:
+        if self._items < 0 and self.ready is not None:
+            self._read()
+        return self._heavy
+
     @property
     def pending(self) -> bool:
-        return self.items < 0
+        """Whether the host does not have the counts (yet): a pinned copy that has landed is read, without waiting."""
+        if self._items < 0 and self.ready is not None and self.ready.query():
+            self._read()
+        return self._items < 0
 
 
 class _PinnedCountSlots:
@@ -875,13 +897,7 @@ def _copy_counts_to_host(plan: "SplitPlan", dev) -> None:
 def resolve_plans(*plans) -> None:
     """Read the counts of every pending plan: from its pinned copy once that has landed, else with a
     single device-to-host copy for all of them."""
-    pending = [p for p in plans if p is not None and p.items < 0]
-    for p in [p for p in pending if p.ready is not None]:
-        p.ready.synchronize()
-        p.items, p.heavy = (int(x) for x in p.host_counts.tolist())
-        p.counts = p.host_counts = p.ready = None
-        p._slot()              # the slot goes back to the pool (the finalizer runs once)
-    pending = [p for p in pending if p.items < 0]
+    pending = [p for p in plans if p is not None and p.items < 0]     # items reads the copies that there are
     if not pending:
         return
     # plans made with one shared counts buffer (split_plan(..., counts=...)) come back in one copy
@@ -899,7 +915,7 @@ def resolve_plans(*plans) -> None:
     else:
         vals = torch.cat([p.counts for p in pending]).cpu().tolist()
     for i, p in enumerate(pending):
-        p.items, p.heavy, p.counts = int(vals[2 * i]), int(vals[2 * i + 1]), None
+        p._items, p._heavy, p.counts = int(vals[2 * i]), int(vals[2 * i + 1]), None
 
 
 def split_plan_first_row(n_rows: int, n_items: int, nnz: int, threshold: int, item_size: int,
@@ -942,7 +958,7 @@ def split_plan(ptr: torch.Tensor, nnz: int, threshold: int = DEFAULT_CHUNK, item
            _p(heavy_rows), heavy_cap, _p(counts), _p(ws), ws.numel(), _stream(dev))
     plan = SplitPlan(-1, -1, nitems, item_off, item_row, heavy_rows, counts, item_cap, heavy_cap)
     if known is not None:
-        plan.items, plan.heavy = int(known[0]), int(known[1])
+        plan._items, plan._heavy = int(known[0]), int(known[1])
     elif resolve:
         resolve_plans(plan)
     elif host_copy:
@@ -953,6 +969,7 @@ def split_plan(ptr: torch.Tensor, nnz: int, threshold: int = DEFAULT_CHUNK, item
 
 
 # ------------------------------------------------------------------ attention index
+DEVICE_PLAN_MAX_ITEMS = 1 << 14      # plans of up to this many items (at capacity) need no host copy of their counts
 NO_READBACK_MAX_ENTRIES = 1 << 23   # tables of up to this many entries (at capacity) build without a host read
 
 
@@ -1131,12 +1148,24 @@ class AttentionIndex:
         src = expand_rows(self.kptr, self.nnz)
         return torch.stack([src, self.kq.to(torch.int64)])
 
+    def _plans_on_device(self, backward: bool) -> tuple:
+        """Which of the plans a call uses keep their counts on the device. A plan's pinned copy is waited for only
+        where the capacities would cost the launches more than the wait costs the stream: in a first layer on a new
+        index the host is ahead of the copy, and waiting for it left the GPU idle until the host had caught up
+        (169K nodes: step 662 -> 630 us). Later layers find the copy landed and pass the counts."""
+        out = []
+        for p in (self.qplan, self.kplan if backward else None):
+            if p is not None and p.item_cap > DEVICE_PLAN_MAX_ITEMS and p.ready is not None:
+                p.items                # waits
+            out.append(p is not None and p.pending)
+        return tuple(out)
+
     def struct(self, backward: bool, entries: bool = False) -> N.AttnIndex:
         self.ensure_backward(entries) if backward else self.ensure_forward()
         if backward and entries:
             self.ensure_entries()
         # the index does not change once built: every layer and step reuses the same struct
-        key = (backward, backward and self.ks_all is not None, self.nnz_known)
+        key = (backward, backward and self.ks_all is not None, self.nnz_known, self._plans_on_device(backward))
         cached = self._structs.get(key)
         if cached is not None:
             return cached
@@ -1159,10 +1188,8 @@ class AttentionIndex:
         t["qptr"], t["kv"] = self.qptr, self.kv_all if self.cap else None
         n["chunk"], n["item"] = self.chunk, self.item
         qp = self.qplan
-        # plans with a pinned copy of their counts take them from it; the others stay pending, their
-        # capacities size the grids and the kernels read the counts from the device
-        resolve_plans(*[p for p in (qp, self.kplan if backward else None) if p is not None and p.ready is not None])
-        # (a plan whose counts are known passes them: the device copy then holds the same values)
+        # a plan without counts on the host stays pending: its capacities size the launches and the kernels read the
+        # counts from the device (where another plan's counts are known the device copy holds the same values)
         on_device = qp.pending or (backward and self.kplan.pending)
         n["q_items"], n["q_heavy"] = (qp.item_cap, qp.heavy_cap) if qp.pending else (qp.items, qp.heavy)
         t["plan_counts"] = self._counts if on_device else None
@@ -1196,7 +1223,7 @@ class AttentionIndex:
         self.ensure_backward(entries) if backward else self.ensure_forward()
         if backward and entries:
             self.ensure_entries()
-        key = ("op", backward, backward and self.ks_all is not None, self.nnz_known)
+        key = ("op", backward, backward and self.ks_all is not None, self.nnz_known, self._plans_on_device(backward))
         cached = self._structs.get(key)
         if cached is None:
             t, n = self._fields(backward)
