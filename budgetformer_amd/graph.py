@@ -48,8 +48,16 @@ class CSRGraph:
         """
         cache = self.__dict__.setdefault("_hubs", {})
         if threshold not in cache:
-            plan = hip_ops.split_plan(self.in_ptr, self.num_edges, threshold, max(threshold, 1))
-            cache[threshold] = plan.heavy_rows[: plan.heavy].clone()
+            # a build asks for both of the usual lists: they are found together, with one host read
+            usual = (hip_ops.LIGHT_MAX, hip_ops.HUB_THRESHOLD)
+            wanted = [t for t in usual if t not in cache] if threshold in usual else [threshold]
+            counts = torch.empty(2 * len(wanted), dtype=torch.int32, device=self.device)
+            plans = [hip_ops.split_plan(self.in_ptr, self.num_edges, t, max(t, 1), resolve=False,
+                                        counts=counts[2 * i:2 * i + 2], host_copy=False)
+                     for i, t in enumerate(wanted)]
+            hip_ops.resolve_plans(*plans)
+            for t, plan in zip(wanted, plans):
+                cache[t] = plan.heavy_rows[: plan.heavy].clone()
         return cache[threshold]
 
     def walk_records(self, reserve_bytes: Optional[int] = None) -> Optional[torch.Tensor]:
@@ -91,12 +99,7 @@ class CSRGraph:
         pass a coalesced edge list as the reference does.
         """
         ei = edge_index.to(device)
-        src, dst = hip_ops._pair_lists(ei)
-        rowptr, col = hip_ops.coo_rows_to_csr(src, dst, num_nodes, num_nodes)
-        if symmetric:
-            return cls(rowptr, col, rowptr, col, int(num_nodes))
-        in_ptr, in_src = hip_ops.coo_rows_to_csr(dst, src, num_nodes, num_nodes)
-        return cls(rowptr, col, in_ptr, in_src, int(num_nodes))
+        return cls(*hip_ops.graph_csrs(ei, num_nodes, symmetric=bool(symmetric)), int(num_nodes))
 
 
 # ------------------------------------------------------------------ topology ingest

@@ -346,8 +346,7 @@ def _get_random_walk_graph(edge_index: torch.Tensor, num_nodes: int, device):
     # the entry pins its source tensor, so a hit is the same tensor (same version), not a reused address
     if hit is not None and hit[0] is edge_index and hit[1] == edge_index._version:
         return hit[2]
-    src, dst = hip_ops._pair_lists(hip_ops.coalesced(edge_index.to(dev), num_nodes))
-    rowptr, col = hip_ops.coo_rows_to_csr(src, dst, num_nodes, num_nodes)
+    rowptr, col, _, _ = hip_ops.graph_csrs(edge_index.to(dev), num_nodes, symmetric=None, coalesced=True)
     placeholder = torch.empty((2, 0), dtype=edge_index.dtype, device=dev)
     _RANDOM_WALK_GRAPH_CACHE.clear()
     _RANDOM_WALK_GRAPH_CACHE[key] = (edge_index, edge_index._version, (placeholder, rowptr, col))

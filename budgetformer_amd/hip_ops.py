@@ -208,27 +208,44 @@ def _coalesced(fn: str, edge_index: torch.Tensor, num_nodes: int, capacity: int)
     return out[:, : cnt.value]
 
 
-def _is_coalesced(edge_index: torch.Tensor, num_nodes: int) -> bool:
-    src, dst = _pair_lists(edge_index)
-    if not 0 < src.numel() < 2 ** 31:
-        return False
-    holds = _coo_holds(src, dst, num_nodes, num_nodes)
+def _holds_coalesced(src: torch.Tensor, dst: torch.Tensor, num_nodes: int) -> int:
+    """``_coo_holds`` of a list by (src, dst), or 0 where it cannot be a coalesced one."""
+    return _coo_holds(src, dst, num_nodes, num_nodes) if 0 < src.numel() < 2 ** 31 else 0
+
+
+def _is_coalesced(holds: int) -> bool:
     return bool(holds & N.COO_STRICT and holds & N.COO_IDS)
 
 
 def coalesce(edge_index: torch.Tensor, num_nodes: int) -> torch.Tensor:
     """Sort by (src, dst) and drop duplicates (torch_geometric.utils.coalesce), on the device. A list that is
     coalesced already is copied, not sorted again."""
-    if _is_coalesced(edge_index, num_nodes):
-        return torch.stack(_pair_lists(edge_index))
-    return _coalesced("bf_coalesce", edge_index, num_nodes, edge_index[0].numel())
+    src, dst = _pair_lists(edge_index)
+    if _is_coalesced(_holds_coalesced(src, dst, num_nodes)):
+        return torch.stack([src, dst])
+    return _coalesced("bf_coalesce", edge_index, num_nodes, src.numel())
 
 
-def coalesced(edge_index: torch.Tensor, num_nodes: int) -> torch.Tensor:
-    """``coalesce`` for a caller that only reads the result: a coalesced list itself, else its coalesced copy."""
-    if _is_coalesced(edge_index, num_nodes):
-        return edge_index
-    return _coalesced("bf_coalesce", edge_index, num_nodes, edge_index[0].numel())
+def graph_csrs(edge_index: torch.Tensor, num_nodes: int, symmetric: bool = False, coalesced: bool = False):
+    """(rowptr, col, in_ptr, in_src) of an edge list: its CSR by source and by target (the same arrays for a
+    ``symmetric`` list, None for both with ``symmetric=None``). With ``coalesced`` the list is coalesced first, where
+    it is not so already. The list's order is looked at once for all of it."""
+    src, dst = _pair_lists(edge_index)
+    n = num_nodes
+    holds = _coo_holds(src, dst, n, n)
+    if coalesced and not _is_coalesced(holds):
+        src, dst = _pair_lists(_coalesced("bf_coalesce", edge_index, n, src.numel()))
+        if holds & N.COO_IDS:          # ids in range stay so, and the result is in (src, dst) order
+            holds = N.COO_IDS | N.COO_ROW_MAJOR | N.COO_STRICT | N.COO_BY_ROW
+        else:
+            holds = _coo_holds(src, dst, n, n)
+    rowptr, col = coo_rows_to_csr(src, dst, n, n, holds=holds)
+    if symmetric or symmetric is None:
+        return (rowptr, col) + ((rowptr, col) if symmetric else (None, None))
+    turned = holds & (N.COO_IDS | N.COO_TYPES)
+    for a, b in ((N.COO_ROW_MAJOR, N.COO_COL_MAJOR), (N.COO_BY_ROW, N.COO_BY_COL)):
+        turned |= (b if holds & a else 0) | (a if holds & b else 0)
+    return (rowptr, col) + coo_rows_to_csr(dst, src, n, n, holds=turned)
 
 
 def coalesce_bidirected(edge_index: torch.Tensor, num_nodes: int) -> torch.Tensor:
@@ -631,15 +648,17 @@ def split_row_items(length: int, item_size: int = DEFAULT_ITEM) -> int:
 
 
 def coo_rows_to_csr(rows: torch.Tensor, cols: torch.Tensor, n_rows: int, n_cols: int,
-                    types: Optional[torch.Tensor] = None, with_keys: bool = False):
+                    types: Optional[torch.Tensor] = None, with_keys: bool = False, holds: Optional[int] = None):
     """CSR of the entries (rows[i], cols[i]) (int64, any order): (ptr int64 [n_rows+1], ids int32 [nnz] ascending
     within a row). ``types`` (int64, 0 or 1): rows ordered by (type, id), the type in bit 31 of each id. With
     ``with_keys`` also (keys, in_order): the entries' sort keys for ``coo_reverse``. Ids are checked on the device
-    (ValueError), and a list that is in row or column order already is sorted by the missing bits only."""
+    (ValueError), and a list that is in row or column order already is sorted by the missing bits only. ``holds``: what
+    ``_coo_holds`` says of this list, where the caller has asked."""
     dev = rows.device
     stream = _stream(dev)
     nnz = rows.numel()
-    holds = _coo_holds(rows, cols, n_rows, n_cols, types)
+    if holds is None:
+        holds = _coo_holds(rows, cols, n_rows, n_cols, types)
     if types is not None and not holds & N.COO_TYPES:
         raise ValueError("edge types must be 0 or 1")
     if not holds & N.COO_IDS:

@@ -185,8 +185,7 @@ def _graph_for(edge_index_global, num_nodes, device) -> CSRGraph:
     # the entry pins its source tensor, so a hit is the same tensor (same version), not a reused address
     if hit is not None and hit[0] is edge_index_global and hit[1] == edge_index_global._version:
         return hit[2]
-    ei = hip_ops.coalesced(edge_index_global.to(dev), int(num_nodes))
-    g = CSRGraph.from_edge_index(ei, int(num_nodes), symmetric=False, device=dev)
+    g = CSRGraph(*hip_ops.graph_csrs(edge_index_global.to(dev), int(num_nodes), coalesced=True), int(num_nodes))
     _GRAPH_CACHE.clear()
     _GRAPH_CACHE[key] = (edge_index_global, edge_index_global._version, g)
     return g

@@ -93,8 +93,19 @@ def test_coalesce_and_bidirected(hip_device, nnz, n):
     assert np.array_equal(to_bidirected(dev, n).cpu().numpy(), ref(np.concatenate([ei, ei[::-1]], axis=1)))
     again = hip_ops.coalesce(got, n)
     assert torch.equal(again, got) and (nnz == 0 or again.data_ptr() != got.data_ptr())
-    assert hip_ops.coalesced(again, n) is again or nnz == 0
-    assert np.array_equal(hip_ops.coalesced(dev, n).cpu().numpy(), ref(ei))
+    # both CSRs of the list as it comes, of its coalesced form, and of the coalesced list itself
+    for x, flag in ((dev, False), (dev, True), (again, True), (again.flip(0), False)):
+        e = ref(ei) if flag else x.cpu().numpy()
+        out = hip_ops.graph_csrs(x, n, coalesced=flag)
+        for ptr, ids, r, c in ((out[0], out[1], e[0], e[1]), (out[2], out[3], e[1], e[0])):
+            o = np.lexsort((c, r))
+            assert np.array_equal(ptr.cpu().numpy(), np.searchsorted(r[o], np.arange(n + 1)))
+            assert np.array_equal(ids.cpu().numpy(), c[o])
+    if nnz:
+        for bad in (n, -1):
+            dev[0, 0] = bad
+            with pytest.raises(ValueError, match="ids outside"):
+                hip_ops.graph_csrs(dev, n)
 
 
 @pytest.mark.parametrize("token", [False, True])
