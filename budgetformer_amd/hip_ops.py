@@ -954,6 +954,13 @@ def split_plan_first_row(n_rows: int, n_items: int, nnz: int, threshold: int, it
                      heavy_cap)
 
 
+def _plan_of(arrays, counted: tuple, counts: torch.Tensor, nnz: int, threshold: int, item_size: int) -> SplitPlan:
+    """The plan of an operator's arrays (nitems, item_off, item_row, heavy_rows); ``counted``: (items, split rows)."""
+    lib = N.load()
+    return SplitPlan(*counted, *arrays, counts, int(lib.bf_split_item_capacity(nnz, threshold, item_size)),
+                     int(lib.bf_split_row_capacity(nnz, threshold)))
+
+
 def split_plan(ptr: torch.Tensor, nnz: int, threshold: int = DEFAULT_CHUNK, item_size: int = DEFAULT_ITEM,
                resolve: bool = True, counts: Optional[torch.Tensor] = None,
                known: Optional[tuple] = None, host_copy: bool = True) -> SplitPlan:
@@ -1114,9 +1121,22 @@ class AttentionIndex:
                                     counts=self._plan_counts(0), known=self._q_known,
                                     host_copy=self._host_copy())
         if self.kptr is None:
-            if self._rkeys is not None and self._rkeys.q_bits + self._rkeys.slot_bits + _bits_for(self.n_kv) <= 64:
-                self.kptr, self.kq_all, ks, srt = reverse_index_packed(self._rkeys, self.qptr, self.n_kv,
-                                                                       entries=entries)
+            rk = self._rkeys
+            if rk is not None and rk.q_bits + rk.slot_bits + _bits_for(self.n_kv) <= 64:
+                if self.kplan is None and self.korder is None and 1 <= self.chunk <= 254:
+                    # the whole key side in one operator
+                    nnz, counts = _entries_of(rk, self.qptr), self._plan_counts(1)
+                    self.kptr, self.kq_all, keys, self.korder, self.kspans, *rest = \
+                        N.load_ops().reverse_index_and_plan(
+                            rk.keys, self.qptr, nnz, self.n_kv, rk.q_bits, rk.slot_bits, rk.global_token,
+                            rk.token_row, entries, self.chunk, self.item, counts)
+                    ks = rest.pop() if entries else None
+                    srt = ReverseKeys(keys, rk.q_bits, rk.slot_bits, rk.global_token, rk.token_row)
+                    self.kplan = _plan_of(rest, (-1, -1), counts, nnz, self.chunk, self.item)
+                    if self._host_copy():
+                        _copy_counts_to_host(self.kplan, self.device)
+                else:
+                    self.kptr, self.kq_all, ks, srt = reverse_index_packed(rk, self.qptr, self.n_kv, entries=entries)
                 if entries:
                     self.ks_all = ks
                 else:
@@ -1276,13 +1296,28 @@ class AttentionIndex:
         if width + (1 if global_token else 0) <= chunk:
             split = tr > chunk
             known = (split_row_items(tr, item) if split else 0, 1 if split else 0)
-        qptr = table_qptr(table, row_len, global_token, tr)
+        bound = n_rows * width + (n_rows if global_token else 0) + max(tr, 0)
+        exact = bound > NO_READBACK_MAX_ENTRIES
+        q_bits, slot_bits = _bits_for(n_q_tab), _bits_for(width)
+        # one operator does the whole query side where its sizes are known and the keys fit their field
+        fused = known is not None and not exact and q_bits + slot_bits <= 33
+        if fused:
+            _require(table, "table", torch.int32)
+            _require(row_len, "row_len", torch.int32, table.device)
         # the token fill puts key 0 first in every table row and shifts the table's own ids past it:
         # key 0 is then attended by every query row from 1 on (with the token row) or from 0 on (without)
         token_column = 0 if not global_token else (1 if tr >= 0 else 2)
-        idx = cls(n_q=n_q_tab, n_kv=n_kv, qptr=qptr, kv_all=None, chunk=chunk, item=item,
+        idx = cls(n_q=n_q_tab, n_kv=n_kv, qptr=None, kv_all=None, chunk=chunk, item=item,
                   token_column=token_column, _q_known=known)
-        bound = n_rows * width + (n_rows if global_token else 0) + max(tr, 0)
+        if fused:
+            counts = idx._counts = torch.empty(4, dtype=torch.int32, device=table.device)
+            idx.qptr, idx.kv_all, keys, *plan = N.load_ops().table_index(
+                table, row_len, bool(global_token), tr, bound, n_rows * width, q_bits, slot_bits, known[0], chunk,
+                item, counts)
+            idx._rkeys = ReverseKeys(keys, q_bits, slot_bits, bool(global_token), tr)
+            idx.qplan = _plan_of(plan, known, counts[:2], bound, chunk, item)
+            return idx
+        idx.qptr = qptr = table_qptr(table, row_len, global_token, tr)
         if known is not None:
             # only the token row can be split: its plan is written in one pass, before any read of nnz
             idx.qplan = split_plan_first_row(n_q_tab, known[0], bound, chunk, item, idx._plan_counts(0))
@@ -1290,8 +1325,8 @@ class AttentionIndex:
         # back, so the host runs ahead of the kernels. A large one reads nnz once and sizes its arrays and
         # grids exactly (a B=32 table fills well under half of its capacity).
         qptr, idx.kv_all, idx._rkeys = table_to_csr(table, row_len, global_token, with_keys=True, qptr=qptr,
-                                                    token_row=tr, exact=bound > NO_READBACK_MAX_ENTRIES)
-        if bound > NO_READBACK_MAX_ENTRIES:
+                                                    token_row=tr, exact=exact)
+        if exact:
             idx._nnz = idx.kv_all.numel()
         return idx
 

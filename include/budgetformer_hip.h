@@ -489,7 +489,7 @@ int bf_reverse_index_packed(const uint64_t* rkey, const int64_t* qptr, int64_t n
                             size_t workspace_bytes, void* stream);
 /* The stable radix sort bf_reverse_index_packed uses, on its own: in[0, n)
  * uint64 sorted by bits [begin_bit, end_bit) into out (n < 2^31; in and out
- * must not overlap). 8- or 9-bit digits, whichever needs fewer passes; each
+ * must not overlap). Equal digits of 6 to 10 bits, by the cost of their passes; each
  * pass counts digits per tile, scans the counts per digit and scatters. No
  * counterpart in the reference (torch.sort / coalesce sort inside PyTorch).
  * Workspace: bf_radix_sort_workspace_size(n, begin_bit, end_bit).          */

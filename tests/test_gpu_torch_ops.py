@@ -157,3 +157,49 @@ def test_edge_ops_against_the_oracle(hip_device, records):
     assert np.array_equal(ks.cpu().numpy(), slots[order])
     assert np.array_equal(kq.cpu().numpy(), rows[order])
     assert np.array_equal(kptr.cpu().numpy(), np.concatenate([[0], np.cumsum(np.bincount(flat, minlength=n))]))
+
+
+@pytest.mark.parametrize("n,width,token_row", [(0, 4, None), (1, 1, None), (300, 17, None), (1500, 64, None),
+                                               (300, 17, 0), (300, 17, 1500), (300, 17, -1)])
+@pytest.mark.parametrize("token", [False, True])
+def test_index_operators_equal_the_single_calls(hip_device, n, width, token_row, token):
+    """table_index and reverse_index_and_plan (a table's whole index) against table_to_csr, reverse_index_packed and
+    row_order_and_plan, bit for bit: whole numbers, so no tolerance. Only the order of equally long rows is free."""
+    from budgetformer_amd import hip_ops
+    from budgetformer_amd.hip_ops import AttentionIndex
+    if not token and token_row is not None:
+        pytest.skip("a token row without the token")
+    rng = np.random.default_rng(n + width)
+    n_kv = max(n, token_row or 0) + 1
+    table = torch.tensor(rng.integers(0, max(n, 1), (n, width)), dtype=torch.int32, device=hip_device)
+    table[:, 0] = 0                                           # one long key row: the key-side plan splits it
+    row_len = torch.tensor(rng.integers(0, width + 1, n), dtype=torch.int32, device=hip_device)
+    idx = AttentionIndex.from_table(table, row_len, token, n_kv=n_kv, check=False, token_row=token_row)
+    qptr, kv, rk = hip_ops.table_to_csr(table, row_len, token, with_keys=True, token_row=token_row)
+    assert torch.equal(idx.qptr, qptr) and torch.equal(idx.kv, kv)
+    tr = n if token_row is None else token_row
+    split = hip_ops.split_plan(qptr, kv.numel(), idx.chunk, idx.item)
+    assert (idx.qplan.items, idx.qplan.heavy) == (split.items, split.heavy) == \
+        ((hip_ops.split_row_items(tr, idx.item), 1) if token and tr > idx.chunk else (0, 0))
+    assert torch.equal(idx.qplan.item_row[:split.items], split.item_row[:split.items])
+    kptr, kq, ks, _ = hip_ops.reverse_index_packed(rk, qptr, n_kv)
+    order, spans, plan = hip_ops.row_order_and_plan(kptr, kv.numel(), idx.chunk, idx.item)
+    for entries in (False, True):
+        if entries:
+            idx = AttentionIndex.from_table(table, row_len, token, n_kv=n_kv, check=False, token_row=token_row)
+        idx.ensure_backward(entries)
+        assert (idx.ks_all is not None) == entries
+        idx.ensure_entries()
+        assert torch.equal(idx.kptr, kptr) and torch.equal(idx.kq, kq)
+        assert torch.equal(idx.ks, ks) if kv.numel() else idx.ks is None or idx.ks.numel() == 0
+        idx.resolve()
+        hip_ops.resolve_plans(plan)
+        assert (idx.kplan.items, idx.kplan.heavy) == (plan.items, plan.heavy)
+        rows = idx.korder.long()
+        lengths = (kptr[1:] - kptr[:-1])
+        assert torch.equal(rows.sort().values, torch.arange(n_kv, device=hip_device))
+        assert torch.equal(idx.kspans, kptr[rows] << 32 | lengths[rows])
+        assert torch.equal(lengths[rows].clamp(max=255), lengths[order.long()].clamp(max=255))
+        heavy = idx.kplan.heavy_rows[:plan.heavy]
+        assert torch.equal(heavy.sort().values, plan.heavy_rows[:plan.heavy].sort().values)
+        assert torch.equal(idx.kplan.nitems[heavy.long()], plan.nitems[heavy.long()])
