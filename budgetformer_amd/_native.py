@@ -20,9 +20,8 @@ ABI_VERSION = 303                   # the header's BF_ABI_VERSION this binding i
 BF_MAX_ITEMS_PER_ROW = 160          # items a split row is cut into at most (the header's #define) ...
 BF_LONG_ROW_FACTOR = 64             # ... unless it is longer than 160 * 64 items' worth (the header's #define)
 
-# what a COO list holds (the header's BF_COO_* bits) and bf_coo_order's workspace in bytes
+# what a COO list holds (the header's BF_COO_* bits)
 COO_IDS, COO_TYPES, COO_ROW_MAJOR, COO_COL_MAJOR, COO_STRICT, COO_BY_COL, COO_BY_ROW = 1, 2, 4, 8, 16, 32, 64
-COO_ORDER_WORKSPACE = 4096
 
 i32, i64, u64, sz, f32 = C.c_int32, C.c_int64, C.c_uint64, C.c_size_t, C.c_float
 vp = C.c_void_p
@@ -100,7 +99,8 @@ _SIGS = {
     "bf_scan_workspace_size": (C.c_int, [i64, C.POINTER(sz)]),
     "bf_coo_to_csr_workspace_size": (C.c_int, [i64, i64, C.POINTER(sz)]),
     "bf_coo_to_csr": (C.c_int, [P_i64, P_i64, i64, i64, i64, P_i64, P_i32, vp, sz, vp]),
-    "bf_coo_order": (C.c_int, [P_i64, P_i64, P_i64, i64, i64, i64, C.POINTER(i32), vp, sz, vp]),
+    "bf_coo_order": (C.c_int, [P_i64, P_i64, P_i64, i64, i64, i64, C.POINTER(i32), vp]),
+    "bf_any_nonzero": (C.c_int, [P_i32, i64, C.POINTER(i32), vp]),
     "bf_coo_to_csr_ordered_workspace_size": (C.c_int, [i64, i64, i64, i32, i32, C.POINTER(sz)]),
     "bf_coo_to_csr_ordered": (C.c_int, [P_i64, P_i64, P_i64, i64, i64, i64, i32, P_i64, P_i32, vp, vp, sz, vp]),
     "bf_coo_reverse_workspace_size": (C.c_int, [i64, i64, i64, i32, i32, C.POINTER(sz)]),

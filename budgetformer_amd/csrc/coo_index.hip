@@ -11,8 +11,6 @@
 // Against the former route (four torch reductions with three host reads, a
 // 64-bit onesweep sort over all bits, separate passes for the ids and the row
 // pointers) a 1.17M-entry list's CSR went from 430 to 190 us, host reads included.
-#include <vector>
-
 #include "bf_common.h"
 #include "bf_sort.h"
 
@@ -31,8 +29,8 @@ int bits_for(uint64_t maxval) {
 }
 
 // ---------------------------------------------------------------- the order of a list
-// Each block ORs what its share of the list violates (the BF_COO_* bits), one word per block: nothing to
-// clear before and no atomics; the host ORs the words.
+// Each block ORs what its share of the list violates (the BF_COO_* bits), one word per block in pinned host
+// memory: nothing to clear before and no atomics; the host ORs the words.
 constexpr int64_t kOrderBlocks = 1024;
 
 __global__ __launch_bounds__(kThreads) void coo_order_kernel(const int64_t* __restrict__ row,
@@ -362,6 +360,41 @@ __global__ __launch_bounds__(kThreads) void table_list_check_kernel(const int32_
   }
 }
 
+// The blocks' sums become their first places; out (pinned host memory) gets the entries, the bad lengths and the bad
+// ids. One workgroup, and the host reads 24 bytes: copying the blocks' words (54 KB in two arrays for 2.3M rows) to
+// add them up there takes 52 us, a kernel's own store of the sums 11.5 us, launch and wait included in both.
+constexpr int kTotalsThreads = 1024;
+__global__ __launch_bounds__(kTotalsThreads) void list_totals_kernel(uint32_t* __restrict__ sums,
+                                                                     const uint32_t* __restrict__ bad, int64_t blocks,
+                                                                     uint64_t* __restrict__ out) {
+  __shared__ uint32_t tmp[kTotalsThreads / 64];
+  __shared__ uint64_t all_bad[2];
+  if (threadIdx.x < 2) all_bad[threadIdx.x] = 0;
+  __syncthreads();
+  uint64_t total = 0;          // the places wrap from 2^32 entries on, which the host refuses
+  uint64_t bad_len = 0, bad_id = 0;
+  for (int64_t base = 0; base < blocks; base += kTotalsThreads) {
+    const int64_t b = base + threadIdx.x;
+    const uint32_t v = b < blocks ? sums[b] : 0;
+    if (b < blocks) {
+      bad_len += bad[2 * b];
+      bad_id += bad[2 * b + 1];
+    }
+    uint32_t tot;
+    const uint32_t e = sort::block_excl_scan<kTotalsThreads>(v, tmp, &tot);
+    if (b < blocks) sums[b] = uint32_t(total) + e;
+    total += tot;
+  }
+  if (bad_len) atomicAdd(reinterpret_cast<unsigned long long*>(&all_bad[0]), (unsigned long long)bad_len);
+  if (bad_id) atomicAdd(reinterpret_cast<unsigned long long*>(&all_bad[1]), (unsigned long long)bad_id);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    out[0] = total;
+    out[1] = all_bad[0];
+    out[2] = all_bad[1];
+  }
+}
+
 template <typename I>   // of a slot within the block: 32 bits unless the rows are very wide
 __global__ __launch_bounds__(kThreads) void table_list_keys_kernel(const int32_t* __restrict__ table,
                                                                    const int32_t* __restrict__ row_len,
@@ -450,29 +483,25 @@ struct Carve {            // consecutive 256-byte aligned pieces of a workspace
 using namespace bf;
 
 extern "C" int bf_coo_order(const int64_t* row, const int64_t* col, const int64_t* type, int64_t nnz, int64_t n_row,
-                            int64_t n_col, int32_t* holds_host, void* workspace, size_t workspace_bytes,
-                            void* stream) {
+                            int64_t n_col, int32_t* holds_host, void* stream) {
   BF_CHECK_ARG(holds_host && nnz >= 0 && n_row >= 0 && n_col >= 0, "coo_order: bad arguments");
   constexpr int32_t kAll = BF_COO_IDS | BF_COO_TYPES | BF_COO_ROW_MAJOR | BF_COO_COL_MAJOR | BF_COO_STRICT |
                            BF_COO_BY_COL | BF_COO_BY_ROW;
   *holds_host = kAll;
   if (nnz == 0) return BF_OK;
   BF_CHECK_ARG(row && col, "coo_order: null tensor");
-  BF_CHECK_ARG(workspace && workspace_bytes >= BF_COO_ORDER_WORKSPACE, "coo_order: workspace %zu < %d bytes",
-               workspace_bytes, BF_COO_ORDER_WORKSPACE);
-  static_assert(BF_COO_ORDER_WORKSPACE == kOrderBlocks * sizeof(uint32_t), "one word per block");
+  static_assert(kHostReadBytes >= kOrderBlocks * sizeof(uint32_t), "one word per block");
+  BF_HOST_READ(read);
   hipStream_t st = as_stream(stream);
   const int64_t want = ceil_div(nnz, int64_t(kThreads) * 4);
   const int64_t blocks = want < kOrderBlocks ? want : kOrderBlocks;
-  auto* words = static_cast<uint32_t*>(workspace);
+  auto* words = read.as<uint32_t>();
   BF_LAUNCH("coo_order_kernel", coo_order_kernel, dim3(unsigned(blocks)), dim3(kThreads), 0, st, row, col, type, nnz,
             n_row, n_col, words);
   BF_CHECK_LAUNCH();
-  uint32_t h[kOrderBlocks];
-  BF_CHECK_HIP(hipMemcpyAsync(h, words, size_t(blocks) * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
   BF_CHECK_HIP(hipStreamSynchronize(st));
   uint32_t broken = 0;
-  for (int64_t b = 0; b < blocks; ++b) broken |= h[b];
+  for (int64_t b = 0; b < blocks; ++b) broken |= words[b];
   *holds_host = kAll & ~int32_t(broken);
   return BF_OK;
 }
@@ -617,7 +646,8 @@ int coalesce_list(const PairKeys& in, int64_t total, int64_t num_nodes, int64_t*
   Carve ws{static_cast<char*>(workspace)};
   auto* keys = ws.take<uint64_t>(size_t(total) * 8);
   auto* counts = ws.take<uint32_t>(size_t(tiles) * 4);
-  auto* count = ws.take<uint32_t>(4);
+  BF_HOST_READ(read);
+  auto* count = read.as<uint32_t>();
   const int end_bit = bits_for(uint64_t(num_nodes) * uint64_t(num_nodes));
   BF_CHECK_OK(sort::radix_sort(in, keys, total, 0, end_bit, ws.p,
                                workspace_bytes - size_t(ws.p - static_cast<char*>(workspace)), st));
@@ -629,10 +659,8 @@ int coalesce_list(const PairKeys& in, int64_t total, int64_t num_nodes, int64_t*
   BF_LAUNCH("unique_write_kernel", unique_write_kernel, dim3(unsigned(tiles)), dim3(kThreads), 0, st, keys, total,
             counts, uint64_t(num_nodes), out_src, out_dst);
   BF_CHECK_LAUNCH();
-  uint32_t h = 0;
-  BF_CHECK_HIP(hipMemcpyAsync(&h, count, sizeof(h), hipMemcpyDeviceToHost, st));
   BF_CHECK_HIP(hipStreamSynchronize(st));
-  *count_host = h;
+  *count_host = *count;
   return BF_OK;
 }
 }  // namespace
@@ -696,16 +724,12 @@ extern "C" int bf_table_list_check(const int32_t* table, const int32_t* row_len,
     BF_LAUNCH("table_list_check_kernel", table_list_check_kernel<uint64_t>, dim3(unsigned(blocks)), dim3(kThreads), 0,
               st, table, row_len, n_rows, width, id_limit, sums, bad);
   BF_CHECK_LAUNCH();
-  std::vector<uint32_t> h(size_t(blocks) * 3);
-  BF_CHECK_HIP(hipMemcpyAsync(h.data(), sums, size_t(blocks) * 4, hipMemcpyDeviceToHost, st));
-  BF_CHECK_HIP(hipMemcpyAsync(h.data() + blocks, bad, size_t(blocks) * 8, hipMemcpyDeviceToHost, st));
+  BF_HOST_READ(read);
+  auto* h = read.as<uint64_t>();
+  BF_LAUNCH("list_totals_kernel", list_totals_kernel, dim3(1), dim3(kTotalsThreads), 0, st, sums, bad, blocks, h);
+  BF_CHECK_LAUNCH();
   BF_CHECK_HIP(hipStreamSynchronize(st));
-  int64_t nnz = 0, bad_len = 0, bad_id = 0;
-  for (int64_t b = 0; b < blocks; ++b) {
-    nnz += h[size_t(b)];
-    bad_len += h[size_t(blocks + 2 * b)];
-    bad_id += h[size_t(blocks + 2 * b + 1)];
-  }
+  const int64_t nnz = int64_t(h[0]), bad_len = int64_t(h[1]), bad_id = int64_t(h[2]);
   BF_CHECK_ARG(bad_len == 0, "check_table: %lld row lengths outside [0, %d]", (long long)bad_len, width);
   BF_CHECK_ARG(bad_id == 0, "check_table: %lld table ids outside [0, %lld)", (long long)bad_id, (long long)id_limit);
   BF_CHECK_ARG(nnz < (int64_t(1) << 31), "table_list_check: %lld entries (at most 2^31 - 1)", (long long)nnz);
@@ -745,10 +769,7 @@ extern "C" int bf_table_to_list(const int32_t* table, const int32_t* row_len, in
     auto* keys = ws.take<uint64_t>(size_t(nnz) * 8);
     sorted = ws.take<uint64_t>(size_t(nnz) * 8);
     const int64_t blocks = list_blocks(n_rows);
-    auto* sums = static_cast<uint32_t*>(checked);    // become the blocks' first places
-    BF_LAUNCH("radix_scan_kernel", sort::radix_scan_kernel, dim3(1), dim3(sort::kThreads), 0, st, sums, blocks,
-              sums + blocks);
-    BF_CHECK_LAUNCH();
+    const auto* sums = static_cast<const uint32_t*>(checked);    // the blocks' first places
     if (width <= kListWidth32)
       BF_LAUNCH("table_list_keys_kernel", table_list_keys_kernel<uint32_t>, dim3(unsigned(blocks)), dim3(kThreads), 0,
                 st, table, row_len, n_rows, width, sums, qb, keys);

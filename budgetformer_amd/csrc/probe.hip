@@ -211,10 +211,37 @@ int clear_nodes(const NodeSpace& s, int64_t n, hipStream_t st) {
   return BF_OK;
 }
 
+// *any = 1 when an entry is not 0: a store by each workgroup that finds one, to pinned host memory cleared before.
+__global__ __launch_bounds__(kThreads) void any_nonzero_kernel(const int32_t* __restrict__ x, int64_t n,
+                                                               int32_t* __restrict__ any) {
+  bool found = false;
+  const int64_t stride = int64_t(gridDim.x) * kThreads;
+  for (int64_t i = int64_t(blockIdx.x) * kThreads + threadIdx.x; i < n && !found; i += stride) found = x[i] != 0;
+  if (__syncthreads_or(found) && threadIdx.x == 0) *any = 1;
+}
+
 }  // namespace
 }  // namespace bf
 
 using namespace bf;
+
+extern "C" int bf_any_nonzero(const int32_t* x, int64_t n, int32_t* any_host, void* stream) {
+  BF_CHECK_ARG(n >= 0 && any_host, "any_nonzero: bad arguments");
+  *any_host = 0;
+  if (n == 0) return BF_OK;
+  BF_CHECK_ARG(x, "any_nonzero: null tensor");
+  hipStream_t st = as_stream(stream);
+  BF_HOST_READ(read);
+  auto* any = read.as<int32_t>();
+  *any = 0;
+  const int64_t want = ceil_div(n, int64_t(kThreads) * 4);
+  BF_LAUNCH("any_nonzero_kernel", any_nonzero_kernel, dim3(unsigned(want < 256 ? want : 256)), dim3(kThreads), 0, st,
+            x, n, any);
+  BF_CHECK_LAUNCH();
+  BF_CHECK_HIP(hipStreamSynchronize(st));
+  *any_host = *any;
+  return BF_OK;
+}
 
 extern "C" int bf_node_set_workspace_size(int64_t num_nodes, size_t* bytes) {
   BF_CHECK_ARG(bytes && num_nodes >= 0, "node_set_workspace_size: bad arguments");
@@ -234,6 +261,8 @@ extern "C" int bf_reception_cone(const int64_t* rowptr, const int32_t* col, cons
                    workspace_bytes >= node_space_bytes(num_nodes),
                "reception_cone: workspace %zu < %zu bytes", workspace_bytes, node_space_bytes(num_nodes));
   hipStream_t st = as_stream(stream);
+  BF_HOST_READ(read);
+  auto* count = read.as<uint32_t>();
   const NodeSpace s = node_space(workspace, num_nodes);
   BF_CHECK_OK(clear_nodes(s, num_nodes, st));
   const int64_t work = ceil_div(num_nodes > num_edges ? num_nodes : num_edges, int64_t(kThreads) * 8);
@@ -255,15 +284,13 @@ extern "C" int bf_reception_cone(const int64_t* rowptr, const int32_t* col, cons
             static_cast<const int64_t*>(nullptr), s.counts, static_cast<uint32_t*>(nullptr));
   BF_CHECK_LAUNCH();
   BF_LAUNCH("radix_scan_kernel", sort::radix_scan_kernel, dim3(1), dim3(sort::kThreads), 0, st, s.counts, s.tiles,
-            s.words + 1);
+            count);
   BF_CHECK_LAUNCH();
   BF_LAUNCH("mark_write_kernel", mark_write_kernel<int64_t>, dim3(unsigned(s.tiles)), dim3(kThreads), 0, st, s.level,
             num_nodes, s.counts, ids);
   BF_CHECK_LAUNCH();
-  uint32_t h = 0;
-  BF_CHECK_HIP(hipMemcpyAsync(&h, s.words + 1, sizeof(h), hipMemcpyDeviceToHost, st));
   BF_CHECK_HIP(hipStreamSynchronize(st));
-  *count_host = h;
+  *count_host = *count;
   return BF_OK;
 }
 
@@ -299,8 +326,9 @@ extern "C" int bf_probe_queries(const int64_t* filter, int64_t n_filter, int64_t
               s.words + 3);
     BF_CHECK_LAUNCH();
   }
-  uint32_t h[4];
-  BF_CHECK_HIP(hipMemcpyAsync(h, s.words, sizeof(h), hipMemcpyDeviceToHost, st));
+  BF_HOST_READ(read);
+  auto* h = read.as<uint32_t>();
+  BF_CHECK_HIP(hipMemcpyAsync(h, s.words, 4 * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
   BF_CHECK_HIP(hipStreamSynchronize(st));
   info_host[0] = h[2];   // queries
   info_host[1] = h[1];   // some query has an in-edge

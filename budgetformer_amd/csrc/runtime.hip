@@ -19,6 +19,42 @@ void set_error(const char* fmt, ...) {
 }
 
 namespace {
+// The free pages of HostRead: on the heap and never freed, as the timer's lists below.
+struct HostPages {
+  std::mutex m;
+  std::vector<void*> free;
+};
+HostPages& host_pages() {
+  static auto* p = new HostPages;
+  return *p;
+}
+}  // namespace
+
+HostRead::HostRead() : page_(nullptr) {
+  HostPages& hp = host_pages();
+  {
+    std::lock_guard<std::mutex> lock(hp.m);
+    if (!hp.free.empty()) {
+      page_ = hp.free.back();
+      hp.free.pop_back();
+      return;
+    }
+  }
+  const hipError_t e = hipHostMalloc(&page_, kHostReadBytes, hipHostMallocPortable);
+  if (e != hipSuccess) {
+    page_ = nullptr;
+    set_error("hipHostMalloc failed: %s", hipGetErrorString(e));
+  }
+}
+
+HostRead::~HostRead() {
+  if (!page_) return;
+  HostPages& hp = host_pages();
+  std::lock_guard<std::mutex> lock(hp.m);
+  hp.free.push_back(page_);
+}
+
+namespace {
 
 struct Pending {
   const char* name;

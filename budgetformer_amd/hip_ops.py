@@ -188,11 +188,8 @@ def _coo_holds(row: torch.Tensor, col: torch.Tensor, n_row: int, n_col: int,
                types: Optional[torch.Tensor] = None) -> int:
     """The N.COO_* bits an edge list keeps to (bf_coo_order): one pass over it and one host read."""
     dev = row.device
-    stream = _stream(dev)
-    ws = _workspace(N.COO_ORDER_WORKSPACE, dev)
     holds = C.c_int32(0)
-    N.call("bf_coo_order", _p(row), _p(col), _p(types), row.numel(), n_row, n_col, C.byref(holds), _p(ws), ws.numel(),
-           stream)
+    N.call("bf_coo_order", _p(row), _p(col), _p(types), row.numel(), n_row, n_col, C.byref(holds), _stream(dev))
     return holds.value
 
 
@@ -460,6 +457,14 @@ def probe_queries(dst_filter: torch.Tensor, in_ptr: torch.Tensor, hubs: Optional
     if info[3]:
         return None
     return ids[: info[0]], kept[: info[2]], bool(info[1])
+
+
+def any_nonzero(x: torch.Tensor) -> bool:
+    """Whether ``x`` (int32) holds anything but zeros (bf_any_nonzero: one pass, one host read)."""
+    _require(x, "x", torch.int32)
+    found = C.c_int32(0)
+    N.call("bf_any_nonzero", _p(x), x.numel(), C.byref(found), _stream(x.device))
+    return bool(found.value)
 
 
 def mark_in_neighbors(in_ptr, in_src, frontier: torch.Tensor, reached: torch.Tensor) -> None:

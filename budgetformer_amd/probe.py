@@ -139,7 +139,7 @@ def build_probe(graph: CSRGraph, dst_filter: torch.Tensor, *, max_real: int, max
         sel, cnt = hip_ops.rw_select_rows(graph.rowptr, graph.col, qids, P, L, k, int(edge_seed) + RW_SEED_OFFSET,
                                           u=u, philox_seed=seed, philox_offset=philox_offset, subtract=subtract,
                                           walk_rec=graph.walk_records(), ids_checked=checked)
-        rw_nonempty = bool(cnt.any())
+        rw_nonempty = hip_ops.any_nonzero(cnt)
         if max_rw > 0:
             rw = (sel, cnt)
     return ProbeBuild(graph, qids, real, rw, real_nonempty, rw_nonempty, global_token=global_token)

@@ -274,6 +274,9 @@ int bf_assemble_rows(const int32_t* real_kv, const int32_t* real_cnt, int32_t re
  * Synchronises the stream. Workspace of both: bf_node_set_workspace_size,
  * 16-byte aligned.                                                          */
 int bf_node_set_workspace_size(int64_t num_nodes, size_t* bytes);
+/* *any_host = 1 when an entry of x int32 [n] is not 0, else 0 (whether a walk
+ * pool holds anything, :1797-1812). Synchronises the stream.                */
+int bf_any_nonzero(const int32_t* x, int64_t n, int32_t* any_host, void* stream);
 int bf_reception_cone(const int64_t* rowptr, const int32_t* col, const int64_t* in_ptr, const int32_t* in_src,
                       int64_t num_nodes, int64_t num_edges, const int64_t* probe_ids, int64_t n_probe, int32_t hops,
                       int64_t* ids, int64_t* count_host, void* workspace, size_t workspace_bytes, void* stream);
@@ -381,8 +384,7 @@ int bf_coo_to_csr(const int64_t* src, const int64_t* dst, int64_t nnz, int64_t n
  * when every entry (pair of neighbouring entries) keeps to it. row / col int64
  * [nnz]; type (may be NULL) int64 [nnz] of 0 or 1, a column then being (type,
  * col). The reference's lists come out of coalesce (gt_sp/utils.py:877-887),
- * in (src, dst) order. One pass and one read back: synchronises the stream.
- * Workspace: BF_COO_ORDER_WORKSPACE bytes.                                  */
+ * in (src, dst) order. One pass and one read back: synchronises the stream.   */
 #define BF_COO_IDS 1         /* rows in [0, n_row), columns in [0, n_col)     */
 #define BF_COO_TYPES 2       /* types 0 or 1                                  */
 #define BF_COO_ROW_MAJOR 4   /* ascending by (row, column)                    */
@@ -390,9 +392,8 @@ int bf_coo_to_csr(const int64_t* src, const int64_t* dst, int64_t nnz, int64_t n
 #define BF_COO_STRICT 16     /* strictly ascending by (row, column)           */
 #define BF_COO_BY_COL 32     /* columns never descend                         */
 #define BF_COO_BY_ROW 64     /* rows never descend                            */
-#define BF_COO_ORDER_WORKSPACE 4096
 int bf_coo_order(const int64_t* row, const int64_t* col, const int64_t* type, int64_t nnz, int64_t n_row,
-                 int64_t n_col, int32_t* holds_host, void* workspace, size_t workspace_bytes, void* stream);
+                 int64_t n_col, int32_t* holds_host, void* stream);
 
 /* bf_coo_to_csr for a list of known order: ptr int64 [n_row + 1], ids int32
  * [nnz] ascending within a row (with type: by (type, id), the type in bit 31).
@@ -447,7 +448,7 @@ int bf_coalesce_bidirected(const int64_t* src, const int64_t* dst, int64_t nnz, 
  * [0, width], ids in [0, id_limit): else BF_ERR_INVALID) and returns its entry
  * count; it synchronises the stream. Its workspace
  * (bf_table_list_check_workspace_size) goes to bf_table_to_list as `checked`,
- * which consumes it; out holds total = nnz + token_row + token_col per row.
+ * out holds total = nnz + token_row + token_col per row.
  * Workspace: bf_table_to_list_workspace_size.                               */
 int bf_table_list_check_workspace_size(int64_t n_rows, size_t* bytes);
 int bf_table_list_check(const int32_t* table, const int32_t* row_len, int64_t n_rows, int32_t width,

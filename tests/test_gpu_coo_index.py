@@ -110,14 +110,14 @@ def test_coalesce_and_bidirected(hip_device, nnz, n):
 
 @pytest.mark.parametrize("token", [False, True])
 @pytest.mark.parametrize("how", ["full", "shard", "ids"])
-@pytest.mark.parametrize("n_rows,width", [(1, 1), (511, 3), (513, 8), (5000, 33)])
+@pytest.mark.parametrize("n_rows,width", [(1, 1), (511, 3), (513, 8), (5000, 33), (530_000, 2)])
 def test_table_to_list_equals_the_index_route(hip_device, n_rows, width, how, token):
     """A table's list against its CSR's reverse index (the route it replaces) and fix_edge_index's order; rows empty,
     full and past a block of rows, one row with the multiset's repeated id; bad tables refused."""
     from budgetformer_amd.edges import EdgeTable
     from budgetformer_amd.hip_ops import AttentionIndex
     rng = np.random.default_rng(n_rows + width)
-    n = 6000
+    n = max(6000, n_rows + 800)
     ids = np.sort(np.minimum((n * rng.random((n_rows, width)) ** 3).astype(np.int32), n - 1), axis=1)
     ids[0, -1] = n - 1
     if width > 2:

@@ -157,3 +157,16 @@ def test_probe_refuses_ids_outside_the_graph_and_takes_an_empty_filter(hip_devic
     pb = build_probe(g, torch.zeros(0, dtype=torch.int64, device=hip_device), max_real=4, max_rw=4)
     assert pb.query_ids.numel() == 0 and not pb.real_nonempty and not pb.rw_nonempty
     assert pb.table(4, 4).to_edge_index().shape == (2, 0)
+
+
+@pytest.mark.parametrize("n", [0, 1, 255, 256, 1025, 300_000])
+def test_any_nonzero(hip_device, n):
+    """Nothing, and a single entry at either end: the read-back page is clean on every call."""
+    from budgetformer_amd import hip_ops
+    x = torch.zeros(n, dtype=torch.int32, device=hip_device)
+    assert not hip_ops.any_nonzero(x)
+    for at in {0, n - 1} if n else ():
+        x[at] = -1
+        assert hip_ops.any_nonzero(x)
+        x[at] = 0
+        assert not hip_ops.any_nonzero(x)
