@@ -170,3 +170,26 @@ def test_any_nonzero(hip_device, n):
         assert hip_ops.any_nonzero(x)
         x[at] = 0
         assert not hip_ops.any_nonzero(x)
+
+
+@pytest.mark.parametrize("dedup", [False, True])
+@pytest.mark.parametrize("b_real,b_rw", [(1, 0), (0, 1), (8, 8), (9, 7), (16, 1), (17, 15), (20, 13), (31, 33), (40, 25)])
+def test_assemble_rows_by_width(hip_device, b_real, b_rw, dedup):
+    """Merged rows on both sides of 16, 32 and 64 entries (a row's lanes, then the LDS form), with repeats within and
+    across the parts, empty and full rows, and a last block that is not full; whole numbers, so no tolerance."""
+    from budgetformer_amd import hip_ops
+    rng = np.random.default_rng(b_real * 100 + b_rw)
+    n = 77
+    sel = [rng.integers(0, 30, (n, b + 2)).astype(np.int32) for b in (b_real, b_rw)]
+    cnt = [rng.integers(0, b + 3, n).astype(np.int32) for b in (b_real, b_rw)]
+    for x, b in zip(cnt, (b_real, b_rw)):
+        x[0], x[-1] = 0, b + 2
+    sel[0][3, 0] = sel[1][3, 0] = 2 ** 31 - 1
+    parts = [(torch.from_numpy(s).to(hip_device), torch.from_numpy(c).to(hip_device)) if b else None
+             for s, c, b in zip(sel, cnt, (b_real, b_rw))]
+    table, row_len = (t.cpu().numpy() for t in hip_ops.assemble_rows(*parts, b_real, b_rw, dedup=dedup))
+    for r in range(n):
+        row = np.concatenate([s[r, :min(c[r], b)] for s, c, b in zip(sel, cnt, (b_real, b_rw))])
+        row = np.unique(row) if dedup else np.sort(row)
+        assert row_len[r] == row.size and np.array_equal(table[r], np.pad(row, (0, table.shape[1] - row.size),
+                                                                         constant_values=-1))
