@@ -864,8 +864,10 @@ class SplitPlan:
 
     @property
     def pending(self) -> bool:
-        """Whether the host does not have the counts (yet): a pinned copy that has landed is read, without waiting."""
-        if self._items < 0 and self.ready is not None and self.ready.query():
+        """Whether the host does not have the counts (yet): a pinned copy that has landed is read, without waiting.
+        A capturing stream may not ask whether it has: the plan then stays pending."""
+        if self._items < 0 and self.ready is not None and not torch.cuda.is_current_stream_capturing() \
+                and self.ready.query():
             self._read()
         return self._items < 0
 

@@ -75,3 +75,45 @@ def test_attention_layer_graph_replays_equal_eager(hip_device, dtype):
         torch.cuda.synchronize(hip_device)
         for name, a, b in zip(("out", "dq", "dk", "dv"), replayed, eager):
             assert torch.equal(a, b), f"replay {rep}: {name} differs from the eager call"
+
+
+def test_layer_captured_while_plan_counts_are_pending(hip_device):
+    """A default index whose plan counts have not been taken from their pinned copy when the capture starts (the
+    layers before it went ahead of the copy): the capture asks no event and launches for the capacities, and every
+    replay equals the eager calls, which take the counts."""
+    from budgetformer_amd.graph import CSRGraph, chung_lu_csr
+    from budgetformer_amd.edges import build_attention_edges
+    from budgetformer_amd.hip_ops import AttentionIndex, attn_backward, attn_forward
+    n, H, hn = 3000, 8, 16
+    rowptr, col = chung_lu_csr(n, 30000, seed=9)
+    g = CSRGraph.from_csr(rowptr, col, n, device=hip_device)
+    tab = build_attention_edges(g, real_edges_per_query=4, rw_edges_per_query=4, walk_length=4,
+                                walks_per_node=2, edge_seed=3, global_token=True)
+    idx = tab.attention_index(chunk=16, item=40)
+    idx.ensure_backward(True)
+    gen = torch.Generator().manual_seed(6)
+    base = [torch.randn(n + 1, H, hn, generator=gen) for _ in range(4)]
+    q, k, v, dout = (t.to(hip_device) for t in base)
+
+    def layer(idx=idx):
+        out, Z = attn_forward(idx, q, k, v)
+        return (out,) + attn_backward(idx, q, k, v, None, Z, dout)[:3]
+
+    layer(AttentionIndex.from_table(tab.table, tab.row_len, True, n_kv=n + 1, chunk=16, item=40, check=False,
+                                    token_row=n))  # another index: the kernels are loaded before the capture
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        assert idx.kplan.ready is not None and idx.kplan.pending
+        captured = layer()
+        assert idx.kplan.ready is not None         # not read inside the capture
+    torch.cuda.synchronize(hip_device)
+    assert not idx.kplan.pending and idx.kplan.heavy > 0        # the copy is read once the capture is over
+    for scale in (1.0, 0.6, 1.4):
+        q.copy_(base[0].to(hip_device) * scale)
+        graph.replay()
+        torch.cuda.synchronize(hip_device)
+        replayed = [t.clone() for t in captured]
+        eager = layer()
+        torch.cuda.synchronize(hip_device)
+        for name, a, b in zip(("out", "dq", "dk", "dv"), replayed, eager):
+            assert torch.equal(a, b), f"scale {scale}: {name} differs from the eager call"
