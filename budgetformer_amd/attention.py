@@ -58,9 +58,9 @@ class _SparseEdgeAttention(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dout, _dZ):
-        if dout is None:
-            return (None,) * 8
         q, k, v, Z, bias_e, factor_e = ctx.saved_tensors
+        if dout is None:                         # a later function gave out no gradient: zeros for the inputs
+            dout = torch.zeros_like(q)
         dq, dk, dv, dbias = hip_ops.attn_backward(ctx.index, q, k, v, None, Z, dout.contiguous(), bias_e, factor_e,
                                                   need_dbias=ctx.need_dbias, dropout=ctx.dropout,
                                                   score_clamp=ctx.score_clamp, keep=ctx.keep)

@@ -203,3 +203,26 @@ def test_index_operators_equal_the_single_calls(hip_device, n, width, token_row,
         heavy = idx.kplan.heavy_rows[:plan.heavy]
         assert torch.equal(heavy.sort().values, plan.heavy_rows[:plan.heavy].sort().values)
         assert torch.equal(idx.kplan.nitems[heavy.long()], plan.nitems[heavy.long()])
+
+
+def test_layer_without_an_output_gradient_gives_zeros(hip_device):
+    """A function after the layer that hands no gradient back (None): the layer's inputs get zeros, not None."""
+    from budgetformer_amd.attention import sparse_edge_attention
+    from budgetformer_amd.hip_ops import AttentionIndex
+
+    class NoGradient(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x):
+            return x.sum()
+
+        @staticmethod
+        def backward(ctx, grad):
+            return None
+
+    gen = torch.Generator().manual_seed(3)
+    ei = torch.randint(0, 50, (2, 400), generator=gen)
+    x = [torch.randn(50, 8, 16, generator=gen).to(hip_device).requires_grad_(True) for _ in range(3)]
+    out = sparse_edge_attention(*x, AttentionIndex.from_coo(ei.to(hip_device), 50, 50))
+    grads = torch.autograd.grad(NoGradient.apply(out), x)
+    for g, t in zip(grads, x):
+        assert torch.equal(g, torch.zeros_like(t))
