@@ -114,12 +114,12 @@ def build_probe(graph: CSRGraph, dst_filter: torch.Tensor, *, max_real: int, max
     """
     dev = graph.device
     ids = dst_filter.to(dev).view(-1).to(torch.int64).contiguous()
-    all_hubs = graph.hubs(hub_threshold) if use_real and max_real > 0 else None
-    found = hip_ops.probe_queries(ids, graph.in_ptr, all_hubs)
+    all_hubs = graph.hubs(hub_threshold) if use_real and max_real > 0 and graph.num_nodes else None
+    found = hip_ops.probe_queries(ids, graph.in_ptr, all_hubs) if graph.num_nodes else None
     checked = found is not None
     if checked:
         qids, hubs, has_edges = found
-    else:                       # an id outside the graph: the ranking calls refuse it
+    else:                       # an id outside the graph (or a graph of no nodes): the ranking calls refuse it
         qids, hubs, has_edges = torch.unique(ids).to(torch.int32), None, False
     n = qids.numel()
     P = max(int(walks_per_node), 1)

@@ -159,6 +159,16 @@ def test_probe_refuses_ids_outside_the_graph_and_takes_an_empty_filter(hip_devic
     assert pb.table(4, 4).to_edge_index().shape == (2, 0)
 
 
+def test_probe_of_a_graph_of_no_nodes_is_empty(hip_device):
+    from budgetformer_amd.graph import CSRGraph
+    from budgetformer_amd.probe import build_probe
+    ptr = torch.zeros(1, dtype=torch.int64, device=hip_device)
+    ids = torch.zeros(0, dtype=torch.int32, device=hip_device)
+    pb = build_probe(CSRGraph(ptr, ids, ptr, ids, 0), torch.zeros(0, dtype=torch.int64, device=hip_device), max_real=4,
+                     max_rw=4)
+    assert pb.query_ids.numel() == 0 and not pb.real_nonempty and not pb.rw_nonempty
+
+
 @pytest.mark.parametrize("n", [0, 1, 255, 256, 1025, 300_000])
 def test_any_nonzero(hip_device, n):
     """Nothing, and a single entry at either end: the read-back page is clean on every call."""
