@@ -8,6 +8,7 @@ stream. PyTorch is used only for device memory and streams.
 from __future__ import annotations
 
 import ctypes as C
+import threading
 import weakref
 from dataclasses import dataclass, field
 from typing import Optional
@@ -824,6 +825,9 @@ def row_order_and_plan(ptr: torch.Tensor, nnz: int, threshold: int, item_size: i
     return order, spans, plan
 
 
+_PLAN_READ = threading.Lock()     # of the plans' pinned counts
+
+
 @dataclass
 class SplitPlan:
     """Rows longer than `threshold` cut into `item_size`-entry items.
@@ -845,10 +849,14 @@ class SplitPlan:
     _slot: Optional[object] = field(default=None, repr=False)   # returns the pinned slot to its pool
 
     def _read(self) -> None:
-        self.ready.synchronize()
-        self._items, self._heavy = (int(x) for x in self.host_counts.tolist())
-        self.counts = self.host_counts = self.ready = None
-        self._slot()               # the slot goes back to the pool (the finalizer runs once)
+        with _PLAN_READ:           # layers of several threads may share an index: one of them reads
+            if self.ready is None:
+                return
+            self.ready.synchronize()
+            items, self._heavy = (int(x) for x in self.host_counts.tolist())
+            self._items = items    # last: a count above -1 says that both are there
+            self.counts = self.host_counts = self.ready = None
+            self._slot()           # the slot goes back to the pool (the finalizer runs once)
 
     @property
     def items(self) -> int:
@@ -866,8 +874,8 @@ class SplitPlan:
     def pending(self) -> bool:
         """Whether the host does not have the counts (yet): a pinned copy that has landed is read, without waiting.
         A capturing stream may not ask whether it has: the plan then stays pending."""
-        if self._items < 0 and self.ready is not None and not torch.cuda.is_current_stream_capturing() \
-                and self.ready.query():
+        ready = self.ready
+        if self._items < 0 and ready is not None and not torch.cuda.is_current_stream_capturing() and ready.query():
             self._read()
         return self._items < 0
 
