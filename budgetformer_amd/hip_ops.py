@@ -38,8 +38,12 @@ def _stream(device: torch.device):
     device of its tensors, so a host tensor is refused here, before any pointer reaches a kernel."""
     if device.type != "cuda":
         raise ValueError(f"the HIP path takes device tensors (got tensors on {device}); it has no CPU fallback")
-    idx = device.index if device.index is not None else torch.cuda.current_device()
-    return C.c_void_p(torch._C._cuda_getCurrentRawStream(idx))
+    return C.c_void_p(_raw_stream(device))
+
+
+def _raw_stream(device: torch.device) -> int:
+    return torch._C._cuda_getCurrentRawStream(device.index if device.index is not None
+                                              else torch.cuda.current_device())
 
 
 def _require(t: torch.Tensor, name: str, dtype: torch.dtype, device: torch.device = None):
@@ -1058,6 +1062,7 @@ class AttentionIndex:
     _rkeys: Optional[ReverseKeys] = field(default=None, repr=False)   # from_table: sort keys, until used
     _sorted: Optional[ReverseKeys] = field(default=None, repr=False)  # sorted keys, until ks is needed
     _coo_keys: Optional[tuple] = field(default=None, repr=False)      # from a COO list: coo_reverse's keys, until used
+    _key_stream: Optional[int] = field(default=None, repr=False)      # raw stream the keys above were allocated on
     _counts: Optional[torch.Tensor] = field(default=None, repr=False)  # both plans' device counts
     # True: the plans leave their counts on the device and the attention calls size their grids for the
     # capacities (no host read at all between building the index and using it, e.g. for a caller that
@@ -1152,13 +1157,15 @@ class AttentionIndex:
                         _copy_counts_to_host(self.kplan, self.device)
                 else:
                     self.kptr, self.kq_all, ks, srt = reverse_index_packed(rk, self.qptr, self.n_kv, entries=entries)
+                self._spend(rk.keys)
                 if entries:
                     self.ks_all = ks
                 else:
-                    self._sorted = srt
+                    self._sorted, self._key_stream = srt, _raw_stream(self.device)
                 self._rkeys = None
             elif self._coo_keys is not None:
                 self.kptr, self.kq_all = coo_reverse(self._coo_keys, self.n_q, self.n_kv, self.typed)
+                self._spend(self._coo_keys[0])
                 self._coo_keys = None
                 if entries:
                     self.ks_all = coo_reverse_slots(self.qptr, self.kv_all, self.kptr, self.kq_all)
@@ -1187,8 +1194,16 @@ class AttentionIndex:
                 self.ks_all = coo_reverse_slots(self.qptr, self.kv_all, self.kptr, self.kq_all)
             else:
                 self.ks_all = reverse_slots(self._sorted, self.qptr)
+                self._spend(self._sorted.keys)
                 self._sorted = None
         return self
+
+    def _spend(self, keys: torch.Tensor) -> None:
+        """``keys`` go after the launches just made. A layer may make them on another stream than the one that built
+        the index, whose next allocation could take the keys' memory while they are still read: the allocator then
+        waits for the reading stream. (Everything else of an index lives as long as the index.)"""
+        if _raw_stream(keys.device) != self._key_stream:
+            keys.record_stream(torch.cuda.current_stream(keys.device))
 
     def entry_rows(self) -> torch.Tensor:
         """Query id of every CSR entry (int64), for per-edge bias gathers."""
@@ -1329,7 +1344,8 @@ class AttentionIndex:
             idx.qptr, idx.kv_all, keys, *plan = N.load_ops().table_index(
                 table, row_len, bool(global_token), tr, bound, n_rows * width, q_bits, slot_bits, known[0], chunk,
                 item, counts)
-            idx._rkeys = ReverseKeys(keys, q_bits, slot_bits, bool(global_token), tr)
+            idx._rkeys, idx._key_stream = (ReverseKeys(keys, q_bits, slot_bits, bool(global_token), tr),
+                                           _raw_stream(table.device))
             idx.qplan = _plan_of(plan, known, counts[:2], bound, chunk, item)
             return idx
         idx.qptr = qptr = table_qptr(table, row_len, global_token, tr)
@@ -1341,6 +1357,7 @@ class AttentionIndex:
         # grids exactly (a B=32 table fills well under half of its capacity).
         qptr, idx.kv_all, idx._rkeys = table_to_csr(table, row_len, global_token, with_keys=True, qptr=qptr,
                                                     token_row=tr, exact=exact)
+        idx._key_stream = _raw_stream(table.device)
         if exact:
             idx._nnz = idx.kv_all.numel()
         return idx
@@ -1371,7 +1388,7 @@ class AttentionIndex:
             types = (both >= n_kv).to(torch.int64)
             qptr, kv, keys = coo_rows_to_csr(dst, both - types * n_kv, n_q, n_kv, types, with_keys=True)
         idx = cls(n_q=n_q, n_kv=n_kv, qptr=qptr, kv_all=kv, chunk=chunk, item=item, _nnz=kv.numel(), typed=True,
-                  _coo_keys=keys)
+                  _coo_keys=keys, _key_stream=_raw_stream(kv.device))
         # no split query rows: a plan of none
         idx.qplan = split_plan_first_row(n_q, 0, kv.numel(), kv.numel() + 1, item, idx._plan_counts(0))
         idx.ensure_backward()
@@ -1385,7 +1402,8 @@ class AttentionIndex:
             raise ValueError(f"edge_index must be [2, E] (got {tuple(edge_index.shape)})")
         src, dst = _pair_lists(edge_index)
         qptr, kv, keys = coo_rows_to_csr(dst, src, n_q, n_kv, with_keys=True)
-        return cls(n_q=n_q, n_kv=n_kv, qptr=qptr, kv_all=kv, chunk=chunk, item=item, _nnz=kv.numel(), _coo_keys=keys)
+        return cls(n_q=n_q, n_kv=n_kv, qptr=qptr, kv_all=kv, chunk=chunk, item=item, _nnz=kv.numel(), _coo_keys=keys,
+                   _key_stream=_raw_stream(kv.device))
 
 
 # ------------------------------------------------------------------ attention
