@@ -314,7 +314,8 @@ __device__ __forceinline__ uint32_t list_lengths(const int32_t* __restrict__ row
   return bad;
 }
 
-__device__ __forceinline__ uint32_t block_sum(uint32_t v, uint32_t* wave /*[kThreads / 64]*/) {
+// Lengths and counts are added up in 64 bits: a block of very wide rows holds more than 2^32 entries.
+__device__ __forceinline__ uint64_t block_sum(uint64_t v, uint64_t* wave /*[kThreads / 64]*/) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   __syncthreads();                       // an earlier sum's words are read
@@ -327,15 +328,16 @@ template <typename I>   // of a slot within the block: 32 bits unless the rows a
 __global__ __launch_bounds__(kThreads) void table_list_check_kernel(const int32_t* __restrict__ table,
                                                                     const int32_t* __restrict__ row_len,
                                                                     int64_t n_rows, int width, int64_t id_limit,
-                                                                    uint32_t* __restrict__ sums,
-                                                                    uint32_t* __restrict__ bad) {
+                                                                    uint64_t* __restrict__ sums,
+                                                                    uint64_t* __restrict__ bad) {
   __shared__ int32_t len[kListRows];
-  __shared__ uint32_t wave[kThreads / 64];
+  __shared__ uint64_t wave[kThreads / 64];
   const uint32_t bad_len = list_lengths(row_len, n_rows, width, len);
   __syncthreads();
-  uint32_t total = 0, bad_id = 0;
+  uint64_t total = 0;
+  uint32_t bad_id = 0;         // of a thread: at most 2 * width slots
 #pragma unroll
-  for (int u = 0; u < kListRows / kThreads; ++u) total += uint32_t(len[u * kThreads + threadIdx.x]);
+  for (int u = 0; u < kListRows / kThreads; ++u) total += uint64_t(len[u * kThreads + threadIdx.x]);
   const int64_t r0 = int64_t(blockIdx.x) * kListRows;
   const int rows = int(n_rows - r0 < kListRows ? n_rows - r0 : kListRows);
   const I slots = I(rows) * I(width);
@@ -352,54 +354,53 @@ __global__ __launch_bounds__(kThreads) void table_list_check_kernel(const int32_
       bad_id += (int32_t(c) < len[r] && (id[u] < 0 || int64_t(id[u]) >= id_limit)) ? 1u : 0u;
     }
   }
-  const uint32_t s = block_sum(total, wave), bl = block_sum(bad_len, wave), bi = block_sum(bad_id, wave);
+  const uint64_t s = block_sum(total, wave), bl = block_sum(bad_len, wave), bi = block_sum(bad_id, wave);
   if (threadIdx.x == 0) {
-    sums[blockIdx.x] = s;                  // a list of 2^31 entries or more is refused on the host
+    sums[blockIdx.x] = s;
     bad[2 * int64_t(blockIdx.x)] = bl;
     bad[2 * int64_t(blockIdx.x) + 1] = bi;
   }
 }
 
-// The blocks' sums become their first places; out (pinned host memory) gets the entries, the bad lengths and the bad
-// ids. One workgroup, and the host reads 24 bytes: copying the blocks' words (54 KB in two arrays for 2.3M rows) to
-// add them up there takes 52 us, a kernel's own store of the sums 11.5 us, launch and wait included in both.
+// The blocks' sums become their first places (32 bits: a list of 2^31 entries or more is refused by the host, which
+// gets the 64-bit total); out (pinned host memory) gets the entries, the bad lengths and the bad ids. One workgroup,
+// and the host reads 24 bytes: copying the blocks' words (54 KB in two arrays for 2.3M rows) to add them up there
+// takes 52 us, a kernel's own store of the sums 11.5 us, launch and wait included in both.
 constexpr int kTotalsThreads = 1024;
-__global__ __launch_bounds__(kTotalsThreads) void list_totals_kernel(uint32_t* __restrict__ sums,
-                                                                     const uint32_t* __restrict__ bad, int64_t blocks,
+__global__ __launch_bounds__(kTotalsThreads) void list_totals_kernel(uint64_t* __restrict__ sums,
+                                                                     const uint64_t* __restrict__ bad, int64_t blocks,
                                                                      uint64_t* __restrict__ out) {
   __shared__ uint32_t tmp[kTotalsThreads / 64];
-  __shared__ uint64_t all_bad[2];
-  if (threadIdx.x < 2) all_bad[threadIdx.x] = 0;
+  __shared__ uint64_t all[3];
+  if (threadIdx.x < 3) all[threadIdx.x] = 0;
   __syncthreads();
-  uint64_t total = 0;          // the places wrap from 2^32 entries on, which the host refuses
-  uint64_t bad_len = 0, bad_id = 0;
+  uint32_t base_at = 0;        // the places wrap from 2^32 entries on; the total does not
+  uint64_t mine[3] = {0, 0, 0};
   for (int64_t base = 0; base < blocks; base += kTotalsThreads) {
     const int64_t b = base + threadIdx.x;
-    const uint32_t v = b < blocks ? sums[b] : 0;
+    const uint64_t v = b < blocks ? sums[b] : 0;
     if (b < blocks) {
-      bad_len += bad[2 * b];
-      bad_id += bad[2 * b + 1];
+      mine[0] += v;
+      mine[1] += bad[2 * b];
+      mine[2] += bad[2 * b + 1];
     }
     uint32_t tot;
-    const uint32_t e = sort::block_excl_scan<kTotalsThreads>(v, tmp, &tot);
-    if (b < blocks) sums[b] = uint32_t(total) + e;
-    total += tot;
+    const uint32_t e = sort::block_excl_scan<kTotalsThreads>(uint32_t(v), tmp, &tot);
+    if (b < blocks) sums[b] = base_at + e;
+    base_at += tot;
   }
-  if (bad_len) atomicAdd(reinterpret_cast<unsigned long long*>(&all_bad[0]), (unsigned long long)bad_len);
-  if (bad_id) atomicAdd(reinterpret_cast<unsigned long long*>(&all_bad[1]), (unsigned long long)bad_id);
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+    if (mine[i]) atomicAdd(reinterpret_cast<unsigned long long*>(&all[i]), (unsigned long long)mine[i]);
   __syncthreads();
-  if (threadIdx.x == 0) {
-    out[0] = total;
-    out[1] = all_bad[0];
-    out[2] = all_bad[1];
-  }
+  if (threadIdx.x < 3) out[threadIdx.x] = all[threadIdx.x];
 }
 
 template <typename I>   // of a slot within the block: 32 bits unless the rows are very wide
 __global__ __launch_bounds__(kThreads) void table_list_keys_kernel(const int32_t* __restrict__ table,
                                                                    const int32_t* __restrict__ row_len,
                                                                    int64_t n_rows, int width,
-                                                                   const uint32_t* __restrict__ prefix, int qb,
+                                                                   const uint64_t* __restrict__ prefix, int qb,
                                                                    uint64_t* __restrict__ keys) {
   __shared__ int32_t len[kListRows];
   __shared__ uint32_t off[kListRows];
@@ -410,7 +411,7 @@ __global__ __launch_bounds__(kThreads) void table_list_keys_kernel(const int32_t
   uint32_t mine = 0, total;
 #pragma unroll
   for (int u = 0; u < kRows; ++u) mine += uint32_t(len[threadIdx.x * kRows + u]);
-  uint32_t at = sort::block_excl_scan<kThreads>(mine, tmp, &total) + prefix[blockIdx.x];
+  uint32_t at = sort::block_excl_scan<kThreads>(mine, tmp, &total) + uint32_t(prefix[blockIdx.x]);
 #pragma unroll
   for (int u = 0; u < kRows; ++u) {
     off[threadIdx.x * kRows + u] = at;
@@ -692,12 +693,12 @@ extern "C" int bf_coalesce_bidirected(const int64_t* src, const int64_t* dst, in
 
 namespace {
 int64_t list_blocks(int64_t n_rows) { return ceil_div(n_rows, int64_t(kListRows)); }
-size_t list_sums_bytes(int64_t n_rows) { return align_up(size_t(list_blocks(n_rows)) * 4 + 4); }
+size_t list_sums_bytes(int64_t n_rows) { return align_up(size_t(list_blocks(n_rows)) * 8 + 8); }
 }  // namespace
 
 extern "C" int bf_table_list_check_workspace_size(int64_t n_rows, size_t* bytes) {
   BF_CHECK_ARG(bytes && n_rows >= 0, "table_list_check_workspace_size: bad arguments");
-  *bytes = list_sums_bytes(n_rows) + align_up(size_t(list_blocks(n_rows)) * 8) + 256;
+  *bytes = list_sums_bytes(n_rows) + align_up(size_t(list_blocks(n_rows)) * 16) + 256;
   return BF_OK;
 }
 
@@ -715,8 +716,8 @@ extern "C" int bf_table_list_check(const int32_t* table, const int32_t* row_len,
                need);
   hipStream_t st = as_stream(stream);
   const int64_t blocks = list_blocks(n_rows);
-  auto* sums = static_cast<uint32_t*>(workspace);
-  auto* bad = reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) + list_sums_bytes(n_rows));
+  auto* sums = static_cast<uint64_t*>(workspace);
+  auto* bad = reinterpret_cast<uint64_t*>(static_cast<char*>(workspace) + list_sums_bytes(n_rows));
   if (width <= kListWidth32)
     BF_LAUNCH("table_list_check_kernel", table_list_check_kernel<uint32_t>, dim3(unsigned(blocks)), dim3(kThreads), 0,
               st, table, row_len, n_rows, width, id_limit, sums, bad);
@@ -769,7 +770,7 @@ extern "C" int bf_table_to_list(const int32_t* table, const int32_t* row_len, in
     auto* keys = ws.take<uint64_t>(size_t(nnz) * 8);
     sorted = ws.take<uint64_t>(size_t(nnz) * 8);
     const int64_t blocks = list_blocks(n_rows);
-    const auto* sums = static_cast<const uint32_t*>(checked);    // the blocks' first places
+    const auto* sums = static_cast<const uint64_t*>(checked);    // the blocks' first places
     if (width <= kListWidth32)
       BF_LAUNCH("table_list_keys_kernel", table_list_keys_kernel<uint32_t>, dim3(unsigned(blocks)), dim3(kThreads), 0,
                 st, table, row_len, n_rows, width, sums, qb, keys);

@@ -146,6 +146,24 @@ def test_table_to_list_equals_the_index_route(hip_device, n_rows, width, how, to
         EdgeTable(table, lens, n).to_edge_index()
 
 
+def test_table_of_two_to_the_32_entries_is_refused(hip_device):
+    """1024 blocks of rows whose lengths add up to 2^32 exactly (0 in 32 bits): refused for its size, and for its ids
+    where those are bad as well. 17 GB of table, no list is written."""
+    from budgetformer_amd.edges import EdgeTable
+    if torch.cuda.mem_get_info(hip_device)[0] < 40 * 2 ** 30:
+        pytest.skip("needs 17 GB for the table")
+    n_rows, width = 1024 * 512, 8192
+    table = torch.zeros(n_rows, width, dtype=torch.int32, device=hip_device)
+    lens = torch.full((n_rows,), width, dtype=torch.int32, device=hip_device)
+    with pytest.raises(ValueError, match=f"{n_rows * width} entries"):
+        EdgeTable(table, lens, 5).to_edge_index()
+    table.fill_(-1)
+    with pytest.raises(ValueError, match=f"{n_rows * width} table ids outside"):
+        EdgeTable(table, lens, 5).to_edge_index()
+    del table
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("n_rows", [1, 63, 4095, 4096, 4097, 70_000])
 @pytest.mark.parametrize("threshold,item,share", [(8, 3, 0.01), (1, 1, 1.0), (1000, 768, 0.0)])
 def test_split_plan_at_block_edges(hip_device, n_rows, threshold, item, share):
