@@ -26,6 +26,7 @@
 // 210M keys: 697 -> 370 us, sort 4.63 -> 4.33 ms).
 #pragma once
 
+#include <algorithm>
 #include <cstdint>
 
 #include "bf_common.h"
@@ -52,6 +53,27 @@ constexpr int kThreads = 256;   // of the scan kernel
 constexpr int kMinRadix = 6, kMaxRadix = 10;
 constexpr float kPassCost[kMaxRadix + 1] = {0, 0, 0, 0, 0, 0, 0.90f, 0.92f, 1.0f, 1.13f, 1.27f};
 
+// The sizes past which make_plan takes larger tiles. Just past one the tiles, and with them the counts' array, are
+// half as many: a plan's workspace does not grow steadily with n (workspace_bytes_max).
+constexpr int64_t kTileSteps[] = {int64_t(1) << 16, int64_t(1) << 21, int64_t(1) << 22, int64_t(1) << 24,
+                                  int64_t(1) << 26};
+
+struct Tile {
+  int threads, items;
+  int64_t count(int64_t n) const {
+    const int64_t keys = int64_t(threads) * items;
+    return (n + keys - 1) / keys;
+  }
+};
+
+inline Tile tile_for(int64_t n, int radix) {
+  if (n <= kTileSteps[0] && radix <= 8) return {256, 4};
+  if (n <= kTileSteps[1]) return {512, 4};
+  if (n <= kTileSteps[radix == 10 ? 2 : 3]) return {512, 8};
+  if (radix == 10) return {512, 16};
+  return {256, radix == 9 && n > kTileSteps[4] ? 32 : 16};
+}
+
 struct Plan {
   int radix;
   int threads;
@@ -75,19 +97,10 @@ inline Plan make_plan(int64_t n, int bits) {
       p.radix = radix;
     }
   }
-  if (n <= (int64_t(1) << 16) && p.radix <= 8) {
-    p.threads = 256, p.items = 4;
-  } else if (n <= (int64_t(1) << 21)) {
-    p.threads = 512, p.items = 4;
-  } else if (n <= (int64_t(1) << (p.radix == 10 ? 22 : 24))) {
-    p.threads = 512, p.items = 8;
-  } else if (p.radix == 10) {
-    p.threads = 512, p.items = 16;
-  } else {
-    p.threads = 256, p.items = p.radix == 9 && n > (int64_t(1) << 26) ? 32 : 16;
-  }
-  const int64_t tile = int64_t(p.threads) * p.items;
-  p.tiles = (n + tile - 1) / tile;
+  const Tile t = tile_for(n, p.radix);
+  p.threads = t.threads;
+  p.items = t.items;
+  p.tiles = t.count(n);
   return p;
 }
 
@@ -101,22 +114,30 @@ __device__ __forceinline__ int64_t live_count(int64_t cap, const int64_t* n_dev,
   return n < 0 ? 0 : (n > cap ? cap : n);
 }
 
-// Workspace of make_plan(n, bits): the second key buffer, the per-tile counts and the digit totals.
-inline size_t workspace_bytes(int64_t n, int bits) {
-  const Plan p = make_plan(n, bits);
-  const size_t digits = size_t(1) << p.radix;
-  return align256(size_t(n > 0 ? n : 1) * 8) + align256(size_t(p.tiles > 0 ? p.tiles : 1) * digits * 4) +
+// The second key buffer, the per-tile counts and the digit totals.
+inline size_t buffer_bytes(int64_t n, int radix, int64_t tiles) {
+  const size_t digits = size_t(1) << radix;
+  return align256(size_t(n > 0 ? n : 1) * 8) + align256(size_t(tiles > 0 ? tiles : 1) * digits * 4) +
          align256(digits * 4);
 }
 
-// The most any bit count needs for n keys.
+// Workspace of make_plan(n, bits).
+inline size_t workspace_bytes(int64_t n, int bits) {
+  const Plan p = make_plan(n, bits);
+  return buffer_bytes(n, p.radix, p.tiles);
+}
+
+// The most that any sort of up to n keys needs, by any bits: a caller that knows its keys only within a capacity
+// (an index's entries less the token's) sizes its workspace so.
 inline size_t workspace_bytes_max(int64_t n) {
-  size_t m = 0;
-  for (int bits = 1; bits <= 64; ++bits) {
-    const size_t b = workspace_bytes(n, bits);
-    if (b > m) m = b;
+  size_t most = 0;
+  for (int radix = kMinRadix; radix <= kMaxRadix; ++radix) {
+    const auto at = [&](int64_t m) { most = std::max(most, buffer_bytes(m, radix, tile_for(m, radix).count(m))); };
+    at(n);
+    for (const int64_t step : kTileSteps)
+      if (step < n) at(step);
   }
-  return m;
+  return most;
 }
 
 // block-wide exclusive scan of one value per thread; *total gets the sum

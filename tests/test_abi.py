@@ -241,3 +241,21 @@ def test_struct_mirrors_match_the_header(tmp_path, struct, mirror):
     subprocess.run([cc, "-I", os.path.dirname(N._HEADER), str(src), "-o", str(exe)], check=True)
     got = [int(x) for x in subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split()]
     assert got == [C.sizeof(cls)] + [getattr(cls, f).offset for f in names]
+
+
+def test_reverse_index_workspace_holds_every_smaller_sort():
+    """bf_reverse_index_packed sorts an index's entries less the token's own: its workspace, sized by the entries,
+    holds the sort of any smaller count by any bits. Sorts take larger tiles past 2^16, 2^21, 2^22, 2^24 and 2^26
+    keys, and just below one of these need more than just past it."""
+    def size(name, *args):
+        out = C.c_size_t(0)
+        N.call(name, *args, C.byref(out))
+        return out.value
+
+    steps = [1 << 16, 1 << 21, 1 << 22, 1 << 24, 1 << 26]
+    counts = sorted({1, 1000, 2_097_152 + 131_072, 2_000_000_000} | {s + d for s in steps for d in (-1, 0, 1, s // 20)})
+    for nnz in counts:
+        have = size("bf_reverse_index_packed_workspace_size", nnz)
+        for m in [m for m in counts if m <= nnz]:
+            for bits in range(1, 64):
+                assert have >= size("bf_radix_sort_workspace_size", m, 0, bits), (nnz, m, bits)

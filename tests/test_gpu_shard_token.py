@@ -122,3 +122,20 @@ def test_shard_attention_equals_full_rows_and_oracle(hip_device, dtype, cuts):
     # the shards' key-side gradients add up to the full build's
     assert_close("sum dk", dk_sum, f_dk, tol)
     assert_close("sum dv", dv_sum, f_dv, tol)
+
+
+@pytest.mark.parametrize("n_rows,width,times", [(131_072, 16, 4), (65_536, 32, 4), (208_000, 10, 2)])
+def test_shard_index_where_keys_and_entries_straddle_a_sort_size(hip_device, n_rows, width, times):
+    """A shard without the token row whose reverse index sorts at most 2^21 keys of more than 2^21 entries (the
+    token column's are not sorted): the sort of the keys takes more workspace than one of the entries would. The
+    index equals the one from (qptr, kv)."""
+    from budgetformer_amd import hip_ops
+    n = n_rows * times
+    assert n_rows * width <= 2 ** 21 < n_rows * (width + 1)
+    rng = np.random.default_rng(width)
+    ids = np.sort((n * rng.random((n_rows, width)) ** 2).astype(np.int32), axis=1)
+    lens = torch.from_numpy(rng.integers(0, width + 1, n_rows).astype(np.int32)).to(hip_device)
+    idx = hip_ops.AttentionIndex.from_table(torch.from_numpy(ids).to(hip_device), lens, True, n_kv=n + 1,
+                                            check=False, token_row=-1).ensure_backward(entries=True)
+    kptr, kq, ks = hip_ops.reverse_index(idx.qptr, idx.kv, n + 1)
+    assert torch.equal(idx.kptr, kptr) and torch.equal(idx.kq, kq) and torch.equal(idx.ks, ks)
