@@ -538,18 +538,19 @@ struct RowPick {
   int64_t row, beg, end;   // row >= n_q: none
 };
 
-// The query row of this lane's group. deal (deal_rows): the workgroup's rows (kBlock / lanes per row consecutive
-// ones) go to its groups longest first, so that the groups of a wave walk rows of about one length. A wave runs
-// until its longest row ends; with rows in id order the lanes of the shorter ones idled (2.9M rows of 128 bf16 with
-// dropout, 0 to 32 entries, 11 on average, four rows to a wave: forward 2.72 -> 2.29 ms, dq pass 2.40 -> 2.13).
-// Each wave ranks the rows by itself, from one load of their row pointers. Split rows (longer than `chunk`) rank
-// last: their groups leave at once.
+// The query row of this lane's group. deal (deal_rows; an instance with DEAL can): the workgroup's rows (kBlock /
+// lanes per row consecutive ones) go to its groups longest first, so that the groups of a wave walk rows of about one
+// length. A wave runs until its longest row ends; with rows in id order the lanes of the shorter ones idled (2.9M rows
+// of 128 bf16 with dropout, 0 to 32 entries, 11 on average, four rows to a wave: forward 2.72 -> 2.29 ms, dq pass
+// 2.40 -> 2.13). Each wave ranks the rows by itself, from one load of their row pointers. Split rows (longer than
+// `chunk`) rank last: their groups leave at once. What a row computes does not depend on the group that takes it.
+template <bool DEAL>
 __device__ __forceinline__ RowPick pick_row(const Shape& sh, unsigned first_block, const int64_t* __restrict__ qptr,
                                             int64_t n_q, int chunk, int deal) {
   const int gpb = kBlock >> sh.lpr_log2;
   const int64_t r0 = int64_t(blockIdx.x - first_block) * gpb;
   const int grp = threadIdx.x >> sh.lpr_log2;
-  if (!deal) {
+  if (!DEAL || !deal) {
     const int64_t row = r0 + grp;
     return row < n_q ? RowPick{row, qptr[row], qptr[row + 1]} : RowPick{row, 0, 0};
   }
@@ -705,7 +706,7 @@ struct FwdWaves<float, 0> {
 };
 
 // Blocks [0, n_items) take the query-side items, the rest one short query row per group.
-template <typename T, int EX>
+template <typename T, int EX, bool DEAL>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(FwdWaves<T, EX>::kMin))) void attn_fwd_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
     const int64_t* __restrict__ qptr, const int32_t* __restrict__ kv, EdgeIn ex,
@@ -736,7 +737,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(FwdWaves
     }
     return;
   }
-  const RowPick pick = pick_row(sh, unsigned(n_items_arg), qptr, n_q, chunk, deal);
+  const RowPick pick = pick_row<DEAL>(sh, unsigned(n_items_arg), qptr, n_q, chunk, deal);
   const int64_t row = pick.row, beg = pick.beg, end = pick.end;
   if (row >= n_q) return;
   if (end - beg > chunk) return;  // split row: its items and the reduce write it
@@ -999,7 +1000,7 @@ __device__ __forceinline__ void sum_token_records(const float* __restrict__ rec0
 // With a token column (rows from tok_first on open with key 0) every workgroup also writes one
 // record of its rows' key-0 terms; a split row's key-0 terms are finished with the row: by its item
 // when the row has one, else by the dq reduce, which writes them into the row's first item's record.
-template <typename T, int EX>
+template <typename T, int EX, bool DEAL>
 __global__ __launch_bounds__(kBlock) void attn_bwd_q_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
     const int64_t* __restrict__ qptr, const int32_t* __restrict__ kv, EdgeIn ex,
@@ -1045,7 +1046,7 @@ __global__ __launch_bounds__(kBlock) void attn_bwd_q_kernel(
     if (token_rec && grp == 0) store_token_record<V>(token_rec + int64_t(blockIdx.x) * (2 * sh.D), sh, g, fk, fv);
     return;
   }
-  const RowPick pick = pick_row(sh, unsigned(n_items_arg), qptr, n_q, chunk, deal);
+  const RowPick pick = pick_row<DEAL>(sh, unsigned(n_items_arg), qptr, n_q, chunk, deal);
   const int64_t row = pick.row, end = pick.end;
   int64_t beg = pick.beg;
   const bool live = row < n_q && end - beg <= chunk;    // a split row: its items and the reduce write it
@@ -1868,13 +1869,21 @@ inline unsigned grid_for(int64_t rows, const Shape& sh) {
   return unsigned(ceil_div(rows, per_block));
 }
 
-// Whether the query passes deal a workgroup's rows out by length (pick_row): where a wave holds four rows or more
-// (with two the ranking costs what it spares: 169K nodes, float32 rows of 128, step 659 -> 663 us), ranks them all
-// (at most 64 to a workgroup) and they are long enough to differ by iterations: more than 10 entries a row by the
-// index's entry count, which is its capacity for a small table (rows of a budget of 8 and the token's entries end
-// within three iterations: 411K rows of 64 fp16, forward 97.5 -> 98.0 us with the ranking).
+// Whether a query pass deals a workgroup's rows out by length (pick_row): groups of 16 lanes from 16 entries a row
+// on, of 8 from 24 on, by nnz, which a table's index gives for its rows full: shorter rows differ by too little.
+// The passes that call it and their shares of the time without it (80K and 600K rows, by width / mean entries):
+//   dropout forward  16 lanes (bf16)  32/11 0.87 0.84, 24/12 0.93 0.92, 16/6 0.94 0.93, 16/13 1.03 1.01, 12/7 1.03 0.99
+//                     8 lanes (fp16)  32/11 0.89 0.83, 24/12 0.97 0.93, 16/6 0.97 0.96, 16/13 1.08 1.02, 12/7 1.09 1.06
+//   dropout dq       16 lanes         32/11 0.89 0.88, 24/12 0.95 0.97, 16/6 0.95 0.97, 16/13 1.05 1.02, 12/7 1.04 1.02
+//                     8 lanes         32/11 0.87 0.87, 24/12 0.97 0.99, 16/6 0.98 1.00, 16/13 1.08 1.02, 12/7 1.07 1.05
+//   dq, no token     16 lanes         32/11 0.90 0.91, 24/12 0.97 0.98, 16/6 0.97 0.98, 16/13 1.04 1.00, 12/7 1.04 1.02
+//   column            8 lanes         32/11 0.90 0.91, 24/12 0.99 1.01, 16/6 1.00 1.01, 16/13 1.08 1.02, 12/7 1.06 1.04
+// The plain forward, the lightest, has its line at 32 (16 lanes 32/11 0.97 0.99, 24/12 1.01 1.01, 16/13 1.01 1.01;
+// 8 lanes 0.92 0.99, 1.02 1.02, 1.03 1.01), without a token column (1.00 1.00 at 32/11). Never dealt are the dq pass
+// with a token column (0.98 to 1.05), groups of 4 lanes, which rank 64 rows (1.03 to 1.32), and of 32, two to a wave
+// (169K nodes, float32 rows of 128: step 659 -> 663 us).
 inline int deal_rows(const bf_attn_index* idx, const Shape& sh) {
-  return sh.lpr_log2 <= 4 && (kBlock >> sh.lpr_log2) <= 64 && idx->nnz > 10 * idx->n_q ? 1 : 0;
+  return (sh.lpr_log2 == 4 && idx->nnz >= 16 * idx->n_q) || (sh.lpr_log2 == 3 && idx->nnz >= 24 * idx->n_q);
 }
 
 inline size_t combine_lds_bytes(const Shape& sh) {
@@ -1945,10 +1954,10 @@ int fwd_impl(const bf_attn_index* idx, const Shape& sh, const void* q, const voi
   const int64_t blocks = int64_t(n_items) + grid_for(idx->n_q, sh);
   if (blocks > 0) {
     const size_t lds = n_items > 0 ? combine_lds_bytes(sh) : 0;
-#define BF_LAUNCH_FWD(EX)                                                                                        \
-  BF_LAUNCH("attn_fwd_kernel", (attn_fwd_kernel<T, EX>), dim3(unsigned(blocks)), dim3(kBlock), lds, st, Q, K, Vv,  \
-            idx->qptr, idx->kv, ex, O, Z, it, n_items, idx->n_q, sh, idx->chunk, deal_rows(idx, sh),                           \
-            idx->plan_counts)
+#define BF_LAUNCH_FWD(EX, DEAL)                                                                                   \
+  BF_LAUNCH("attn_fwd_kernel", (attn_fwd_kernel<T, EX, DEAL>), dim3(unsigned(blocks)), dim3(kBlock), lds, st, Q, K, \
+            Vv, idx->qptr, idx->kv, ex, O, Z, it, n_items, idx->n_q, sh, idx->chunk,                                \
+            DEAL ? deal_rows(idx, sh) : 0, idx->plan_counts)
     // the dropout-only instance stores the keep mask a window at a time, for one byte per entry (H <= 8)
     // and groups wide enough to share an iteration's draws; other shapes (more heads; H <= 3 with one lane
     // per head) take the general instance, which stores it too
@@ -1956,14 +1965,20 @@ int fwd_impl(const bf_attn_index* idx, const Shape& sh, const void* q, const voi
     switch (edge_mode(ex, false)) {
       case 4:
         if (shared_draws && ex.kbytes == 1) {
-          BF_LAUNCH_FWD(4);
+          BF_LAUNCH_FWD(4, true);
         } else {
-          BF_LAUNCH_FWD(2);
+          BF_LAUNCH_FWD(2, false);
         }
         break;
-      case 2: BF_LAUNCH_FWD(2); break;
-      case 1: BF_LAUNCH_FWD(1); break;
-      default: BF_LAUNCH_FWD(0); break;
+      case 2: BF_LAUNCH_FWD(2, false); break;
+      case 1: BF_LAUNCH_FWD(1, true); break;
+      default:
+        if (deal_rows(idx, sh) && !idx->token_column && idx->nnz >= 32 * idx->n_q) {
+          BF_LAUNCH_FWD(0, true);
+        } else {
+          BF_LAUNCH_FWD(0, false);
+        }
+        break;
     }
 #undef BF_LAUNCH_FWD
     BF_CHECK_LAUNCH();
@@ -2058,22 +2073,30 @@ int bwd_impl(const bf_attn_index* idx, const Shape& sh, const void* q, const voi
                          : nullptr;
   if (q_blocks > 0) {
     const size_t lds = (idx->q_items > 0 || token_rec) ? combine_lds_bytes(sh) : 0;
-#define BF_LAUNCH_Q(EX)                                                                                          \
-  BF_LAUNCH("attn_bwd_q_kernel", (attn_bwd_q_kernel<T, EX>), dim3(unsigned(q_blocks)), dim3(kBlock), lds, st, Q, K, \
-            Vv, idx->qptr, idx->kv, ex, Z, dO, static_cast<T*>(dq), dbias, rstat, qit, idx->q_items,                \
-            idx->n_q, sh, idx->chunk, deal_rows(idx, sh), token_rec, tok_first, idx->plan_counts)
+#define BF_LAUNCH_Q(EX, DEAL)                                                                                    \
+  BF_LAUNCH("attn_bwd_q_kernel", (attn_bwd_q_kernel<T, EX, DEAL>), dim3(unsigned(q_blocks)), dim3(kBlock), lds, st, \
+            Q, K, Vv, idx->qptr, idx->kv, ex, Z, dO, static_cast<T*>(dq), dbias, rstat, qit, idx->q_items,          \
+            idx->n_q, sh, idx->chunk, deal, token_rec, tok_first, idx->plan_counts)
+    // not with a token column: its terms are summed over a workgroup's groups, in an order that the dealing changes
+    const int deal = token_rec ? 0 : deal_rows(idx, sh);
     // the mask is read back where an entry's bits fill one byte (H <= 8); wider rows of heads draw
     switch (edge_mode(ex, dbias != nullptr)) {
       case 4:
         if (ex.kbytes == 1) {
-          BF_LAUNCH_Q(4);
+          BF_LAUNCH_Q(4, true);
         } else {
-          BF_LAUNCH_Q(1);
+          BF_LAUNCH_Q(1, true);
         }
         break;
-      case 2: BF_LAUNCH_Q(2); break;
-      case 1: BF_LAUNCH_Q(1); break;
-      default: BF_LAUNCH_Q(0); break;
+      case 2: BF_LAUNCH_Q(2, false); break;
+      case 1: BF_LAUNCH_Q(1, true); break;
+      default:
+        if (deal) {
+          BF_LAUNCH_Q(0, true);
+        } else {
+          BF_LAUNCH_Q(0, false);   // the flag costs the 16-bit pass up to 1% (80K rows)
+        }
+        break;
     }
 #undef BF_LAUNCH_Q
     BF_CHECK_LAUNCH();

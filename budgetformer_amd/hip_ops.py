@@ -1075,6 +1075,7 @@ class AttentionIndex:
     _q_known: Optional[tuple] = field(default=None, repr=False)
     _structs: dict = field(default_factory=dict, repr=False)          # C view per (backward, with ks)
     _nnz: Optional[int] = field(default=None, repr=False)             # qptr[n_q], once read
+    _full: Optional[int] = field(default=None, repr=False)            # a table's entries with every row full
 
     @property
     def cap(self) -> int:
@@ -1238,7 +1239,7 @@ class AttentionIndex:
         cached = self._structs.get(key)
         if cached is not None:
             return cached
-        s = self._make_struct(backward)
+        s = self._make_struct(backward, self.nnz_known)
         self._structs[key] = s
         return s
 
@@ -1247,13 +1248,15 @@ class AttentionIndex:
                       "k_nitems", "k_item_off", "k_item_row", "k_heavy_rows", "k_order", "k_spans", "plan_counts")
     _INT_FIELDS = ("n_q", "n_kv", "nnz", "chunk", "item", "q_items", "q_heavy", "k_items", "k_heavy", "token_column")
 
-    def _fields(self, backward: bool):
-        """bf_attn_index's fields: ({pointer field: tensor or None}, {integer field: int})."""
+    def _fields(self, backward: bool, count: bool):
+        """bf_attn_index's fields: ({pointer field: tensor or None}, {integer field: int}); nnz is the entry count
+        with ``count``, else what the rows could hold."""
         t = dict.fromkeys(self._TENSOR_FIELDS)
         n = dict.fromkeys(self._INT_FIELDS, 0)
-        # the kernels take the entries from the row pointers; nnz sizes only the per-edge tensors (bias,
-        # factor, dbias), whose calls read it first, and otherwise passes the capacity
-        n["n_q"], n["n_kv"], n["nnz"] = self.n_q, self.n_kv, self.nnz if self.nnz_known else self.cap
+        # the kernels take the entries from the row pointers; nnz sizes the per-edge tensors (bias, factor,
+        # dbias) and says how long rows are to the rule that deals them out (calls without such tensors only)
+        full = self.cap if self._full is None or not self.cap else min(self._full, 2 ** 31 - 1)
+        n["n_q"], n["n_kv"], n["nnz"] = self.n_q, self.n_kv, self.nnz if count else full
         t["qptr"], t["kv"] = self.qptr, self.kv_all if self.cap else None
         n["chunk"], n["item"] = self.chunk, self.item
         qp = self.qplan
@@ -1277,8 +1280,8 @@ class AttentionIndex:
         n["token_column"] = int(self.token_column)
         return t, n
 
-    def _make_struct(self, backward: bool) -> N.AttnIndex:
-        t, n = self._fields(backward)
+    def _make_struct(self, backward: bool, count: bool) -> N.AttnIndex:
+        t, n = self._fields(backward, count)
         s = N.AttnIndex()
         for name, tensor in t.items():
             setattr(s, name, tensor.data_ptr() if tensor is not None else None)
@@ -1286,16 +1289,21 @@ class AttentionIndex:
             setattr(s, name, value)
         return s
 
-    def op_args(self, backward: bool, entries: bool = False):
+    def op_args(self, backward: bool, entries: bool = False, per_edge: Optional[bool] = None):
         """The index as the torch operators take it: ([16 tensors or None], [10 ints]), in the order of
-        bf_attn_index's fields (``_TENSOR_FIELDS``, ``_INT_FIELDS``); cached like ``struct``."""
+        bf_attn_index's fields (``_TENSOR_FIELDS``, ``_INT_FIELDS``); cached like ``struct``. ``per_edge``: whether
+        the call has [nnz, H] tensors and needs the entry count; without them it passes the entries of a table's
+        full rows (a list's own count), known from the build on, so that the kernels a call takes do not depend on
+        what was asked of the index before (None: the count where it is known, for callers with such tensors of
+        their own)."""
         self.ensure_backward(entries) if backward else self.ensure_forward()
         if backward and entries:
             self.ensure_entries()
-        key = ("op", backward, backward and self.ks_all is not None, self.nnz_known, self._plans_on_device(backward))
+        count = self.nnz_known if per_edge is None else per_edge
+        key = ("op", backward, backward and self.ks_all is not None, count, self._plans_on_device(backward))
         cached = self._structs.get(key)
         if cached is None:
-            t, n = self._fields(backward)
+            t, n = self._fields(backward, count)
             cached = ([t[f] for f in self._TENSOR_FIELDS], [int(n[f]) for f in self._INT_FIELDS])
             self._structs[key] = cached
         return cached
@@ -1338,7 +1346,7 @@ class AttentionIndex:
         # key 0 is then attended by every query row from 1 on (with the token row) or from 0 on (without)
         token_column = 0 if not global_token else (1 if tr >= 0 else 2)
         idx = cls(n_q=n_q_tab, n_kv=n_kv, qptr=None, kv_all=None, chunk=chunk, item=item,
-                  token_column=token_column, _q_known=known)
+                  token_column=token_column, _q_known=known, _full=bound)
         if fused:
             counts = idx._counts = torch.empty(4, dtype=torch.int32, device=table.device)
             idx.qptr, idx.kv_all, keys, *plan = N.load_ops().table_index(
@@ -1456,9 +1464,8 @@ def attn_forward(idx: AttentionIndex, q, k, v, bias=None, factor=None, dropout: 
     q.k / sqrt(hn), in (0, 5]. With ``keep_mask`` also returns the dropout's keep mask (uint8
     [kv capacity, ceil(H/8)], empty without a dropout) for ``attn_backward(keep=...)``, whose dq pass then
     reads the bits instead of drawing them again (the same bits: results equal bit for bit)."""
-    if bias is not None or factor is not None:
-        idx.nnz      # per-edge tensors are [nnz, H]: the index passes the count itself
-    t, n = idx.op_args(backward=False)
+    # per-edge tensors are [nnz, H]: the index then passes the count itself
+    t, n = idx.op_args(backward=False, per_edge=bias is not None or factor is not None)
     out, Z, keep = N.load_ops().sparse_attn_fwd(q, k, v, t, n, bias, factor, *_dropout_op_args(dropout),
                                                 float(score_clamp), bool(keep_mask))
     return (out, Z, keep) if keep_mask else (out, Z)
@@ -1501,9 +1508,8 @@ def attn_backward(idx: AttentionIndex, q, k, v, out, Z, dout, bias=None, factor=
     rate, seed, off = _dropout_op_args(dropout)
     if not 0.0 <= rate <= 1.0:
         raise ValueError(f"dropout rate {rate} outside [0, 1]")
-    if bias is not None or factor is not None or need_dbias:
-        idx.nnz      # per-edge tensors are [nnz, H]: the index passes the count itself
-    t, n = idx.op_args(backward=True, entries=bias is not None or factor is not None or need_dbias or rate > 0.0)
+    per_edge = bias is not None or factor is not None or need_dbias     # [nnz, H]: the index passes the count itself
+    t, n = idx.op_args(backward=True, entries=per_edge or rate > 0.0, per_edge=per_edge)
     dq, dk, dv, dbias = N.load_ops().sparse_attn_bwd(q, k, v, t, n, Z, dout, bias, factor, bool(need_dbias), rate,
                                                      seed, off, float(score_clamp), keep)
     return dq, dk, dv, (dbias if need_dbias else None)

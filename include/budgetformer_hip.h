@@ -576,7 +576,9 @@ int bf_row_order_and_plan(const int64_t* ptr, int64_t n_rows, int32_t threshold,
 typedef struct bf_attn_index {
   int64_t n_q;                  /* queries (rows of qptr)                          */
   int64_t n_kv;                 /* key/value rows                                   */
-  int64_t nnz;                  /* edges                                            */
+  int64_t nnz;                  /* edges: the count where the call has per-edge tensors
+                                   (bias, factor, dbias); else it may be any bound of
+                                   it below 2^31, and says how long rows may be        */
   const int64_t* qptr;          /* [n_q+1]                                          */
   const int32_t* kv;            /* [nnz]   kv id per edge, query-major              */
   const int64_t* kptr;          /* [n_kv+1] reverse offsets (backward only)         */

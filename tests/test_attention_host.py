@@ -76,3 +76,29 @@ def test_host_tensors_are_refused_before_any_library_call():
         hip_ops.expand_rows(torch.tensor([0, 1, 2]), 2)
     with pytest.raises(ValueError, match="no CPU fallback"):
         chung_lu_device(100, 400, device="cpu")
+
+
+@pytest.mark.parametrize("per_edge", [False, True])
+def test_a_call_passes_the_same_sizes_before_and_after_the_entry_count_is_read(monkeypatch, per_edge):
+    """The launches are chosen by the integers a call passes: without per-edge tensors the capacity, with them the
+    count, whatever was read before."""
+    from budgetformer_amd import _native as N
+    from budgetformer_amd import hip_ops
+    empty = torch.empty(0, dtype=torch.int32)
+    plan = hip_ops.SplitPlan(0, 0, empty, empty, empty, empty)
+    idx = hip_ops.AttentionIndex(n_q=3, n_kv=4, qptr=torch.tensor([0, 2, 2, 5]),
+                                 kv_all=torch.zeros(12, dtype=torch.int32), qplan=plan, kplan=plan,
+                                 kptr=torch.tensor([0, 5, 5, 5, 5]), kq_all=torch.zeros(12, dtype=torch.int32),
+                                 ks_all=torch.zeros(12, dtype=torch.int32), korder=empty)
+    seen = []
+    ops = types.SimpleNamespace(sparse_attn_fwd=lambda q, k, v, t, n, *a: (seen.append(n), (q, q, q))[1],
+                                sparse_attn_bwd=lambda q, k, v, t, n, *a: (seen.append(n), (q, q, q, q))[1])
+    monkeypatch.setattr(N, "load_ops", lambda: ops)
+    x = torch.zeros(3, 2, 4)
+    bias = torch.zeros(5, 2) if per_edge else None
+    for _ in range(2):
+        hip_ops.attn_forward(idx, x, x, x, bias=bias)
+        hip_ops.attn_backward(idx, x, x, x, None, x, x, bias=bias)
+        assert idx.nnz == 5
+    nnz = hip_ops.AttentionIndex._INT_FIELDS.index("nnz")
+    assert [n[nnz] for n in seen] == [5 if per_edge else 12] * 4

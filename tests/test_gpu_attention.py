@@ -6,6 +6,7 @@ the larger of max|got - ref| / max|ref| per tensor and the same per row with eac
 scale floored at 0.1 x the tensor's (parity_helpers; the newer tests floor bf16 rows at
 1e-3).
 """
+import numpy as np
 import pytest
 import torch
 
@@ -514,9 +515,9 @@ def test_query_passes_past_16m_rows_equal_the_compact_problem(hip_device):
                                         (torch.float32, 4, 8), (torch.float32, 8, 16)])
 @pytest.mark.parametrize("n", [1, 33, 1000])
 def test_rows_dealt_by_length(hip_device, dtype, H, hn, n):
-    """Rows of 0 to 40 entries, more than 10 on average, so that a workgroup's rows go to its groups by length (all
-    shapes but float32 rows of 128, which keep id order): a partial last workgroup, empty rows, split rows among the
-    short ones (chunk 36), against the float64 oracle."""
+    """Rows of 0 to 40 entries, 20 on average, so that the dq pass gives a workgroup's rows to its groups by length
+    where a row takes 16 lanes (bf16 rows of 128; the plain forward and other shapes keep id order): a partial last
+    workgroup, empty rows, split rows among the short ones (chunk 36), against the float64 oracle."""
     g = torch.Generator().manual_seed(n + H * hn)
     lens = torch.randint(0, 41, (n,), generator=g)
     lens[n // 2] = 40
@@ -540,3 +541,70 @@ def test_rows_dealt_by_length(hip_device, dtype, H, hn, n):
     for name, got, ref in (("out", out, ro[:n]), ("dq", qd.grad, rdq[:n]), ("dk", kd.grad, rdk[:500]),
                            ("dv", vd.grad, rdv[:500])):
         assert_close(name, got.detach(), ref, tol)
+
+
+@pytest.mark.parametrize("drop", [None, "drawn", "kept"])
+@pytest.mark.parametrize("dtype,H,hn", [(torch.bfloat16, 8, 16), (torch.float16, 8, 8), (torch.float32, 8, 8),
+                                        (torch.float32, 4, 8), (torch.float32, 8, 16), (torch.bfloat16, 4, 8)])
+def test_dealt_rows_equal_rows_in_id_order(hip_device, dtype, H, hn, drop):
+    """Rows of 0 to 70 entries (split from 65 on), dealt by length in the passes that deal (8 and 16 lanes to a row),
+    against the same rows in an index with so many empty rows behind them
+    that none does: a row's results do not depend on it."""
+    from budgetformer_amd.hip_ops import AttentionIndex, Dropout, attn_backward, attn_forward
+    n, n_kv = 1003, 500
+    g = torch.Generator().manual_seed(H * hn)
+    lens = torch.randint(0, 71, (n,), generator=g)
+    rows = torch.repeat_interleave(torch.arange(n), lens)
+    ei = torch.stack([torch.randint(0, n_kv, (rows.numel(),), generator=g), rows]).to(hip_device)
+    q, dout = (torch.randn(5 * n, H, hn, generator=g).to(dtype).to(hip_device) for _ in range(2))
+    k, v = (torch.randn(n_kv, H, hn, generator=g).to(dtype).to(hip_device) for _ in range(2))
+    d = None if drop is None else Dropout(0.4, 11)
+    res = []
+    for n_q in (n, 5 * n):
+        idx = AttentionIndex.from_coo(ei, n_q, n_kv, chunk=64)
+        assert idx.nnz >= 32 * n_q if n_q == n else idx.nnz < 16 * n_q
+        out, Z, keep = attn_forward(idx, q[:n_q], k, v, dropout=d, keep_mask=True)
+        res.append((out[:n], Z[:n]) + attn_backward(idx, q[:n_q], k, v, None, Z, dout[:n_q], dropout=d,
+                                                    keep=keep if drop == "kept" else None)[:3])
+    for name, a, b in zip(("out", "Z", "dq", "dk", "dv"), *res):
+        assert torch.equal(a[:n], b[:n]), name
+
+
+@pytest.mark.parametrize("drop", [False, True])
+@pytest.mark.parametrize("chunk", [128, 12])
+def test_reading_the_entry_count_changes_no_result(hip_device, chunk, drop):
+    """A table index with the token column, 18 entries a row with every row full and about 7 by its count: the same
+    layer before and after the count is read is the same bit for bit, and the oracle's."""
+    from budgetformer_amd.hip_ops import AttentionIndex, Dropout, attn_backward, attn_forward
+    from oracle import philox
+    from parity_helpers import assert_close
+    n, width, H, hn = 2003, 16, 8, 16
+    rng = np.random.default_rng(4)
+    ids = np.stack([np.sort(rng.choice(n, width, replace=False)) for _ in range(n)]).astype(np.int32)
+    lens = np.minimum(rng.integers(0, 17, n), rng.integers(0, 17, n)).astype(np.int32)
+    idx = AttentionIndex.from_table(torch.from_numpy(ids).to(hip_device), torch.from_numpy(lens).to(hip_device), True,
+                                    n_kv=n + 1, chunk=chunk, check=False)
+    g = torch.Generator().manual_seed(9)
+    base = [torch.randn(n + 1, H, hn, generator=g).to(torch.bfloat16) for _ in range(4)]
+    q, k, v, dout = (t.to(hip_device) for t in base)
+    d = Dropout(0.3, 5) if drop else None
+
+    def layer():
+        out, Z, keep = attn_forward(idx, q, k, v, dropout=d, keep_mask=True)
+        return (out,) + attn_backward(idx, q, k, v, None, Z, dout, dropout=d, keep=keep if drop else None)[:3]
+
+    before = layer()
+    assert not idx.nnz_known and idx.cap > 16 * idx.n_q and idx.nnz < 10 * idx.n_q
+    after = layer()
+    for name, a, b in zip(("out", "dq", "dk", "dv"), before, after):
+        assert torch.equal(a, b), name
+    ei = torch.stack([idx.kv.cpu().long(), idx.entry_rows().cpu()])
+    f64 = None
+    if drop:
+        keep = philox.dropout_keep_csr(idx.qptr.cpu().numpy(), H, d.rate, seed=d.seed)
+        f64 = torch.from_numpy(keep).double() / (1.0 - d.rate)
+    q64, k64, v64, d64 = (t.double() for t in base)
+    ro, rZ = sa.attention_forward_stats(k64, q64, v64, ei, None, f64)
+    ref = sa.attention_backward_closed_form(k64, q64, v64, ei, ro, rZ, d64, None, f64)
+    for name, a, r in zip(("out", "dq", "dk", "dv"), after, (ro,) + tuple(ref[:3])):
+        assert_close(name, a, r, 2e-2)
