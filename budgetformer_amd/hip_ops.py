@@ -1014,7 +1014,10 @@ def split_plan(ptr: torch.Tensor, nnz: int, threshold: int = DEFAULT_CHUNK, item
 
 
 # ------------------------------------------------------------------ attention index
-DEVICE_PLAN_MAX_ITEMS = 1 << 14      # plans of up to this many items (at capacity) need no host copy of their counts
+# Plans of up to this many items (at capacity) need no host copy of their counts. The line bounds the records that a
+# call at capacity makes room for (2 D + H floats an item: 17 MB here at D = 128), not the time: a step on a new index
+# is faster without the wait on both sides of it (15K items 655 -> 634 us, 27K 1205 -> 1182, 76K 1718 -> 1693).
+DEVICE_PLAN_MAX_ITEMS = 1 << 14
 NO_READBACK_MAX_ENTRIES = 1 << 23   # tables of up to this many entries (at capacity) build without a host read
 
 
@@ -1025,6 +1028,16 @@ def _to_cap(t: torch.Tensor, cap: int) -> torch.Tensor:
     out = torch.empty(max(cap, 1), dtype=t.dtype, device=t.device)[:cap]
     out[:t.numel()] = t
     return out
+
+
+def _on_device(plan: Optional[SplitPlan]) -> bool:
+    """Whether a call must take the plan's counts from the device (AttentionIndex._plans_on_device)."""
+    if plan is None or plan._items >= 0:
+        return False
+    if plan.item_cap > DEVICE_PLAN_MAX_ITEMS and plan.ready is not None \
+            and not torch.cuda.is_current_stream_capturing():
+        plan.items                 # waits
+    return plan.pending
 
 
 @dataclass
@@ -1222,13 +1235,9 @@ class AttentionIndex:
         """Which of the plans a call uses keep their counts on the device. A plan's pinned copy is waited for only
         where the capacities would cost the launches more than the wait costs the stream: in a first layer on a new
         index the host is ahead of the copy, and waiting for it left the GPU idle until the host had caught up
-        (169K nodes: step 662 -> 630 us). Later layers find the copy landed and pass the counts."""
-        out = []
-        for p in (self.qplan, self.kplan if backward else None):
-            if p is not None and p.item_cap > DEVICE_PLAN_MAX_ITEMS and p.ready is not None:
-                p.items                # waits
-            out.append(p is not None and p.pending)
-        return tuple(out)
+        (169K nodes: step 662 -> 630 us). Later layers find the copy landed and pass the counts. A capturing stream
+        neither waits nor asks: the graph launches for the capacities."""
+        return _on_device(self.qplan), _on_device(self.kplan) if backward else False
 
     def struct(self, backward: bool, entries: bool = False) -> N.AttnIndex:
         self.ensure_backward(entries) if backward else self.ensure_forward()
