@@ -7,6 +7,7 @@
 #include <stdarg.h>
 
 #include "../../include/budgetformer_hip.h"
+#include "host_read.h"
 
 namespace bf {
 
@@ -40,29 +41,18 @@ void set_error(const char* fmt, ...);
     if (_rc != BF_OK) return _rc; \
   } while (0)
 
-// Pinned host memory of kHostReadBytes for the numbers an entry point reads back before it returns: kernels store
-// them there themselves, or an asynchronous copy does. A 24-byte read takes 11.5 us so, launch and wait included,
-// against 15 us by a copy to pinned memory and 22.6 us by one to ordinary memory (a further bounce in the runtime).
-// A page is held for the scope (its entry point synchronises the stream before it leaves) and goes back to a list
-// that later calls of any thread take from: there are as many pages as calls were ever in flight at once.
-constexpr size_t kHostReadBytes = 4096;
-class HostRead {
- public:
-  HostRead();
-  ~HostRead();
-  HostRead(const HostRead&) = delete;
-  HostRead& operator=(const HostRead&) = delete;
-  template <typename T>
-  T* as() const {
-    return static_cast<T*>(page_);
-  }
-  bool ok() const { return page_ != nullptr; }
-
- private:
-  void* page_;
+// A call's page of pinned host memory (host_read.h): BF_HOST_READ(name, stream), then name.as<T>() for the kernels
+// and name.wait() before it is read.
+struct HipPages {
+  using Stream = hipStream_t;
+  using Status = hipError_t;
+  static constexpr hipError_t kDone = hipSuccess;
+  static bool alloc(void** page);
+  static void release(void* page);
+  static hipError_t wait(hipStream_t st);
 };
-#define BF_HOST_READ(name)    \
-  const ::bf::HostRead name;  \
+#define BF_HOST_READ(name, st)              \
+  ::bf::PinnedRead<::bf::HipPages> name(st); \
   if (!name.ok()) return BF_ERR_HIP
 
 // Optional per-kernel timing (bf_prof_enable): an event pair around each launch.

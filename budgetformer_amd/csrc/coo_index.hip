@@ -492,15 +492,15 @@ extern "C" int bf_coo_order(const int64_t* row, const int64_t* col, const int64_
   if (nnz == 0) return BF_OK;
   BF_CHECK_ARG(row && col, "coo_order: null tensor");
   static_assert(kHostReadBytes >= kOrderBlocks * sizeof(uint32_t), "one word per block");
-  BF_HOST_READ(read);
   hipStream_t st = as_stream(stream);
+  BF_HOST_READ(read, st);
   const int64_t want = ceil_div(nnz, int64_t(kThreads) * 4);
   const int64_t blocks = want < kOrderBlocks ? want : kOrderBlocks;
   auto* words = read.as<uint32_t>();
   BF_LAUNCH("coo_order_kernel", coo_order_kernel, dim3(unsigned(blocks)), dim3(kThreads), 0, st, row, col, type, nnz,
             n_row, n_col, words);
   BF_CHECK_LAUNCH();
-  BF_CHECK_HIP(hipStreamSynchronize(st));
+  BF_CHECK_HIP(read.wait());
   uint32_t broken = 0;
   for (int64_t b = 0; b < blocks; ++b) broken |= words[b];
   *holds_host = kAll & ~int32_t(broken);
@@ -647,7 +647,7 @@ int coalesce_list(const PairKeys& in, int64_t total, int64_t num_nodes, int64_t*
   Carve ws{static_cast<char*>(workspace)};
   auto* keys = ws.take<uint64_t>(size_t(total) * 8);
   auto* counts = ws.take<uint32_t>(size_t(tiles) * 4);
-  BF_HOST_READ(read);
+  BF_HOST_READ(read, st);
   auto* count = read.as<uint32_t>();
   const int end_bit = bits_for(uint64_t(num_nodes) * uint64_t(num_nodes));
   BF_CHECK_OK(sort::radix_sort(in, keys, total, 0, end_bit, ws.p,
@@ -660,7 +660,7 @@ int coalesce_list(const PairKeys& in, int64_t total, int64_t num_nodes, int64_t*
   BF_LAUNCH("unique_write_kernel", unique_write_kernel, dim3(unsigned(tiles)), dim3(kThreads), 0, st, keys, total,
             counts, uint64_t(num_nodes), out_src, out_dst);
   BF_CHECK_LAUNCH();
-  BF_CHECK_HIP(hipStreamSynchronize(st));
+  BF_CHECK_HIP(read.wait());
   *count_host = *count;
   return BF_OK;
 }
@@ -725,11 +725,11 @@ extern "C" int bf_table_list_check(const int32_t* table, const int32_t* row_len,
     BF_LAUNCH("table_list_check_kernel", table_list_check_kernel<uint64_t>, dim3(unsigned(blocks)), dim3(kThreads), 0,
               st, table, row_len, n_rows, width, id_limit, sums, bad);
   BF_CHECK_LAUNCH();
-  BF_HOST_READ(read);
+  BF_HOST_READ(read, st);
   auto* h = read.as<uint64_t>();
   BF_LAUNCH("list_totals_kernel", list_totals_kernel, dim3(1), dim3(kTotalsThreads), 0, st, sums, bad, blocks, h);
   BF_CHECK_LAUNCH();
-  BF_CHECK_HIP(hipStreamSynchronize(st));
+  BF_CHECK_HIP(read.wait());
   const int64_t nnz = int64_t(h[0]), bad_len = int64_t(h[1]), bad_id = int64_t(h[2]);
   BF_CHECK_ARG(bad_len == 0, "check_table: %lld row lengths outside [0, %d]", (long long)bad_len, width);
   BF_CHECK_ARG(bad_id == 0, "check_table: %lld table ids outside [0, %lld)", (long long)bad_id, (long long)id_limit);

@@ -781,10 +781,10 @@ extern "C" int bf_table_csr_ptr(const int32_t* row_len, int64_t n_rows, int32_t 
     BF_CHECK_HIP(prim::inclusive_sum(temp, temp_bytes, static_cast<const int64_t*>(lens), qptr + 1, n_q, st));
   }
   if (!nnz_host) return BF_OK;   // the caller reads qptr[n_q] itself, when it needs it
-  BF_HOST_READ(read);
+  BF_HOST_READ(read, st);
   auto* h = read.as<int64_t>();
   BF_CHECK_HIP(hipMemcpyAsync(h, qptr + n_q, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  BF_CHECK_HIP(hipStreamSynchronize(st));
+  BF_CHECK_HIP(read.wait());
   *nnz_host = *h;
   return BF_OK;
 }
@@ -807,10 +807,10 @@ extern "C" int bf_check_table(const int32_t* table, const int32_t* row_len, int6
               n_rows, width, id_limit, bad);
     BF_CHECK_LAUNCH();
   }
-  BF_HOST_READ(read);
+  BF_HOST_READ(read, st);
   auto* h = read.as<int64_t>();
   BF_CHECK_HIP(hipMemcpyAsync(h, bad, 2 * sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  BF_CHECK_HIP(hipStreamSynchronize(st));
+  BF_CHECK_HIP(read.wait());
   if (bad_host) {
     bad_host[0] = h[0];
     bad_host[1] = h[1];

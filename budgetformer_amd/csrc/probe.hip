@@ -231,14 +231,14 @@ extern "C" int bf_any_nonzero(const int32_t* x, int64_t n, int32_t* any_host, vo
   if (n == 0) return BF_OK;
   BF_CHECK_ARG(x, "any_nonzero: null tensor");
   hipStream_t st = as_stream(stream);
-  BF_HOST_READ(read);
+  BF_HOST_READ(read, st);
   auto* any = read.as<int32_t>();
   *any = 0;
   const int64_t want = ceil_div(n, int64_t(kThreads) * 4);
   BF_LAUNCH("any_nonzero_kernel", any_nonzero_kernel, dim3(unsigned(want < 256 ? want : 256)), dim3(kThreads), 0, st,
             x, n, any);
   BF_CHECK_LAUNCH();
-  BF_CHECK_HIP(hipStreamSynchronize(st));
+  BF_CHECK_HIP(read.wait());
   *any_host = *any;
   return BF_OK;
 }
@@ -261,7 +261,7 @@ extern "C" int bf_reception_cone(const int64_t* rowptr, const int32_t* col, cons
                    workspace_bytes >= node_space_bytes(num_nodes),
                "reception_cone: workspace %zu < %zu bytes", workspace_bytes, node_space_bytes(num_nodes));
   hipStream_t st = as_stream(stream);
-  BF_HOST_READ(read);
+  BF_HOST_READ(read, st);
   auto* count = read.as<uint32_t>();
   const NodeSpace s = node_space(workspace, num_nodes);
   BF_CHECK_OK(clear_nodes(s, num_nodes, st));
@@ -289,7 +289,7 @@ extern "C" int bf_reception_cone(const int64_t* rowptr, const int32_t* col, cons
   BF_LAUNCH("mark_write_kernel", mark_write_kernel<int64_t>, dim3(unsigned(s.tiles)), dim3(kThreads), 0, st, s.level,
             num_nodes, s.counts, ids);
   BF_CHECK_LAUNCH();
-  BF_CHECK_HIP(hipStreamSynchronize(st));
+  BF_CHECK_HIP(read.wait());
   *count_host = *count;
   return BF_OK;
 }
@@ -326,10 +326,10 @@ extern "C" int bf_probe_queries(const int64_t* filter, int64_t n_filter, int64_t
               s.words + 3);
     BF_CHECK_LAUNCH();
   }
-  BF_HOST_READ(read);
+  BF_HOST_READ(read, st);
   auto* h = read.as<uint32_t>();
   BF_CHECK_HIP(hipMemcpyAsync(h, s.words, 4 * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-  BF_CHECK_HIP(hipStreamSynchronize(st));
+  BF_CHECK_HIP(read.wait());
   info_host[0] = h[2];   // queries
   info_host[1] = h[1];   // some query has an in-edge
   info_host[2] = h[3];   // hubs among them

@@ -18,41 +18,15 @@ void set_error(const char* fmt, ...) {
   va_end(ap);
 }
 
-namespace {
-// The free pages of HostRead: on the heap and never freed, as the timer's lists below.
-struct HostPages {
-  std::mutex m;
-  std::vector<void*> free;
-};
-HostPages& host_pages() {
-  static auto* p = new HostPages;
-  return *p;
-}
-}  // namespace
-
-HostRead::HostRead() : page_(nullptr) {
-  HostPages& hp = host_pages();
-  {
-    std::lock_guard<std::mutex> lock(hp.m);
-    if (!hp.free.empty()) {
-      page_ = hp.free.back();
-      hp.free.pop_back();
-      return;
-    }
-  }
-  const hipError_t e = hipHostMalloc(&page_, kHostReadBytes, hipHostMallocPortable);
-  if (e != hipSuccess) {
-    page_ = nullptr;
-    set_error("hipHostMalloc failed: %s", hipGetErrorString(e));
-  }
+bool HipPages::alloc(void** page) {
+  const hipError_t e = hipHostMalloc(page, kHostReadBytes, hipHostMallocPortable);
+  if (e != hipSuccess) set_error("hipHostMalloc failed: %s", hipGetErrorString(e));
+  return e == hipSuccess;
 }
 
-HostRead::~HostRead() {
-  if (!page_) return;
-  HostPages& hp = host_pages();
-  std::lock_guard<std::mutex> lock(hp.m);
-  hp.free.push_back(page_);
-}
+void HipPages::release(void* page) { (void)hipHostFree(page); }
+
+hipError_t HipPages::wait(hipStream_t st) { return hipStreamSynchronize(st); }
 
 namespace {
 
