@@ -521,8 +521,11 @@ extern "C" int bf_coo_to_csr_ordered_workspace_size(int64_t nnz, int64_t n_row, 
 extern "C" int bf_coo_to_csr_ordered(const int64_t* row, const int64_t* col, const int64_t* type, int64_t nnz,
                                      int64_t n_row, int64_t n_col, int32_t holds, int64_t* ptr, int32_t* ids,
                                      uint64_t* rkeys, void* workspace, size_t workspace_bytes, void* stream) {
-  BF_CHECK_ARG(nnz >= 0 && n_row >= 0 && n_col >= 0 && ptr, "coo_to_csr_ordered: bad arguments");
-  BF_CHECK_ARG(n_row < (int64_t(1) << 31) && n_col < (int64_t(1) << 31) && nnz < (int64_t(1) << 31),
+  BF_CHECK_ARG(nnz >= 0 && n_row >= 0 && n_col > 0 && ptr, "coo_to_csr_ordered: bad arguments");
+  // rows are 32-bit only in a reverse index; a key holds a row's and an id's bits, the id's at most 31
+  const FieldBits b = field_bits(n_row, n_col, type != nullptr);
+  BF_CHECK_ARG((!rkeys || n_row < (int64_t(1) << 31)) && b.rb + b.cb + b.tb <= 64 && n_col < (int64_t(1) << 31) &&
+                   nnz < (int64_t(1) << 31),
                "coo_to_csr_ordered: sizes must fit int32");
   size_t need = 0;
   BF_CHECK_OK(bf_coo_to_csr_ordered_workspace_size(nnz, n_row, n_col, type != nullptr, holds, &need));
@@ -534,7 +537,6 @@ extern "C" int bf_coo_to_csr_ordered(const int64_t* row, const int64_t* col, con
     return BF_OK;
   }
   BF_CHECK_ARG(row && col && ids, "coo_to_csr_ordered: null tensor");
-  const FieldBits b = field_bits(n_row, n_col, type != nullptr);
   const ListKeys in{row, col, type, b.cb, b.cb + b.tb};
   const KeyFields f{b.cb + b.tb, 0, (uint64_t(1) << b.cb) - 1, type ? b.cb : -1};
   const int rk_row = b.tb, rk_col = b.rb + b.tb;

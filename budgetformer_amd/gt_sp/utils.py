@@ -417,8 +417,7 @@ def compute_khop_pool_dgl_neighbor(edge_index: torch.Tensor, num_nodes: int, fan
         return torch.zeros((2, 0), dtype=torch.long, device=out_dev)
     dev = out_dev if out_dev.type == "cuda" else torch.device("cuda", torch.cuda.current_device())
     n = max(int(num_nodes), int(edge_index.max().item()) + 1)
-    src, dst = hip_ops._pair_lists(edge_index.to(dev))
-    rowptr, col = hip_ops.coo_rows_to_csr(src, dst, n, n)     # out-neighbour CSR
+    rowptr, col, _, _ = hip_ops.graph_csrs(edge_index.to(dev), n, symmetric=None)     # out-neighbour CSR
     seed = _draw_walk_seed() if seed is None else int(seed)
     return hip_ops.khop_fanout_pool(rowptr, col, [int(f) for f in fanout], seed=seed,
                                     min_hop=int(min_hop)).to(out_dev)

@@ -211,8 +211,9 @@ def _coalesced(fn: str, edge_index: torch.Tensor, num_nodes: int, capacity: int)
 
 
 def _holds_coalesced(src: torch.Tensor, dst: torch.Tensor, num_nodes: int) -> int:
-    """``_coo_holds`` of a list by (src, dst), or 0 where it cannot be a coalesced one."""
-    return _coo_holds(src, dst, num_nodes, num_nodes) if 0 < src.numel() < 2 ** 31 else 0
+    """``_coo_holds`` of a list by (src, dst), or 0 where it cannot be a coalesced one (bf_coalesce then refuses the
+    sizes that it does not take)."""
+    return _coo_holds(src, dst, num_nodes, num_nodes) if 0 < src.numel() < 2 ** 31 and num_nodes < 2 ** 32 else 0
 
 
 def _is_coalesced(holds: int) -> bool:
@@ -224,7 +225,7 @@ def coalesce(edge_index: torch.Tensor, num_nodes: int) -> torch.Tensor:
     coalesced already is copied, not sorted again."""
     src, dst = _pair_lists(edge_index)
     if _is_coalesced(_holds_coalesced(src, dst, num_nodes)):
-        return torch.stack([src, dst])
+        return torch.stack([src.view(-1), dst.view(-1)])
     return _coalesced("bf_coalesce", edge_index, num_nodes, src.numel())
 
 
@@ -232,6 +233,8 @@ def graph_csrs(edge_index: torch.Tensor, num_nodes: int, symmetric: bool = False
     """(rowptr, col, in_ptr, in_src) of an edge list: its CSR by source and by target (the same arrays for a
     ``symmetric`` list, None for both with ``symmetric=None``). With ``coalesced`` the list is coalesced first, where
     it is not so already. The list's order is looked at once for all of it."""
+    if not coalesced and (edge_index.dim() != 2 or edge_index.size(0) < 2):
+        raise ValueError(f"edge_index must be [2, E] (got {tuple(edge_index.shape)})")
     src, dst = _pair_lists(edge_index)
     n = num_nodes
     holds = _coo_holds(src, dst, n, n)
@@ -637,8 +640,8 @@ def table_to_list(table: torch.Tensor, row_len: torch.Tensor, num_nodes: int, q_
     n_rows, width = table.shape
     if query_ids is not None:
         _require(query_ids, "query_ids", torch.int32, dev)
-        if query_ids.numel() != n_rows:
-            raise ValueError(f"query_ids must hold one id per table row ({n_rows})")
+        if query_ids.numel() < n_rows:
+            raise ValueError(f"query_ids must hold an id for each table row ({n_rows})")
     stream = _stream(dev)
     checked = _workspace(_size_query("bf_table_list_check_workspace_size", n_rows), dev)
     cnt = C.c_int64(0)
@@ -1398,6 +1401,8 @@ class AttentionIndex:
             qptr, kv, keys = coo_rows_to_csr(dst, src, n_q, n_kv, types, with_keys=True)
         except ValueError:
             # an id is taken with its type as one number, id + type * n_kv below 2 * n_kv
+            if not types.numel():
+                raise
             both = src + types * n_kv
             if types.min().item() < 0 or types.max().item() > 1 or both.min().item() < 0 or \
                     both.max().item() >= 2 * n_kv:
@@ -1418,7 +1423,11 @@ class AttentionIndex:
         if edge_index.dim() != 2 or edge_index.size(0) < 2:
             raise ValueError(f"edge_index must be [2, E] (got {tuple(edge_index.shape)})")
         src, dst = _pair_lists(edge_index)
-        qptr, kv, keys = coo_rows_to_csr(dst, src, n_q, n_kv, with_keys=True)
+        keys = None
+        if n_q < 2 ** 31:
+            qptr, kv, keys = coo_rows_to_csr(dst, src, n_q, n_kv, with_keys=True)
+        else:                       # a reverse entry's query is 32-bit: the CSR alone
+            qptr, kv = coo_rows_to_csr(dst, src, n_q, n_kv)
         return cls(n_q=n_q, n_kv=n_kv, qptr=qptr, kv_all=kv, chunk=chunk, item=item, _nnz=kv.numel(), _coo_keys=keys,
                    _key_stream=_raw_stream(kv.device))
 

@@ -259,3 +259,28 @@ def test_reverse_index_workspace_holds_every_smaller_sort():
         for m in [m for m in counts if m <= nnz]:
             for bits in range(1, 64):
                 assert have >= size("bf_radix_sort_workspace_size", m, 0, bits), (nnz, m, bits)
+
+
+def test_edge_list_sizes_refused_and_taken():
+    """Host-side checks of the list entry points: no columns refused, also for an empty list; row counts of 2^31 and
+    more taken by the CSR, whose rows are 64-bit, and refused where reverse keys are asked for (the call then gets
+    past the sizes to its missing workspace: host buffers, never read)."""
+    buf = (C.c_int64 * 4)()
+    p = C.cast(buf, C.c_void_p)
+    for name, args in (("bf_coo_to_csr", (p, p, 0, 3, 0, p, p, None, 0, None)),
+                       ("bf_coo_to_csr_ordered", (p, p, None, 0, 3, 0, 0, p, p, None, None, 0, None)),
+                       ("bf_coo_to_csr_ordered", (p, p, None, 0, 0, 0, 0, p, p, p, None, 0, None))):
+        with pytest.raises(ValueError, match="bad arguments"):
+            N.call(name, *args)
+    with pytest.raises(ValueError, match="workspace"):
+        N.call("bf_coo_to_csr", p, p, 2, 2 ** 31, 5, p, p, None, 0, None)
+    with pytest.raises(ValueError, match="sizes must fit"):
+        N.call("bf_coo_to_csr_ordered", p, p, None, 2, 2 ** 31, 5, 0, p, p, p, None, 0, None)
+
+
+@pytest.mark.parametrize("shape", [(2,), (1, 4), (2, 3, 4)])
+def test_a_graph_takes_only_a_two_row_list(shape):
+    import torch
+    from budgetformer_amd.graph import CSRGraph
+    with pytest.raises(ValueError, match=r"must be \[2, E\]"):
+        CSRGraph.from_edge_index(torch.zeros(shape, dtype=torch.int64), 5, device="cpu")

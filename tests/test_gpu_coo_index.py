@@ -182,3 +182,29 @@ def test_split_plan_at_block_edges(hip_device, n_rows, threshold, item, share):
     assert np.array_equal(plan.item_off.cpu().numpy()[:n_rows], off)
     assert np.array_equal(plan.item_row.cpu().numpy()[:plan.items], np.repeat(np.arange(n_rows), n))
     assert np.array_equal(plan.heavy_rows.cpu().numpy()[:plan.heavy], np.flatnonzero(n))
+
+
+def test_list_calls_refuse_and_take_what_they_did(hip_device):
+    """Empty graphs and lists without columns are refused; a coalesced list of any shape comes back [2, E]; a table
+    list takes query ids past its rows."""
+    from budgetformer_amd import hip_ops
+    from budgetformer_amd.edges import EdgeTable
+    from budgetformer_amd.graph import CSRGraph
+    from budgetformer_amd.hip_ops import AttentionIndex
+    none = torch.zeros(2, 0, dtype=torch.int64, device=hip_device)
+    for call in (lambda: CSRGraph.from_edge_index(none, 0), lambda: hip_ops.graph_csrs(none, 0, coalesced=True),
+                 lambda: hip_ops.coo_to_csr(none, 3, 0), lambda: AttentionIndex.from_coo(none, 0),
+                 lambda: AttentionIndex.from_typed_coo(torch.cat([none, none[:1]]), 3, 0),
+                 lambda: hip_ops.coalesce(none, 0)):
+        with pytest.raises(ValueError):
+            call()
+    ei = torch.tensor([[0, 1, 1, 4], [2, 0, 3, 4]], device=hip_device)
+    assert torch.equal(hip_ops.coalesce(ei.view(2, 2, 2), 5), ei)
+    assert torch.equal(hip_ops.graph_csrs(ei.view(2, 2, 2), 5, coalesced=True)[1].long(), ei[1])
+    table = torch.tensor([[0, 2], [1, -1]], dtype=torch.int32, device=hip_device)
+    lens = torch.tensor([2, 1], dtype=torch.int32, device=hip_device)
+    ids = torch.tensor([3, 4, 0], dtype=torch.int32, device=hip_device)
+    got = EdgeTable(table, lens, 5, query_ids=ids).to_edge_index()
+    assert got.tolist() == [[0, 1, 2], [3, 4, 3]]
+    with pytest.raises(ValueError, match="query_ids"):
+        EdgeTable(table, lens, 5, query_ids=ids[:1]).to_edge_index()
