@@ -575,24 +575,32 @@ __global__ void split_count_kernel(const int64_t* __restrict__ ptr, int64_t n_ro
   if (r < n_rows) packed[r] = split_count(ptr[r + 1] - ptr[r], threshold, item_size);
 }
 
-// The plan of up to kPtrInBlockMax blocks of kPtrRows rows in two launches, as
-// the table's row pointers: each block's sum of its rows' packed counts, then
-// each block adds up the sums before it, scans its own rows and writes. A scan
-// over every row's count (a packed array written, scanned and read back) took
-// 58 us at 2.9M rows, this 31. Rows to split are few: a wave scans only a
-// round of 64 rows that holds one, and writes a split row's items together.
+// The plan in two launches, as the table's row pointers: each block's sum of
+// its rows' packed counts, then each block adds up the sums before it, scans
+// its own rows and writes. Blocks of 256 rows, from 1M rows on (4096 blocks'
+// sums to add up) of 1024; past 4M rows a scan over every row's count, which
+// took 56 us where this takes 21 (2.9M rows, 61M or 14M edges, threshold 128).
+// A wave scans only a round of 64 rows that holds one to split. A row's lane
+// writes its first items and the wave the rest of long rows, one row after the
+// other: where a graph is numbered by degree its hubs follow each other, and
+// with a turn of the wave for every split row (1024 rows a wave) the plan of a
+// hub list took 177 us at 169K nodes, threshold 32 (now 16), and 294 at 2.4M
+// (now 74).
+constexpr int64_t kPlanInBlockMax = 4096;
+constexpr int kPlanOwnItems = 4;
 __device__ __forceinline__ uint64_t block_sum_u64(uint64_t v, uint64_t* tmp /*[kThreads / 64]*/) {
   return uint64_t(block_sum_i64(int64_t(v), reinterpret_cast<int64_t*>(tmp)));
 }
 
+template <int PER>     // rows per thread
 __global__ __launch_bounds__(kThreads) void plan_sums_kernel(const int64_t* __restrict__ ptr, int64_t n_rows,
                                                              int threshold, int item_size,
                                                              uint64_t* __restrict__ bsum) {
   __shared__ uint64_t tmp[kThreads / 64];
-  const int64_t t0 = int64_t(blockIdx.x) * kPtrRows + threadIdx.x;
+  const int64_t t0 = int64_t(blockIdx.x) * (kThreads * PER) + threadIdx.x;
   uint64_t s = 0;
 #pragma unroll
-  for (int u = 0; u < kPtrRowsPerThread; ++u) {
+  for (int u = 0; u < PER; ++u) {
     const int64_t r = t0 + u * kThreads;
     if (r < n_rows) s += split_count(ptr[r + 1] - ptr[r], threshold, item_size);
   }
@@ -600,6 +608,7 @@ __global__ __launch_bounds__(kThreads) void plan_sums_kernel(const int64_t* __re
   if (threadIdx.x == 0) bsum[blockIdx.x] = s;
 }
 
+template <int PER>
 __global__ __launch_bounds__(kThreads) void plan_write_kernel(
     const int64_t* __restrict__ ptr, int64_t n_rows, int threshold, int item_size, const uint64_t* __restrict__ bsum,
     int64_t item_cap, int32_t* __restrict__ nitems, int32_t* __restrict__ item_off, int32_t* __restrict__ item_row,
@@ -609,10 +618,10 @@ __global__ __launch_bounds__(kThreads) void plan_write_kernel(
   uint64_t before = 0;
   for (int64_t k = threadIdx.x; k < int64_t(blockIdx.x); k += kThreads) before += bsum[k];
   before = block_sum_u64(before, tmp);
-  const int64_t t0 = int64_t(blockIdx.x) * kPtrRows + int64_t(w) * (64 * kPtrRowsPerThread) + lane;
-  uint64_t v[kPtrRowsPerThread], mine = 0;
+  const int64_t t0 = int64_t(blockIdx.x) * (kThreads * PER) + int64_t(w) * (64 * PER) + lane;
+  uint64_t v[PER], mine = 0;
 #pragma unroll
-  for (int u = 0; u < kPtrRowsPerThread; ++u) {
+  for (int u = 0; u < PER; ++u) {
     const int64_t r = t0 + u * 64;
     v[u] = r < n_rows ? split_count(ptr[r + 1] - ptr[r], threshold, item_size) : 0;
     mine += v[u];
@@ -626,7 +635,7 @@ __global__ __launch_bounds__(kThreads) void plan_write_kernel(
   for (int i = 0; i < kThreads / 64; ++i)
     if (i < w) base += wtot[i];
 #pragma unroll
-  for (int u = 0; u < kPtrRowsPerThread; ++u) {
+  for (int u = 0; u < PER; ++u) {
     const int64_t r = t0 + u * 64;
     uint64_t x = v[u];
     uint64_t split = __ballot(x != 0);
@@ -651,12 +660,14 @@ __global__ __launch_bounds__(kThreads) void plan_write_kernel(
         counts[1] = int32_t(heavy < heavy_cap ? heavy : heavy_cap);
       }
     }
-    while (split) {                                  // each split row's items by the whole wave
-      const int src = __ffsll((unsigned long long)split) - 1;
-      split &= split - 1;
-      const int32_t row = int32_t(t0 - lane) + u * 64 + src, cnt = __shfl(n, src, 64);
-      const int64_t first = int64_t(__shfl(off, src, 64) >> 32);
-      for (int64_t j = lane; j < cnt && first + j < item_cap; j += 64) item_row[first + j] = row;
+    const int32_t first = int32_t(off >> 32);
+    for (int i = 0; i < kPlanOwnItems; ++i)
+      if (i < n && first + int64_t(i) < item_cap) item_row[first + i] = int32_t(r);
+    for (uint64_t rest = __ballot(n > kPlanOwnItems); rest; rest &= rest - 1) {   // long rows by the whole wave
+      const int src = __ffsll((unsigned long long)rest) - 1;
+      const int32_t cnt = __builtin_amdgcn_readlane(n, src), at = __builtin_amdgcn_readlane(first, src);
+      const int32_t row = int32_t(t0 - lane) + u * 64 + src;
+      for (int64_t j = kPlanOwnItems + lane; j < cnt && at + j < item_cap; j += 64) item_row[at + j] = row;
     }
   }
 }
@@ -1046,16 +1057,17 @@ extern "C" int bf_split_plan(const int64_t* ptr, int64_t n_rows, int32_t thresho
   void* temp = static_cast<char*>(workspace) + 2 * slab;
   size_t temp_bytes = 0;
   (void)prim::exclusive_sum(nullptr, temp_bytes, static_cast<const uint64_t*>(packed), packed_off, n_rows, st);
-  const int64_t ptr_blocks = ceil_div(n_rows, kPtrRows);
-  if (ptr_blocks <= kPtrInBlockMax) {               // packed: one sum per block
-    BF_LAUNCH("plan_sums_kernel", plan_sums_kernel, dim3(unsigned(ptr_blocks)), dim3(kThreads), 0, st, ptr, n_rows,
-              threshold, item_size, packed);
+  const auto by_blocks = [&](auto sums, auto write, int per) -> int {   // packed: one sum per block
+    const unsigned blocks = unsigned(ceil_div(n_rows, int64_t(kThreads) * per));
+    BF_LAUNCH("plan_sums_kernel", sums, dim3(blocks), dim3(kThreads), 0, st, ptr, n_rows, threshold, item_size, packed);
     BF_CHECK_LAUNCH();
-    BF_LAUNCH("plan_write_kernel", plan_write_kernel, dim3(unsigned(ptr_blocks)), dim3(kThreads), 0, st, ptr, n_rows,
-              threshold, item_size, packed, item_cap, nitems, item_off, item_row, heavy_rows, heavy_cap, counts);
+    BF_LAUNCH("plan_write_kernel", write, dim3(blocks), dim3(kThreads), 0, st, ptr, n_rows, threshold, item_size,
+              packed, item_cap, nitems, item_off, item_row, heavy_rows, heavy_cap, counts);
     BF_CHECK_LAUNCH();
     return BF_OK;
-  }
+  };
+  if (n_rows <= kPlanInBlockMax * kThreads) return by_blocks(plan_sums_kernel<1>, plan_write_kernel<1>, 1);
+  if (n_rows <= kPlanInBlockMax * kThreads * 4) return by_blocks(plan_sums_kernel<4>, plan_write_kernel<4>, 4);
   BF_LAUNCH("split_count_kernel", split_count_kernel, dim3(blocks_for(n_rows)), dim3(kThreads), 0, st, ptr, n_rows,
             threshold, item_size, packed);
   BF_CHECK_LAUNCH();

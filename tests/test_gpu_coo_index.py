@@ -208,3 +208,22 @@ def test_list_calls_refuse_and_take_what_they_did(hip_device):
     assert got.tolist() == [[0, 1, 2], [3, 4, 3]]
     with pytest.raises(ValueError, match="query_ids"):
         EdgeTable(table, lens, 5, query_ids=ids[:1]).to_edge_index()
+
+
+@pytest.mark.parametrize("n_rows", [255, 256, 257, 5000, 1_048_576, 1_048_577, 4_194_304, 4_194_305])
+def test_split_plan_of_rows_in_order_of_length(hip_device, n_rows):
+    """Long rows next to each other, as in a graph numbered by degree: rows of no item, of fewer items than their lane
+    writes, of more, and of more than a wave has lanes; at the edges of the plan's three forms."""
+    from budgetformer_amd import hip_ops
+    lens = np.minimum(40_000.0 / (1.0 + np.arange(n_rows)) ** 0.9, 9000.0).astype(np.int64)
+    ptr = np.concatenate([[0], np.cumsum(lens)])
+    for threshold, item in ((32, 32), (3, 50)):
+        plan = hip_ops.split_plan(torch.from_numpy(ptr).to(hip_device), int(ptr[-1]), threshold, item)
+        split = lens > threshold
+        n = np.zeros(n_rows, dtype=np.int64)
+        n[split] = [hip_ops.split_row_items(int(x), item) for x in lens[split]]
+        assert (plan.items, plan.heavy) == (n.sum(), split.sum())
+        assert np.array_equal(plan.nitems.cpu().numpy()[:n_rows], n)
+        assert np.array_equal(plan.item_off.cpu().numpy()[:n_rows], np.cumsum(n) - n)
+        assert np.array_equal(plan.item_row.cpu().numpy()[:plan.items], np.repeat(np.arange(n_rows), n))
+        assert np.array_equal(plan.heavy_rows.cpu().numpy()[:plan.heavy], np.flatnonzero(split))
