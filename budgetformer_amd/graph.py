@@ -48,16 +48,11 @@ class CSRGraph:
         """
         cache = self.__dict__.setdefault("_hubs", {})
         if threshold not in cache:
-            # a build asks for both of the usual lists: they are found together, with one host read
+            # a build asks for both of the usual lists: they are found together, with one host read (169K nodes:
+            # 46 us, 36 for one of them; 2.9M nodes 68, 45)
             usual = (hip_ops.LIGHT_MAX, hip_ops.HUB_THRESHOLD)
             wanted = [t for t in usual if t not in cache] if threshold in usual else [threshold]
-            counts = torch.empty(2 * len(wanted), dtype=torch.int32, device=self.device)
-            plans = [hip_ops.split_plan(self.in_ptr, self.num_edges, t, max(t, 1), resolve=False,
-                                        counts=counts[2 * i:2 * i + 2], host_copy=False)
-                     for i, t in enumerate(wanted)]
-            hip_ops.resolve_plans(*plans)
-            for t, plan in zip(wanted, plans):
-                cache[t] = plan.heavy_rows[: plan.heavy].clone()
+            cache.update(zip(wanted, hip_ops.rows_longer_than(self.in_ptr, self.num_edges, wanted)))
         return cache[threshold]
 
     def walk_records(self, reserve_bytes: Optional[int] = None) -> Optional[torch.Tensor]:

@@ -1016,6 +1016,28 @@ def split_plan(ptr: torch.Tensor, nnz: int, threshold: int = DEFAULT_CHUNK, item
     return plan
 
 
+def rows_longer_than(ptr: torch.Tensor, nnz: int, thresholds) -> list:
+    """For each threshold the ascending ids (int32) of the CSR rows longer than it: the split rows of plans that cut
+    no row (bf_split_plan), whose other arrays share one scratch buffer; one host read for all of them."""
+    dev = ptr.device
+    _require(ptr, "ptr", torch.int64)
+    lib, n, item, k = N.load(), ptr.numel() - 1, 2 ** 31 - 1, len(thresholds)
+    caps = [(int(lib.bf_split_item_capacity(nnz, t, item)), int(lib.bf_split_row_capacity(nnz, t))) for t in thresholds]
+    at = 2 * k + 2 * max(n, 1) + max(max(c[0] for c in caps), 1)        # counts, nitems, item_off, item_row; the lists
+    buf = torch.empty(at + sum(max(c[1], 1) for c in caps), dtype=torch.int32, device=dev)
+    ws = _workspace(_size_query("bf_split_plan_workspace_size", n), dev)
+    base, stream, first = buf.data_ptr(), _stream(dev), []
+    nitems, item_off = base + 8 * k, base + 8 * k + 4 * max(n, 1)
+    for i, (t, (item_cap, row_cap)) in enumerate(zip(thresholds, caps)):
+        N.call("bf_split_plan", _p(ptr), n, t, item, C.c_void_p(nitems), C.c_void_p(item_off),
+               C.c_void_p(item_off + 4 * max(n, 1)), item_cap, C.c_void_p(base + 4 * at), row_cap,
+               C.c_void_p(base + 8 * i), _p(ws), ws.numel(), stream)
+        first.append(at)
+        at += max(row_cap, 1)
+    rows = buf[:2 * k].cpu().tolist()[1::2]
+    return [buf[a:a + r].clone() for a, r in zip(first, rows)]
+
+
 # ------------------------------------------------------------------ attention index
 # Plans of up to this many items (at capacity) need no host copy of their counts. The line bounds the records that a
 # call at capacity makes room for (2 D + H floats an item: 17 MB here at D = 128), not the time: a step on a new index

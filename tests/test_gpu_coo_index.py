@@ -227,3 +227,16 @@ def test_split_plan_of_rows_in_order_of_length(hip_device, n_rows):
         assert np.array_equal(plan.item_off.cpu().numpy()[:n_rows], np.cumsum(n) - n)
         assert np.array_equal(plan.item_row.cpu().numpy()[:plan.items], np.repeat(np.arange(n_rows), n))
         assert np.array_equal(plan.heavy_rows.cpu().numpy()[:plan.heavy], np.flatnonzero(split))
+
+
+@pytest.mark.parametrize("n_rows", [0, 1, 257, 1_100_000])
+def test_rows_longer_than(hip_device, n_rows):
+    """The hub lists of a graph: several thresholds at once, one that no row passes, an empty CSR."""
+    from budgetformer_amd import hip_ops
+    lens = np.minimum((3.0 / np.maximum(np.random.default_rng(n_rows).random(n_rows), 1e-4)).astype(np.int64), 20_000)
+    ptr = torch.from_numpy(np.concatenate([[0], np.cumsum(lens)])).to(hip_device)
+    got = hip_ops.rows_longer_than(ptr, int(lens.sum()), (32, 1, 1024, 30_000))
+    for t, ids in zip((32, 1, 1024, 30_000), got):
+        assert ids.dtype == torch.int32 and np.array_equal(ids.cpu().numpy(), np.flatnonzero(lens > t))
+    with pytest.raises(ValueError):
+        hip_ops.rows_longer_than(ptr, int(lens.sum()), (32, 0))
