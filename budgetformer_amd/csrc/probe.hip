@@ -65,18 +65,21 @@ __global__ __launch_bounds__(kThreads) void mark_ids_kernel(const int64_t* __res
     *outside = 1u;
 }
 
-// One hop: every in-neighbour of a node of level `hop` that has none yet gets level `next` (concurrent writers agree).
+// One hop: every in-neighbour of a node of level `hop` that has none yet gets level `next` (concurrent writers agree);
+// *grew (if given) becomes hop_no when there is one.
 // A 16-lane group walks a row; rows longer than kBlockRow are left to the whole workgroup, and a workgroup's rows
 // lie gridDim.x apart, since graphs often number their hubs next to each other: with a group per row, hubs of up
 // to 13K edges in one workgroup made a hop of a 169K-node graph 60 us; the workgroup on its long rows 45, the rows
 // spread out as well 10.
 __global__ __launch_bounds__(kThreads) void cone_hop_kernel(const int64_t* __restrict__ in_ptr,
                                                             const int32_t* __restrict__ in_src, int64_t n, int hop, int next,
-                                                            uint8_t* __restrict__ level) {
+                                                            uint8_t* __restrict__ level, uint32_t hop_no,
+                                                            uint32_t* __restrict__ grew) {
   __shared__ int64_t long_beg[kRowsPerBlock], long_end[kRowsPerBlock];
   __shared__ int n_long;
   if (threadIdx.x == 0) n_long = 0;
   __syncthreads();
+  bool marked_any = false;
   // every step-th source of [i, end), kMarkUnroll of them and then their levels in flight together
   auto mark = [&](int64_t i, int64_t end, int step) {
     for (; i < end; i += int64_t(step) * kMarkUnroll) {
@@ -91,7 +94,10 @@ __global__ __launch_bounds__(kThreads) void cone_hop_kernel(const int64_t* __res
       for (int u = 0; u < kMarkUnroll; ++u) lev[u] = src[u] >= 0 && src[u] < n ? level[src[u]] : uint8_t(1);
 #pragma unroll
       for (int u = 0; u < kMarkUnroll; ++u)
-        if (lev[u] == 0) level[src[u]] = uint8_t(next);
+        if (lev[u] == 0) {
+          level[src[u]] = uint8_t(next);
+          marked_any = true;
+        }
     }
   };
   const int64_t v = int64_t(threadIdx.x / kGroup) * gridDim.x + blockIdx.x;
@@ -110,7 +116,13 @@ __global__ __launch_bounds__(kThreads) void cone_hop_kernel(const int64_t* __res
   }
   __syncthreads();
   for (int k = 0; k < n_long; ++k) mark(long_beg[k] + threadIdx.x, long_end[k], kThreads);
+  if (grew && __ballot(marked_any) && (threadIdx.x & 63) == 0) *grew = hop_no;
 }
+
+// Hops between two looks at whether the cone still grows, so that one deeper than its graph ends early; a cone of up
+// to this many hops takes none. 169K nodes, 400 layers: 1540 us without looks, 155 with; a chain that grows on 1050,
+// 2270.
+constexpr int kLookHops = 16;
 
 // Bit u: node t0 + u of this thread's 16 consecutive nodes is marked.
 __device__ __forceinline__ uint32_t marked(const uint8_t* __restrict__ level, int64_t n, int64_t t0) {
@@ -275,10 +287,18 @@ extern "C" int bf_reception_cone(const int64_t* rowptr, const int32_t* col, cons
     BF_CHECK_LAUNCH();
   }
   // levels cycle through 1..254 to fit a byte: a node met again under an old level has no unmarked neighbour left
+  uint32_t* const grew = hops > kLookHops ? s.words + 1 : nullptr;
   for (int h = 0; h < hops; ++h) {
     BF_LAUNCH("cone_hop_kernel", cone_hop_kernel, dim3(unsigned(ceil_div(num_nodes, int64_t(kRowsPerBlock)))),
-              dim3(kThreads), 0, st, in_ptr, in_src, num_nodes, 1 + h % 254, 1 + (h + 1) % 254, s.level);
+              dim3(kThreads), 0, st, in_ptr, in_src, num_nodes, 1 + h % 254, 1 + (h + 1) % 254, s.level,
+              uint32_t(h + 1), grew);
     BF_CHECK_LAUNCH();
+    if ((h + 1) % kLookHops == 0 && h + 1 < hops) {
+      BF_HOST_READ(look, st);
+      BF_CHECK_HIP(hipMemcpyAsync(look.as<uint32_t>(), grew, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+      BF_CHECK_HIP(look.wait());
+      if (*look.as<uint32_t>() != uint32_t(h + 1)) break;
+    }
   }
   BF_LAUNCH("mark_count_kernel", mark_count_kernel, dim3(unsigned(s.tiles)), dim3(kThreads), 0, st, s.level, num_nodes,
             static_cast<const int64_t*>(nullptr), s.counts, static_cast<uint32_t*>(nullptr));

@@ -203,3 +203,22 @@ def test_assemble_rows_by_width(hip_device, b_real, b_rw, dedup):
         row = np.unique(row) if dedup else np.sort(row)
         assert row_len[r] == row.size and np.array_equal(table[r], np.pad(row, (0, table.shape[1] - row.size),
                                                                          constant_values=-1))
+
+
+@pytest.mark.parametrize("layers", [2, 16, 17, 18, 33, 34, 300, 5000])
+def test_deep_cones(hip_device, layers):
+    """Cones past the hops between two looks (16) and past the levels a byte holds, on a long chain that still grows
+    and on a short one that has ended (with another component that is never reached)."""
+    from budgetformer_amd.graph import CSRGraph
+    from budgetformer_amd.probe import reception_cone
+    long, short = 1000, 20
+    a = torch.arange(long - 1)
+    b = torch.arange(short - 1)
+    # every node reaches the next one: the cone of the last node is the nodes before it
+    graph = CSRGraph.from_edge_index(torch.stack([a, a + 1]), long, device=hip_device)
+    got = reception_cone(graph, torch.tensor([long - 1], device=hip_device), layers)
+    assert got.tolist() == list(range(max(long - layers, 0), long))
+    both = torch.cat([torch.stack([b, b + 1]), torch.stack([b, b + 1]) + 50], dim=1)
+    graph = CSRGraph.from_edge_index(both, 70, device=hip_device)
+    got = reception_cone(graph, torch.tensor([short - 1], device=hip_device), layers)
+    assert got.tolist() == list(range(max(short - layers, 0), short))
