@@ -173,13 +173,18 @@ def load():
             f"budgetformer_amd: HIP library not found at {path}; build it with "
             f"`python -m budgetformer_amd.build` (no CPU fallback exists)")
     lib = C.CDLL(path)
+    bound = getattr(lib, "bf_version", None)
+    if bound is None or bound() != ABI_VERSION:
+        raise RuntimeError(f"budgetformer_amd: {path} implements ABI {bound() if bound else 'unknown'}, this binding "
+                           f"expects {ABI_VERSION}; rebuild it with `python -m budgetformer_amd.build`")
+    missing = [name for name in _SIGS if not hasattr(lib, name)]
+    if missing:                  # built before these entry points were added (additions keep the version)
+        raise RuntimeError(f"budgetformer_amd: {path} lacks {', '.join(missing)}; rebuild it with "
+                           f"`python -m budgetformer_amd.build`")
     for name, (res, args) in _SIGS.items():
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
-    if lib.bf_version() != ABI_VERSION:
-        raise RuntimeError(f"budgetformer_amd: {path} implements ABI {lib.bf_version()}, this binding expects "
-                           f"{ABI_VERSION}; rebuild it with `python -m budgetformer_amd.build`")
     _lib = lib
     return lib
 

@@ -678,8 +678,8 @@ __global__ __launch_bounds__(kThreads) void plan_write_kernel(
 // entries are written. A row's thread writes the item_row of its first
 // kOwnItems items; rows with more (the Graphormer token row and column, hubs)
 // are queued in LDS and their remaining items written by the whole block.
-// packed_off NULL: the exclusive sums are formed here, each block adding up
-// the slots before it (plans of at most kPlanInBlockSlots slots).
+// packed_off NULL (plans with an order, of at most kPlanInBlockSlots slots): the
+// exclusive sums are formed here, each block adding up the slots before it.
 constexpr int kOwnItems = 32;
 constexpr int64_t kPlanInBlockSlots = 32768;
 
@@ -696,8 +696,8 @@ __global__ __launch_bounds__(kThreads) void split_rows_kernel(
   const int64_t j = int64_t(blockIdx.x) * kThreads + threadIdx.x;
   uint64_t in_block_off = 0;
   if (!packed_off) {
-    // With an order the split rows hold its first slots (longest first), so a slot's entry is zero only
-    // past the last split row: a thread stops at its first zero. Four loads in flight per step.
+    // The split rows hold the order's first slots (longest first), so a slot's entry is zero only past the
+    // last split row: a thread stops at its first zero. Four loads in flight per step.
     const int64_t lim = int64_t(blockIdx.x) * kThreads;
     uint64_t before = 0;
     for (int64_t k = threadIdx.x; k < lim; k += 4 * kThreads) {
@@ -705,7 +705,7 @@ __global__ __launch_bounds__(kThreads) void split_rows_kernel(
 #pragma unroll
       for (int u = 0; u < 4; ++u) x[u] = k + u * kThreads < lim ? packed[k + u * kThreads] : 0;
       before += x[0] + x[1] + x[2] + x[3];
-      if (order && x[3] == 0) break;
+      if (x[3] == 0) break;
     }
     // the block's total of `before` is the sum over every earlier slot
     const uint64_t lo = block_excl_scan_u64(before, scan_tmp);

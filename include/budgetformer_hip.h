@@ -57,7 +57,12 @@ enum { BF_DTYPE_F32 = 0, BF_DTYPE_BF16 = 1, BF_DTYPE_F16 = 2 };
  *        and more than 8191 walk candidates per query);
  *   302  bf_row_stream_probe (calibration);
  *   303  bf_attn_dropout gains `keep` (the forward stores its keep bits, the
- *        backward's query-major pass reads them back).                      */
+ *        backward's query-major pass reads them back). Added since, with no
+ *        change to what was there (a caller finds them by name): bf_coo_order,
+ *        bf_coo_to_csr_ordered, bf_coo_reverse, bf_coo_reverse_slots,
+ *        bf_coalesce_bidirected, bf_table_list_check, bf_table_to_list,
+ *        bf_reception_cone, bf_probe_queries, bf_any_nonzero and the
+ *        workspace sizes of those that have one.                            */
 #define BF_ABI_VERSION 303
 int bf_version(void);
 /* Message of the last failed call on this thread ("" if none). */

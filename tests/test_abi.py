@@ -284,3 +284,22 @@ def test_a_graph_takes_only_a_two_row_list(shape):
     from budgetformer_amd.graph import CSRGraph
     with pytest.raises(ValueError, match=r"must be \[2, E\]"):
         CSRGraph.from_edge_index(torch.zeros(shape, dtype=torch.int64), 5, device="cpu")
+
+
+@pytest.mark.parametrize("stale", ["missing", "version"])
+def test_a_library_built_before_an_entry_point_is_refused_with_what_to_do(monkeypatch, stale):
+    class Stale:
+        def __init__(self, path):
+            pass
+
+        def __getattr__(self, name):
+            if name == "bf_version":
+                return lambda: N.ABI_VERSION - (stale == "version")
+            if stale == "missing" and name == "bf_coo_order":
+                raise AttributeError(name)
+            return type("fn", (), {})()
+
+    monkeypatch.setattr(N, "_lib", None)
+    monkeypatch.setattr(N.C, "CDLL", Stale)
+    with pytest.raises(RuntimeError, match="bf_coo_order.*rebuild" if stale == "missing" else "ABI 302.*rebuild"):
+        N.load()

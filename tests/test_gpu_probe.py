@@ -222,3 +222,19 @@ def test_deep_cones(hip_device, layers):
     graph = CSRGraph.from_edge_index(both, 70, device=hip_device)
     got = reception_cone(graph, torch.tensor([short - 1], device=hip_device), layers)
     assert got.tolist() == list(range(max(short - layers, 0), short))
+
+
+def test_mark_in_neighbors(hip_device):
+    """The single hop of the C interface: every source of an edge into the frontier, and nothing unmarked."""
+    from budgetformer_amd import hip_ops
+    rng = np.random.default_rng(8)
+    n = 1003
+    src, dst = rng.integers(0, n, 5000), np.sort(rng.integers(0, n, 5000))
+    frontier, reached = rng.random(n) < 0.05, rng.random(n) < 0.1
+    want = reached.copy()
+    want[src[frontier[dst]]] = True
+    marks = torch.from_numpy(reached.astype(np.uint8)).to(hip_device)
+    hip_ops.mark_in_neighbors(torch.from_numpy(np.searchsorted(dst, np.arange(n + 1))).to(hip_device),
+                              torch.from_numpy(src.astype(np.int32)).to(hip_device),
+                              torch.from_numpy(frontier.astype(np.uint8)).to(hip_device), marks)
+    assert np.array_equal(marks.cpu().numpy().astype(bool), want)
