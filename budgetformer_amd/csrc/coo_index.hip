@@ -168,6 +168,9 @@ __global__ __launch_bounds__(kThreads) void coo_reverse_keys_kernel(ListKeys in,
 // ks of a list's reverse index: entry i of key row s names query kq[i]; its slot is where s (with the entry's
 // type) sits in that query's ascending row. Equal entries of one (row, column) follow each other in both
 // orders, so the k-th of them takes the k-th slot. Key rows come from a search within the block's own rows.
+// Three searches an entry, where a pair sort used to carry the slots through every list's index: only a bias, factor
+// or dropout needs them (COO list and layer with dropout, float32 rows of 128: 20K nodes 524 -> 382 us, 169K
+// 1027 -> 836, 600K 2829 -> 2680; with a bias 580 -> 435, 1217 -> 1019, 3766 -> 3614).
 __global__ __launch_bounds__(kThreads) void coo_reverse_slots_kernel(const int64_t* __restrict__ qptr,
                                                                      const int32_t* __restrict__ kv,
                                                                      const int64_t* __restrict__ kptr,

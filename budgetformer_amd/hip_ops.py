@@ -348,7 +348,8 @@ def rw_select_rows(rowptr, col, qids: torch.Tensor, walks_per_node: int, walk_le
                    key_seed: int, u=None, philox_seed: int = 0, philox_offset: int = 0, subtract=None,
                    walk_rec=None, ids_checked: bool = False):
     """bf_rw_select for an explicit query list; ``subtract=(in_ptr, in_src)`` drops candidates that are
-    already graph edges into the query. ``ids_checked``: the ids are known to lie in the graph. Returns (sel_kv [n,k_rw] key order, sel_cnt [n])."""
+    already graph edges into the query. ``ids_checked``: the ids are known to lie in the graph. Returns
+    (sel_kv [n,k_rw] key order, sel_cnt [n])."""
     dev = rowptr.device
     _require(rowptr, "rowptr", torch.int64)
     _require(col, "col", torch.int32, dev)
@@ -380,7 +381,8 @@ def rw_select_rows(rowptr, col, qids: torch.Tensor, walks_per_node: int, walk_le
 def real_select_rows(in_ptr, in_src, qids: torch.Tensor, k_real: int, key_seed: int,
                      hubs: Optional[torch.Tensor] = None, hub_threshold: int = HUB_THRESHOLD,
                      ids_checked: bool = False):
-    """Real-edge top-k_real in key order for an explicit query list (``ids_checked`` as in rw_select_rows): (sel_kv [n,k_real], sel_cnt [n])."""
+    """Real-edge top-k_real in key order for an explicit query list (``ids_checked`` as in rw_select_rows):
+    (sel_kv [n,k_real], sel_cnt [n])."""
     dev = in_ptr.device
     _require(in_ptr, "in_ptr", torch.int64)
     _require(in_src, "in_src", torch.int32, dev)
