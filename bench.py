@@ -273,8 +273,8 @@ def main(argv=None):
     ap.add_argument("--warmup", type=int, default=3)
     ap.add_argument("--config", default="c2", choices=sorted(CONFIGS))
     ap.add_argument("--extra", default=None,
-                    help="comma-separated configs measured after the main one and reported in the same JSON line "
-                         "under extra_configs (default: c3,c4,c5 when --config is c2, else none; 'none' for none)")
+                    help="comma-separated configs measured after the main one, their main figures reported in the same "
+                         "JSON line under extra_configs and the full records on stderr (default: c3,c4,c5 when --config is c2, else none; 'none' for none)")
     ap.add_argument("--no-cpu-baseline", action="store_true", help="skip the CPU oracle timing")
     ap.add_argument("--chunk", type=int, default=None, help="split threshold (rows longer than this are split)")
     ap.add_argument("--item", type=int, default=None, help="entries per split item")
@@ -336,8 +336,23 @@ def main(argv=None):
                         if k in rec})
     if records:
         result["extra_configs"] = records
-    print(json.dumps(result), flush=True)
+    print(f"[bench] full record: {json.dumps(result)}", file=sys.stderr, flush=True)
+    print(json.dumps(brief(result)), flush=True)
     return 0
+
+
+def brief(result):
+    """The JSON line of a result: all of it but the per-kernel and floor tables (on stderr, in the full record), and
+    of the extra configs their main figures. A reader that keeps the last 8 KB of the output has the whole line."""
+    line = {k: v for k, v in result.items() if k not in ("kernels", "gather_floor", "extra_configs")}
+    keep = ("dtype", "steps", "warmup", "ms_per_step", "value", "unit", "attn_fwd_bwd_ms", "edge_build_ms")
+    roof = ("kernel", "bound", "achieved", "peak", "unit", "frac", "frac_of_floor")
+    extra = [{"workload": r["config"]["workload"], **{k: r[k] for k in keep if k in r},
+              "rw_edges_per_s": r.get("builder", {}).get("rw_edges_per_s"),
+              "cpu_baseline": r.get("cpu_baseline", {}).get("value"),
+              "roofline": {k: r["roofline"][k] for k in roof if k in r.get("roofline", {})}}
+             for r in result.get("extra_configs", [])]
+    return {**line, "extra_configs": extra} if extra else line
 
 
 def run(config, steps, warmup, chunk=None, item=None, with_cpu=True):
