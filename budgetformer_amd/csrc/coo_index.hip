@@ -317,8 +317,8 @@ __device__ __forceinline__ uint32_t list_lengths(const int32_t* __restrict__ row
   return bad;
 }
 
-// Lengths and counts are added up in 64 bits: a block of very wide rows holds more than 2^32 entries.
-__device__ __forceinline__ uint64_t block_sum(uint64_t v, uint64_t* wave /*[kThreads / 64]*/) {
+template <typename S>
+__device__ __forceinline__ S block_sum(S v, S* wave /*[kThreads / 64]*/) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   __syncthreads();                       // an earlier sum's words are read
@@ -334,13 +334,13 @@ __global__ __launch_bounds__(kThreads) void table_list_check_kernel(const int32_
                                                                     uint64_t* __restrict__ sums,
                                                                     uint64_t* __restrict__ bad) {
   __shared__ int32_t len[kListRows];
-  __shared__ uint64_t wave[kThreads / 64];
+  __shared__ I wave[kThreads / 64];
   const uint32_t bad_len = list_lengths(row_len, n_rows, width, len);
   __syncthreads();
-  uint64_t total = 0;
-  uint32_t bad_id = 0;         // of a thread: at most 2 * width slots
+  I total = 0;                   // as the slots: 2^31 entries at most in a block numbered in 32 bits
+  uint32_t bad_id = 0;
 #pragma unroll
-  for (int u = 0; u < kListRows / kThreads; ++u) total += uint64_t(len[u * kThreads + threadIdx.x]);
+  for (int u = 0; u < kListRows / kThreads; ++u) total += I(len[u * kThreads + threadIdx.x]);
   const int64_t r0 = int64_t(blockIdx.x) * kListRows;
   const int rows = int(n_rows - r0 < kListRows ? n_rows - r0 : kListRows);
   const I slots = I(rows) * I(width);
@@ -357,7 +357,7 @@ __global__ __launch_bounds__(kThreads) void table_list_check_kernel(const int32_
       bad_id += (int32_t(c) < len[r] && (id[u] < 0 || int64_t(id[u]) >= id_limit)) ? 1u : 0u;
     }
   }
-  const uint64_t s = block_sum(total, wave), bl = block_sum(bad_len, wave), bi = block_sum(bad_id, wave);
+  const I s = block_sum(total, wave), bl = block_sum(I(bad_len), wave), bi = block_sum(I(bad_id), wave);
   if (threadIdx.x == 0) {
     sums[blockIdx.x] = s;
     bad[2 * int64_t(blockIdx.x)] = bl;
@@ -393,8 +393,13 @@ __global__ __launch_bounds__(kTotalsThreads) void list_totals_kernel(uint64_t* _
     base_at += tot;
   }
 #pragma unroll
-  for (int i = 0; i < 3; ++i)
-    if (mine[i]) atomicAdd(reinterpret_cast<unsigned long long*>(&all[i]), (unsigned long long)mine[i]);
+  for (int i = 0; i < 3; ++i) {
+    if (!__ballot(mine[i] != 0)) continue;        // the bad ones, nearly always
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) mine[i] += __shfl_xor(mine[i], o, 64);
+    if ((threadIdx.x & 63) == 0)                  // a wave at a time: a thread each would meet in one LDS word
+      atomicAdd(reinterpret_cast<unsigned long long*>(&all[i]), (unsigned long long)mine[i]);
+  }
   __syncthreads();
   if (threadIdx.x < 3) out[threadIdx.x] = all[threadIdx.x];
 }
